@@ -839,6 +839,65 @@ def test_small_causal_forward_rule_runs_the_64_query_tiling():
                              tag=f"fwd tiling 11 B1 Hq6 Hkv2 N333 D{D} causal={causal}")
 
 
+def _forced_forward(q, k, v, causal, variant):
+    D = q.shape[-1]
+    _lib.set_tiling(_lib.KERNEL_FWD, D, causal, variant)
+    try:
+        return _ops.flash_fwd(q, k, v, causal, D ** -0.5)
+    finally:
+        _lib.set_tiling(_lib.KERNEL_FWD, D, causal, -1)
+
+
+# (B, Hq, Hkv, N_q, N_kv, D, causal, tiling the rule takes), on both sides of its lines
+FWD_SIZE_RULE_CASES = [
+    (1, 32, 8, 3001, 3001, 128, True, 6),      # W = 768 work-groups of 128 queries
+    (1, 32, 8, 3900, 3900, 128, True, 7),      # 512 of 256: pairs on every CU
+    (1, 32, 8, 2048, 2048, 128, True, 8),      # W = 512, long loops
+    (1, 32, 8, 1500, 1500, 128, True, 11),     # W = 384, short loops
+    (1, 32, 8, 1700, 1700, 128, True, 6),      # W = 448, short loops
+    (1, 4, 4, 8192, 8192, 128, True, 6),       # W = 256, split keys
+    (1, 2, 1, 3000, 3000, 128, True, 11),      # W = 48
+    (1, 2, 1, 4096, 5000, 128, True, 6),       # W = 64, split keys
+    (3, 8, 4, 33, 700, 128, True, 11),         # one short tile, few visible keys
+    (4, 16, 16, 1025, 1025, 128, False, 6),
+    (3, 32, 8, 4096, 4096, 128, False, 7),     # six whole rounds
+    (3, 32, 8, 2000, 2000, 128, False, 6),     # whole rounds, short loops
+    (1, 16, 16, 2033, 2033, 128, False, 8),    # W = 256, one pass
+    (1, 8, 8, 1000, 1000, 128, False, 11),
+    (1, 8, 8, 1000, 5000, 128, False, 6),      # W = 64, split keys
+    (1, 32, 8, 96, 700, 128, False, 2),
+    (1, 16, 16, 2047, 2047, 64, False, 8),
+    (1, 16, 16, 2100, 2100, 64, False, 6),     # W = 272, one pass
+    (1, 8, 2, 2048, 2048, 64, False, 11),
+    (1, 2, 2, 8192, 8192, 64, False, 6),       # W = 128, split keys
+    (1, 16, 16, 4095, 4095, 32, False, 8),     # W = 512 at D = 32
+    (1, 16, 4, 1000, 1000, 64, True, 11),      # W = 128
+]
+
+
+@pytest.mark.parametrize("case", FWD_SIZE_RULE_CASES,
+                         ids=lambda c: f"B{c[0]}H{c[1]}-{c[2]}Nq{c[3]}Nkv{c[4]}D{c[5]}"
+                                       f"{'c' if c[6] else 'b'}")
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+def test_forward_size_rule(case, dtype):
+    """The forward's choice of tiling by launch size: bit for bit the tiling it
+    should take when that is forced, and within one rounding of P and O of the
+    classic 4 x 32 tiling (tiling 6 at D = 32; rel-L2: 2^-9 in bf16 and 2^-12 in fp16 for each of
+    the two roundings, doubled; LSE is computed in fp32 by both)."""
+    B, Hq, Hkv, N, Nkv, D, causal, expect = case
+    _note(f"forward size rule {case} {dtype}")
+    q, k, v, _ = (t.to(DEV) for t in make_inputs(B, Hq, Hkv, N, D, seed=N + Nkv + D, n_kv=Nkv,
+                                                   dtype=dtype))
+    rule = _ops.flash_fwd(q, k, v, causal, D ** -0.5)
+    same = _forced_forward(q, k, v, causal, expect)
+    classic = _forced_forward(q, k, v, causal, 2 if D > 32 else 6)
+    torch.cuda.synchronize()
+    assert torch.equal(rule[0], same[0]) and torch.equal(rule[1], same[1])
+    rel = float((rule[0].float() - classic[0].float()).norm() / classic[0].float().norm())
+    assert rel <= (2 ** -7 if dtype == torch.bfloat16 else 2 ** -10), rel
+    assert float((rule[1] - classic[1]).abs().max()) <= 1e-5
+
+
 def test_decoding_forward_rule_runs_the_64_query_tiling():
     """Launches of at most 32 queries (decoding, any head size) whose queries fit
     one 64-query work-group of packed heads (N_q <= 64 / P, P = gcd(Hq / Hkv,

@@ -143,38 +143,8 @@ __device__ __forceinline__ void dq_pipe16_body(const BwdArgs& a, const unsigned 
   int i_row = kv_lo;  // first key row of the next unit to fetch
   auto issue = [&](int slot) __attribute__((always_inline)) {
     const int row0 = i_row < kv_hi ? i_row : Nkv;  // past the range: zeros
-    const uint32_t vt = (uint32_t)row0 * (D * 2u) + dma.voff[0];
-    const uint32_t base = lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u;
-    uint32_t saved;
-    if constexpr (Dma::PER_WAVE == 1) {
-      asm volatile(
-          "s_mov_b32 %0, m0\n\t"
-          "s_mov_b32 m0, %4\n\t"
-          "buffer_load_dwordx4 %1, %2, 0 offen lds\n\t"
-          "s_mov_b32 m0, %5\n\t"
-          "buffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
-          "s_mov_b32 m0, %0"
-          : "=&s"(saved)
-          : "v"(vt), "s"(r_k), "s"(r_v), "s"(base), "s"(base + T::TILE * 2u)
-          : "memory");
-    } else {
-      const uint32_t vt1 = (uint32_t)row0 * (D * 2u) + dma.voff[1];
-      asm volatile(
-          "s_mov_b32 %0, m0\n\t"
-          "s_mov_b32 m0, %5\n\t"
-          "buffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
-          "s_mov_b32 m0, %6\n\t"
-          "buffer_load_dwordx4 %2, %3, 0 offen lds\n\t"
-          "s_mov_b32 m0, %7\n\t"
-          "buffer_load_dwordx4 %1, %4, 0 offen lds\n\t"
-          "s_mov_b32 m0, %8\n\t"
-          "buffer_load_dwordx4 %2, %4, 0 offen lds\n\t"
-          "s_mov_b32 m0, %0"
-          : "=&s"(saved)
-          : "v"(vt), "v"(vt1), "s"(r_k), "s"(r_v), "s"(base), "s"(base + 1024u),
-            "s"(base + T::TILE * 2u), "s"(base + T::TILE * 2u + 1024u)
-          : "memory");
-    }
+    issue_kv_unit<T::TILE * 2>(dma, r_k, r_v, (uint32_t)row0 * (D * 2u),
+                               lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
     i_row += T::KT;
   };
 #pragma unroll

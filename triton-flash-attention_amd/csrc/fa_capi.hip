@@ -74,15 +74,16 @@ int override_of(int kind, int di, int causal) {
 //   fwd : 0 = 4 waves x 32 queries, 64-key tiles; 1 = 8 waves, 64; 2 = 4 waves, 32;
 //         3 = 2 waves, 64; 4 = 4 waves, 128; 5 = 4 waves, 32-key units, software-
 //         pipelined, 2 units per barrier (D <= 64); 6 = the same, 1 unit per
-//         barrier and a 6-slot ring (three work-groups per CU); 7 = 8 waves, 32-key
-//         units, pipelined, one work-group per CU (D = 128); 8 = 8 waves as two
-//         4-wave groups that split the keys of 128 queries (D <= 64); 9 = tiling 6
+//         barrier and a 6-slot ring (three work-groups per CU; at D = 128 a 5-slot
+//         ring and two); 7 = 8 waves, 32-key units, pipelined, one work-group per CU
+//         (D = 128); 8 = 8 waves as two 4-wave groups that split the keys of 128
+//         queries; 9 = tiling 6
 //         run as a persistent grid of bin-packed jobs under the causal mask when
 //         its job plan beats the grid's modelled tail (D <= 64; fwd_launch_plan;
 //         measured slower than 6 at every shape where a plan forms, so the table
 //         does not take it); 10 = tiling 6 on 16x16x32 MFMAs (D <= 64); 11 = 10
-//         with 64-query work-groups (all D; select_fwd takes it for small causal
-//         launches at D <= 64 and for decoding)
+//         with 64-query work-groups (all D; select_fwd takes it for small launches
+//         and for decoding)
 //         (not every variant exists for every D)
 //   dkdv: 0 = 4 waves x 32 keys, 64-query tiles; 1 = 4 waves, 32; 2 = 2 waves, 64;
 //         3 = 8 waves, 64; 4 = 4 waves, 32-query units, software-pipelined (all D;
@@ -191,16 +192,58 @@ const fa::Variant* select_dq(int di, int causal, int64_t N, int64_t BH, int dt) 
   return var;
 }
 
-// Forward tiling for a launch of N queries over BH query heads. At D = 128 the
-// table's 8-wave pipelined kernel (256 queries per work-group, one per CU) is
-// faster once the launch has long query sequences and enough work-groups; for
-// short queries or small launches the 4-wave tiling is (MI355X, one box:
-// B2 H32 N8192 causal 1091 vs 1181 us, bidirectional 1941 vs 2316 us; 512
-// queries x 64 heads against 8192 keys 204 vs 218 us; 128 queries x 256 heads
-// 270 vs 223 us; B1 H16 N1024 36 vs 33 us; decoding 2-6 % slower). A tiling
-// set with fa_set_tiling is used as set.
+// Forward tilings by launch size. W = B * Hq * query tiles of 128, the
+// work-groups of the 128-query tilings; L = keys of the longest loop (all N_kv, or
+// the visible ones under the mask). A tiling set with fa_set_tiling is used as set.
+//
+// D = 128 (MI355X, one box, bf16 or fp16, us; 7 = 8 waves x 256 queries per
+// work-group and CU, the table's entry; 6 = 4 waves x 128 queries, two per CU; 8 =
+// 128 queries with two key groups, one per CU; 11 = 64 queries):
+//   * 6 by default: its work-groups are half as long as 7's, so launches whose
+//     rounds do not come out even end with less idle (7 / 6): causal B1 Hq32 Hkv8
+//     N 3001 121.5 / 81.5, N 3800 172.1 / 123.2, N 5000 223.5 / 214.8, B4 H16 N 1024
+//     34.6 / 29.6, N 4096 280.9 / 275.4; bidirectional B4 H16 N 1025 61.8 / 52.3,
+//     N 1500 87.2 / 76.3, B2 Hq32 Hkv8 N 4500 605 / 587, B8 Hq32 Hkv8 N 1100 188 / 167.
+//   * 7 where its rounds are whole and its loops long, as it stages K and V half
+//     as often: without the mask from three rounds of 256 work-groups exactly and
+//     L >= 4096 (B2 H32 N 8192 1902 / 1947, B1 H32 N 8192 892 / 907, B4 H16 N 4096
+//     495.6 / 499.6; with shorter loops B16 Hq32 Hkv8 N 1024 302 / 294); under the
+//     mask at exactly two work-groups per CU, where the heaviest-first order pairs
+//     tile t with tile T - 1 - t (B1 Hq32 N 4096 133.4 / 136.8, B1 H16 N 8192 257.4 /
+//     265.2, B1 H8 N 16384 493 / 513; with more, B2 H32 N 4096 280 / 271).
+//   * W <= 512 causal from L = 2048: 8, which deals the long tiles to whole CUs (6 /
+//     11 / 8): B1 H16 N 4096 86.9 / 88.5 / 79.4, B1 H8 N 8192 163 / - / 143, B1 H14
+//     N 4096 78.4 / 76.6 / 70.6, N 3000 55.0 / 48.5 / 48.3, B1 H8 N 4096 61.1 / 56.7 /
+//     53.9. With L > 4096 and W <= 256 splitting the keys over work-groups (tiling
+//     6) beats it: B1 H4 N 8192 89.6 / 98.5, B1 H2 N 16384 152.7 / 186.8.
+//   * Without the mask 8 takes 128 < W <= 256 (one work-group per CU; launches of
+//     one query tile keep 6 and its key ranges, B8 Hq32 Hkv8 N_q 128 against 8192 keys
+//     154.5 / 169.2): B1 H16 N 2048
+//     38.9 against 39.2 (6) and 43.6 (11), B1 H4 N 8192 131.7 / 137.3 / 155.6; past
+//     W = 256 it needs a second round (B1 H12 N 3000 90.9 / 75.1).
+//   * 11 for the smallest: causal L < 2048 up to W = 384 (6 / 11: B1 Hq32 Hkv8 N 512
+//     14.3 / 11.2, N 1024 21.9 / 19.7, B2 H16 N 1300 29.0 / 24.6; at W = 512 B4 H16
+//     N 1024 29.6 / 31.5), and W <= 128 with L < 4096 (B1 H8 N 1024 without the mask
+//     19.5 / 16.6, B1 H4 N 3000 causal 35.1 / 32.1); with longer loops 6 and its key
+//     ranges (B1 H2 N 8192 causal 63.5 / 95.8, B1 H8 N_q 1024 against 4096 33.6 / 36.8).
 constexpr int kFwdWideVariant = 7;
+constexpr int kFwdPipeVariant = 6;
+// Queries that pack (at most 32) but do not fit tiling 11, and 65-96 queries
+// without the mask, run the classic 4-wave tiling at D = 128 (tiling 2 / 6: B8 Hq32
+// Hkv8 N_q 17 against 8192 keys 54.6 / 63.9, N_q 32 63.2 / 82.7).
 constexpr int kFwdNarrowVariant = 2;
+constexpr int64_t kFwdNarrowQueries = 96;
+constexpr int64_t kFwdComputeUnits = 256;
+// Without the mask at D <= 64, from two query tiles, 128 < W <= 256 (up to 512 at D = 32, where two of
+// its work-groups fit a CU) takes the two-key-group tiling 8 in one pass; tiling
+// 6 with its keys split, as such launches ran before, / 8: D = 64 B1 H16 N 2048
+// 34.6 / 23.1, B1 H8 N 4096 53.6 / 41.4, B1 H4 N 8192 86.8 / 78.5, B1 H10 N 2500
+// 33.1 / 25.4, B1 H16 N 1500 (not split) 19.3 / 17.8; D = 32 25.5 / 18.3, 39.4 /
+// 31.8, 65.1 / 58.6, B1 H16 N 4096 58.4 / 54.6. Smaller launches of short loops
+// (W <= 128, L < 4096; causal 512 <= N < 2048 below W = 256) take tiling 11: D = 64 B1 H16
+// N 1024 14.3 / 12.1 (causal 15.8 / 12.4), B1 H8 N 2048 22.7 / 20.5; with longer
+// loops tiling 6 splits its keys (B1 H2 N 8192 52.9 / 70.2).
+
 // At D = 32 a causal launch over few heads (B*H * (query tiles + 1) < 1536)
 // takes the two-key-group forward: 8 waves per work-group as two groups that
 // split its keys, so a CU whose last long tiles run alone keeps twice the
@@ -261,7 +304,28 @@ constexpr int64_t kFwdShortQueries = 64;
 
 int fwd_pack(const fa::Variant& var, int64_t group, int64_t N);  // below
 
-const fa::Variant* select_fwd(int di, int causal, int64_t N, int64_t BH, int64_t group, int dt) {
+int64_t visible_keys(int64_t N, int64_t Nkv, int causal);  // below
+
+// select_fwd's choice at D = 128 for more queries than decoding takes (the rules above).
+int fwd_variant_d128(int causal, int64_t N, int64_t L, int64_t BH) {
+  if (N <= kFwdDecodeQueries || (!causal && N <= kFwdNarrowQueries)) return kFwdNarrowVariant;
+  const int64_t W = (N + 127) / 128 * BH;
+  const int64_t wide = (N + 255) / 256 * BH;  // tiling 7's work-groups
+  if (W <= 128) return L < 4096 ? kFwd16HalfVariant : kFwdPipeVariant;
+  if (causal) {
+    if (L < 2048) return W <= 384 ? kFwd16HalfVariant : kFwdPipeVariant;
+    if (W <= 256 && L > 4096) return kFwdPipeVariant;
+    if (W <= 512) return kFwdKeyGroupVariant;
+    return wide == 2 * kFwdComputeUnits && L > 3584 ? kFwdWideVariant : kFwdPipeVariant;
+  }
+  if (W <= 256 && N > 128) return kFwdKeyGroupVariant;
+  return wide % kFwdComputeUnits == 0 && wide >= 3 * kFwdComputeUnits && L >= 4096
+             ? kFwdWideVariant
+             : kFwdPipeVariant;
+}
+
+const fa::Variant* select_fwd(int di, int causal, int64_t N, int64_t Nkv, int64_t BH,
+                              int64_t group, int dt) {
   int index = -1;
   const int ov = override_of(fa::kFwd, di, causal);
   const fa::Variant* var = select(fa::kFwd, di, causal, ov, &index, dt);
@@ -275,13 +339,18 @@ const fa::Variant* select_fwd(int di, int causal, int64_t N, int64_t BH, int64_t
     const fa::Variant* half = pick(kFwd16HalfVariant);
     if (half != var && N <= half->rows / fwd_pack(*half, group, N)) return half;
   }
-  if (index == kFwdWideVariant) {
-    if (N >= 512 && (N + var->rows - 1) / var->rows * BH >= 128) return var;
-    return pick(kFwdNarrowVariant);
+  const int64_t L = visible_keys(N, Nkv, causal);
+  if (di == fa::head_dim_index(128)) return pick(fwd_variant_d128(causal, N, L, BH));
+  const int64_t W = (N + 127) / 128 * BH;
+  if (!causal && N > 128) {
+    if (W <= 128 && L < 4096) return pick(kFwd16HalfVariant);
+    if (W > 128 && W <= (di == fa::head_dim_index(32) ? 512 : 256))
+      return pick(kFwdKeyGroupVariant);
   }
-  if (causal && di != fa::head_dim_index(128)) {
-    const int64_t W = (N + 127) / 128 * BH;
+  if (causal) {
     if (N >= 2048 && W <= 512 && (W >= 384 || (W >= 256 && N <= 4096)))
+      return pick(kFwd16HalfVariant);
+    if (di == fa::head_dim_index(64) && N >= 512 && N < 2048 && W < 256)
       return pick(kFwd16HalfVariant);
   }
   if (di == fa::head_dim_index(32) && causal && N > 32) {
@@ -466,6 +535,13 @@ int64_t split_workspace_bytes(int nsplit, int64_t B, int64_t Hkv, int64_t Nkv, i
 // decoding shapes: ~3 work-groups per CU with long ranges beat more, shorter
 // ones (partials and merge cost more than the extra parallelism returns).
 constexpr int64_t kFwdSplitBelowWorkgroups = 512;
+// Tiling 6 without the mask, and at D = 128, splits launches of more than 128
+// queries up to one work-group per CU only: from there the partials and their merge cost more than the fuller GPU
+// returns (split / one pass, us: D = 64 B1 H16 N 3000 57.0 / 52.1, N 3500 77.2 /
+// 63.8; D = 128 B1 H12 N 4096 120.6 / 109.2). The two-key-group tiling, which
+// splits its keys inside the work-group, does not split there at all (D = 128
+// causal B1 H16 N 2048 46.3 / 31.5, B1 H12 N 4096 88.5 / 61.1).
+constexpr int64_t kFwdLateSplitBelow = 257;
 constexpr int64_t kFwdSplitTargetWorkgroups = 768;
 // The 64-query forward (kFewSplits) decodes at D >= 64 faster with one
 // work-group per CU than with three: its key ranges run quicker, so partials
@@ -507,10 +583,10 @@ int64_t visible_keys(int64_t N, int64_t Nkv, int causal) {
 // add empty work-groups and partials (B1 Hq32 Hkv8, 128 queries against 32768
 // keys, D128, causal: 24 ranges, of which 23 were empty). A launch that does
 // not split keeps the whole key range.
-FwdSplit key_split(int64_t wgs, int64_t Nkv, int64_t visible, bool can_split,
+FwdSplit key_split(int64_t wgs, int64_t Nkv, int64_t visible, int64_t below,
                    int64_t target = kFwdSplitTargetWorkgroups) {
   const int whole = (int)((Nkv + 127) / 128 * 128);
-  if (wgs >= kFwdSplitBelowWorkgroups || !can_split) return {1, whole};
+  if (wgs >= below) return {1, whole};
   int64_t s = (target + wgs - 1) / wgs;
   s = std::min<int64_t>(s, std::max<int64_t>(1, visible / kFwdMinSplitKeys));
   s = std::min<int64_t>(s, kMaxFwdSplit);
@@ -524,15 +600,19 @@ FwdSplit fwd_split(const fa::Variant& var, int64_t B, int64_t Hq, int64_t N, int
   const int64_t rows = var.rows / pack;  // query rows per head and work-group
   const int64_t target = (var.flags & fa::kFewSplits) && D >= 64 ? kFwdSplitTargetFew
                                                                 : kFwdSplitTargetWorkgroups;
-  return key_split((N + rows - 1) / rows * B * Hq / pack, Nkv, visible_keys(N, Nkv, causal),
-                   var.flags & fa::kSplitsKv, target);
+  int64_t below = var.flags & fa::kSplitsKv ? kFwdSplitBelowWorkgroups : 0;
+  if ((var.flags & fa::kLateSplit) && (D == 128 || !causal) && N > 128)
+    below = std::min(below, kFwdLateSplitBelow);
+  if ((var.flags & fa::kKeyGroups) && (D == 128 || !causal)) below = 0;
+  return key_split((N + rows - 1) / rows * B * Hq / pack, Nkv, visible_keys(N, Nkv, causal), below,
+                   target);
 }
 
 // dQ: the same split of its key loop; the partials (fp32 dQ) are summed.
 FwdSplit dq_split(const fa::Variant& var, int64_t B, int64_t Hq, int64_t N, int64_t Nkv,
                   int causal) {
   return key_split((N + var.rows - 1) / var.rows * B * Hq, Nkv, visible_keys(N, Nkv, causal),
-                   true);
+                   kFwdSplitBelowWorkgroups);
 }
 
 int64_t dq_workspace_bytes(const FwdSplit& sp, int64_t B, int64_t Hq, int64_t N, int64_t D) {
@@ -751,7 +831,7 @@ static int fwd_check(int dt, const char* name, const fa_half_t* q, const fa_half
   if ((rc = check_kv_length(Nkv, D))) return rc;
   if ((rc = check_aligned(name, {q, k, v, o, lse}))) return rc;
   if ((rc = check_scale(scale))) return rc;
-  *var = select_fwd(fa::head_dim_index(D), causal, N, B * Hq, Hq / Hkv, dt);
+  *var = select_fwd(fa::head_dim_index(D), causal, N, Nkv, B * Hq, Hq / Hkv, dt);
   if (!*var) return fail(FA_ERR_BAD_TILING, "%s: no kernel for the selected tiling", name);
   const FwdSplit sp = fwd_split(**var, B, Hq, N, Nkv, D, fwd_pack(**var, Hq / Hkv, N), causal);
   *need = fwd_workspace_bytes(sp, B, Hq, N, D);
@@ -813,7 +893,7 @@ int64_t fa_fwd_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t N_q, 
   // Enough for either element type (their tilings can differ when overridden).
   int64_t bytes = 0;
   for (int dt : {fa::kF16, fa::kBF16}) {
-    const fa::Variant* var = select_fwd(fa::head_dim_index(D), causal, N_q, B * Hq, Hq / Hkv, dt);
+    const fa::Variant* var = select_fwd(fa::head_dim_index(D), causal, N_q, N_kv, B * Hq, Hq / Hkv, dt);
     if (!var) return fail(FA_ERR_BAD_TILING, "fa_fwd_workspace_bytes: no kernel for the selected tiling");
     const FwdSplit sp = fwd_split(*var, B, Hq, N_q, N_kv, D, fwd_pack(*var, Hq / Hkv, N_q), causal);
     bytes = std::max(bytes, fwd_workspace_bytes(sp, B, Hq, N_q, D));
@@ -827,7 +907,7 @@ int fa_fwd_plan_info(int64_t B, int64_t Hq, int64_t Hkv, int64_t N_q, int64_t N_
   int rc = check_common(B, Hq, Hkv, N_q, D);
   if (rc) return rc;
   if ((rc = check_kv_length(N_kv, D))) return rc;
-  const fa::Variant* var = select_fwd(fa::head_dim_index(D), causal, N_q, B * Hq, Hq / Hkv, fa::kF16);
+  const fa::Variant* var = select_fwd(fa::head_dim_index(D), causal, N_q, N_kv, B * Hq, Hq / Hkv, fa::kF16);
   if (!var) return fail(FA_ERR_BAD_TILING, "fa_fwd_plan_info: no kernel for the selected tiling");
   const int pack = fwd_pack(*var, Hq / Hkv, N_q);
   const FwdSplit sp = fwd_split(*var, B, Hq, N_q, N_kv, D, pack, causal);

@@ -467,6 +467,46 @@ struct DmaStager {
   }
 };
 
+// The K rows and the V rows of one key unit -> LDS tiles at byte address
+// `base` (K) and base + TILE_BYTES (V), this wave's one or two 1 KiB pieces of
+// each, in one asm block. `row_off` is the unit's first row as a byte offset.
+template <int TILE_BYTES, class Dma>
+__device__ __forceinline__ void issue_kv_unit(const Dma& dma, int4v r_k, int4v r_v,
+                                              uint32_t row_off, uint32_t base) {
+  static_assert(Dma::PER_WAVE == 1 || Dma::PER_WAVE == 2, "one or two tile pieces per wave");
+  const uint32_t vt = row_off + dma.voff[0];
+  uint32_t saved;
+  if constexpr (Dma::PER_WAVE == 1) {
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %4\n\t"
+        "buffer_load_dwordx4 %1, %2, 0 offen lds\n\t"
+        "s_mov_b32 m0, %5\n\t"
+        "buffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "v"(vt), "s"(r_k), "s"(r_v), "s"(base), "s"(base + TILE_BYTES)
+        : "memory");
+  } else {
+    const uint32_t vt1 = row_off + dma.voff[1];
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %5\n\t"
+        "buffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
+        "s_mov_b32 m0, %6\n\t"
+        "buffer_load_dwordx4 %2, %3, 0 offen lds\n\t"
+        "s_mov_b32 m0, %7\n\t"
+        "buffer_load_dwordx4 %1, %4, 0 offen lds\n\t"
+        "s_mov_b32 m0, %8\n\t"
+        "buffer_load_dwordx4 %2, %4, 0 offen lds\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "v"(vt), "v"(vt1), "s"(r_k), "s"(r_v), "s"(base), "s"(base + 1024u),
+          "s"(base + TILE_BYTES), "s"(base + TILE_BYTES + 1024u)
+        : "memory");
+  }
+}
+
 // Work-group order: tile-major, head-minor. With B*H a multiple of 8 every
 // tile of head h lands on XCD (h % 8) (work-groups are dealt to the 8 XCDs
 // round-robin), so the K/V of a head stays in one XCD's L2.

@@ -378,13 +378,26 @@ __global__ __launch_bounds__(64 * NW) void fwd_kernel(FwdArgs a) {
 // to the 8-unit unroll; padding units are masked the same way.
 // ---------------------------------------------------------------------------
 // UPS = units per barrier step: 2 (8-slot ring, 64 KiB at D = 64, two
-// work-groups per CU) or 1 (6-slot ring, 48 KiB, three work-groups per CU).
+// work-groups per CU) or 1 (6-slot ring, 48 KiB, three work-groups per CU; at
+// D = 128 a 5-slot ring of 80 KiB, two per CU, each wave moving two 1 KiB pieces
+// of K and of V per unit).
+// At D = 128 the two 4-wave work-groups run the same MFMAs per CU as one 8-wave
+// work-group of 256 queries and twice its K/V staging, but the launch is dealt
+// in 128-query work-groups with barriers of their own: a ragged or causal
+// launch ends with less idle. MI355X, one box, 8 waves vs 2 x 4, us: bf16 causal
+// B1 Hq32 Hkv8 N 2048 72.4 / 47.0, N 3001 121.5 / 81.5, N 3800 172.1 / 123.2,
+// N 5000 223.5 / 214.8; B4 H16 N 4096 280.9 / 275.4; bidirectional B4 H16 N 1025
+// 61.8 / 52.3, N 4096 495.6 / 499.6, B2 H32 N 8192 1902 / 1947 (7.8 TFLOP at
+// 1.13 PFLOP/s: with whole rounds of long loops the staging it saves decides).
 // KG = key groups: with KG = 2 the NW waves form two groups of NW/2 that
 // serve the same queries, each streaming one half of the work-group's key
 // range through a ring of its own with the UPS = 1 pipeline; the two partial
 // results are merged through LDS at the end. That halves the longest
 // work-group of a causal launch whose end is set by its last query tiles
 // (few heads: the tiles reading all keys run alone on the GPU at the end).
+// At D = 128 (two 80 KiB rings, one work-group per CU): causal B1 H16 N 4096 79.4
+// us against 86.9 with the two 4-wave work-groups and 116.2 with 8 waves of
+// 256 queries; B1 H8 N 8192 136.6 / 157.5 / 176.3.
 template <int D, int NW, int UPS, int KG = 1>
 struct FwdPipeTile {
   static constexpr int NWG = NW / KG;  // waves per key group
@@ -393,13 +406,18 @@ struct FwdPipeTile {
   static constexpr int KT = 32;
   static constexpr int TILE = KT * D;  // halves of the K (or V) unit
   static constexpr int STAGE = 2 * TILE;
-  static constexpr int NSTAGE = UPS == 2 ? 8 : 6;
-  static constexpr int AHEAD = UPS == 2 ? 5 : 4;  // units issued before step 0
+  // One unit per barrier: 6 slots, but 5 where two rings of 16 KiB units
+  // (D = 128 with two key groups, or two work-groups per CU) share the 160 KiB.
+  static constexpr int NSTAGE = UPS == 2 ? 8 : (D == 128 && (KG == 2 || NW == 4) ? 5 : 6);
+  // Units issued before step 0, and those of them that may be in flight at a
+  // barrier (a step reads up to two units ahead of its own).
+  static constexpr int AHEAD = UPS == 2 ? 5 : NSTAGE - 2;
+  static constexpr int IN_FLIGHT = UPS == 2 ? 2 : AHEAD - 2;
   // Work-groups per CU: three 4-wave work-groups with one unit per barrier,
-  // two with two; at D = 128 (16 KiB units, a 96 KiB ring) a work-group takes
-  // a CU alone; with two key groups (two rings) two at D = 32 and one at D = 64.
+  // two with two; at D = 128 (16 KiB units) one 8-wave or two 4-wave ones;
+  // with two key groups (two rings) two at D = 32 and one above.
   static constexpr int WGS_PER_CU =
-      KG == 2 ? (D <= 32 ? 2 : 1) : (NW == 8 || D == 128 ? 1 : (UPS == 2 ? 2 : 3));
+      KG == 2 ? (D <= 32 ? 2 : 1) : (NW == 8 ? 1 : (D == 128 || UPS == 2 ? 2 : 3));
   static constexpr int WAVES_PER_SIMD = WGS_PER_CU * NW / 4;
   static_assert(UPS == 1 || UPS == 2, "units per step");
   static_assert(KG == 1 || (KG == 2 && UPS == 1 && NW == 8), "two 4-wave key groups, one unit each");
@@ -409,9 +427,9 @@ template <int D, int NW, int UPS, int KG = 1>
 constexpr bool fwd_pipe_tiling_ok() {
   using T = FwdPipeTile<D, NW, UPS, KG>;
   constexpr int instr = T::TILE * 2 / 1024;
-  return (T::TILE * 2) % 1024 == 0 && instr <= T::NWG && T::NWG % instr == 0 &&
-         T::WGS_PER_CU * KG * T::NSTAGE * T::STAGE * 2 <= 160 * 1024 &&
-         (KG == 1 ? (D <= 64 || NW == 8) : D <= 64);
+  return (T::TILE * 2) % 1024 == 0 &&
+         ((instr <= T::NWG && T::NWG % instr == 0) || (UPS == 1 && instr == 2 * T::NWG)) &&
+         T::WGS_PER_CU * KG * T::NSTAGE * T::STAGE * 2 <= 160 * 1024 && (D <= 64 || UPS == 1);
 }
 
 #ifndef FA_FWD_LEAD
@@ -446,9 +464,8 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
                                               int head_blk, half_t* lds_all) {
   using T = FwdPipeTile<D, NW, UPS, KG>;
   using Dma = DmaStager<D, T::KT, T::NWG>;
-  static_assert(Dma::PER_WAVE == 1, "one tile piece per wave");
   constexpr int NS = T::NSTAGE;
-  constexpr int IPU = 2;  // this wave's DMA instructions per unit: K, V
+  constexpr int IPU = 2 * Dma::PER_WAVE;  // this wave's DMA instructions per unit: K, V
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -511,19 +528,8 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
   int i_row = kv_lo;  // first key row of the next unit to fetch
   auto issue = [&](int slot) __attribute__((always_inline)) {
     const int row0 = i_row < kv_hi ? i_row : Nkv;  // past the range: zeros
-    const uint32_t vt = (uint32_t)row0 * (D * 2u) + dma.voff[0];
-    const uint32_t base = lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u;
-    uint32_t saved;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %4\n\t"
-        "buffer_load_dwordx4 %1, %2, 0 offen lds\n\t"
-        "s_mov_b32 m0, %5\n\t"
-        "buffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(saved)
-        : "v"(vt), "s"(r_k), "s"(r_v), "s"(base), "s"(base + T::TILE * 2u)
-        : "memory");
+    issue_kv_unit<T::TILE * 2>(dma, r_k, r_v, (uint32_t)row0 * (D * 2u),
+                               lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
     i_row += T::KT;
   };
 #pragma unroll
@@ -540,8 +546,8 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
     for (int i = tid - gk * 64 * T::NWG; i < T::TILE / 8; i += 64 * T::NWG)
       *reinterpret_cast<u32x4*>(zs + 8 * i) = z;
   }
-  // Units 0 .. AHEAD-3 landed (the last two in flight), zeros written.
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(2 * IPU) : "memory");
+  // All but the last IN_FLIGHT units landed, zeros written.
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(T::IN_FLIGHT * IPU) : "memory");
 
   int k_off[D / 16];  // row reads of K: row row_perm(ql), chunk 2*kk + g
 #pragma unroll
@@ -747,14 +753,14 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
 
   // One barrier step: UPS units; issues the units AHEAD.. ahead into the
   // slots of units finished before the last barrier, then waits for all but
-  // the two most recent units (the next step reads up to 2 units ahead).
+  // the IN_FLIGHT most recent units (the next step reads up to 2 units ahead).
   auto step = [&](auto p_c) __attribute__((always_inline)) {
     constexpr int P = decltype(p_c)::value;
     static_for_fwd_issue<UPS>([&](auto e_c) {
       issue((UPS * P + T::AHEAD + decltype(e_c)::value) % NS);
     });
     static_for_fwd_issue<UPS>([&](auto e_c) { body(fic<UPS * P + decltype(e_c)::value>{}); });
-    wait_vm_and_barrier<2 * IPU>();
+    wait_vm_and_barrier<T::IN_FLIGHT * IPU>();
   };
 
   static_assert(NS % UPS == 0, "whole steps per ring turn");
@@ -900,39 +906,8 @@ __device__ __forceinline__ void fwd_pipe16_body(const FwdArgs& a, int split, int
   int i_row = kv_lo;  // first key row of the next unit to fetch
   auto issue = [&](int slot) __attribute__((always_inline)) {
     const int row0 = i_row < kv_hi ? i_row : Nkv;  // past the range: zeros
-    const uint32_t vt = (uint32_t)row0 * (D * 2u) + dma.voff[0];
-    const uint32_t base = lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u;
-    uint32_t saved;
-    if constexpr (Dma::PER_WAVE == 1) {
-      asm volatile(
-          "s_mov_b32 %0, m0\n\t"
-          "s_mov_b32 m0, %4\n\t"
-          "buffer_load_dwordx4 %1, %2, 0 offen lds\n\t"
-          "s_mov_b32 m0, %5\n\t"
-          "buffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
-          "s_mov_b32 m0, %0"
-          : "=&s"(saved)
-          : "v"(vt), "s"(r_k), "s"(r_v), "s"(base), "s"(base + T::TILE * 2u)
-          : "memory");
-    } else {
-      // D = 128: the wave's two consecutive 1 KiB pieces of the K and the V unit
-      const uint32_t vt1 = (uint32_t)row0 * (D * 2u) + dma.voff[1];
-      asm volatile(
-          "s_mov_b32 %0, m0\n\t"
-          "s_mov_b32 m0, %5\n\t"
-          "buffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
-          "s_mov_b32 m0, %6\n\t"
-          "buffer_load_dwordx4 %2, %3, 0 offen lds\n\t"
-          "s_mov_b32 m0, %7\n\t"
-          "buffer_load_dwordx4 %1, %4, 0 offen lds\n\t"
-          "s_mov_b32 m0, %8\n\t"
-          "buffer_load_dwordx4 %2, %4, 0 offen lds\n\t"
-          "s_mov_b32 m0, %0"
-          : "=&s"(saved)
-          : "v"(vt), "v"(vt1), "s"(r_k), "s"(r_v), "s"(base), "s"(base + 1024u),
-            "s"(base + T::TILE * 2u), "s"(base + T::TILE * 2u + 1024u)
-          : "memory");
-    }
+    issue_kv_unit<T::TILE * 2>(dma, r_k, r_v, (uint32_t)row0 * (D * 2u),
+                               lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
     i_row += T::KT;
   };
 #pragma unroll
@@ -946,7 +921,7 @@ __device__ __forceinline__ void fwd_pipe16_body(const FwdArgs& a, int split, int
     const u32x4 z = {zr, zr, zr, zr};
     for (int i = tid; i < T::TILE / 8; i += T::NT) *reinterpret_cast<u32x4*>(zs + 8 * i) = z;
   }
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(2 * IPU) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(T::IN_FLIGHT * IPU) : "memory");
 
   // Row reads of K (A operand of S^T): key row 16 kb + rows16(c16), chunk 4 kd + sg.
   int k_off[2][KD];
@@ -1192,12 +1167,12 @@ __device__ __forceinline__ void fwd_pipe16_body(const FwdArgs& a, int split, int
 
   // One barrier step per unit (tiling 6's pipeline): issue the unit AHEAD
   // ahead into the slot of the unit finished before the last barrier, run the
-  // body, wait for all but the two most recent units.
+  // body, wait for all but the IN_FLIGHT most recent units.
   auto step = [&](auto p_c) __attribute__((always_inline)) {
     constexpr int Pp = decltype(p_c)::value;
     issue((Pp + T::AHEAD) % NS);
     body(fic<Pp>{});
-    wait_vm_and_barrier<2 * IPU>();
+    wait_vm_and_barrier<T::IN_FLIGHT * IPU>();
   };
   if (npad > 0) {
     fwd_static_for<0, NS>([&](auto p_c) {
@@ -1543,8 +1518,9 @@ static const Variant kFwdVariants[] = {
     FA_FWD_VARIANT(2, 64),
     FA_FWD_VARIANT(4, 128),
     {4, 128, 32, {FA_ENTRIES(fwd_pipe_entry, F16, 4, 2), FA_NO_ENTRIES}, kSplitsKv},
+    // 6 (all D; at D = 128 two work-groups per CU)
     {4, 128, 32, {FA_ENTRIES(fwd_pipe_entry, F16, 4, 1), FA_ENTRIES(fwd_pipe_entry, BF16, 4, 1)},
-     kSplitsKv},
+     kSplitsKv | kLateSplit},
     {8, 256, 32, {FA_ENTRIES(fwd_pipe_entry, F16, 8, 1), FA_ENTRIES(fwd_pipe_entry, BF16, 8, 1)},
      kSplitsKv},
     {8, 128, 32,

@@ -121,7 +121,7 @@ struct Variant {
   int rows;
   int tile;
   void* fn[2][3][2];  // [element type: fp16, bf16][D index: 32, 64, 128][causal]; null = not compiled
-  int flags;          // kFusesDelta, kSplitsKv, kPairs, kKeyGroups, kJobs, kFewSplits
+  int flags;          // kFusesDelta, kSplitsKv, kPairs, kKeyGroups, kJobs, kFewSplits, kLateSplit
   int per_cu = 0;     // kJobs: work-groups resident per CU (the plan's slots per CU)
 };
 
@@ -152,6 +152,9 @@ constexpr int kJobs = 16;
 // The forward variant's split-KV launches at D >= 64 aim at one work-group per
 // CU (fewer, longer key ranges) instead of three.
 constexpr int kFewSplits = 32;
+// The forward variant splits its keys into ranges only up to 256 work-groups
+// (at D = 128 and without the mask); the others below 512.
+constexpr int kLateSplit = 64;
 
 // Most key ranges a split-KV forward uses; its merge holds one partial per
 // range in registers.

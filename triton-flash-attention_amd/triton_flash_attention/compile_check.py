@@ -30,11 +30,14 @@ SUPPORTED_ARCHS = ("gfx950",)
 
 # Kernel instances the default tiling table (kDefault in csrc/fa_capi.hip) and
 # its shape rules select, as demangled name prefixes, for D = 32, 64, 128, both
-# mask modes and both element types (at D = 128 the forward takes the 8-wave
-# pipelined kernel, and the 4-wave one for short queries; at D = 32 causal
-# launches over few heads take the two-key-group forward, and the other causal
-# launches from 512 queries its 16x16x32 form; small causal launches at D <= 64,
-# and decoding at every head size, the 16x16x32 form with 64-query work-groups;
+# mask modes and both element types (at D = 128 the forward takes the 4-wave
+# pipelined kernel, the 8-wave one where its rounds are whole, the two-key-group
+# one for launches of about one work-group per CU, and the classic one for short
+# queries; at D = 32 causal launches over few heads take the two-key-group
+# forward, and the other causal launches from 512 queries its 16x16x32 form; at
+# D <= 64 small launches without the mask the two-key-group forward; the smallest
+# launches, and decoding at every head size, the 16x16x32 form with 64-query
+# work-groups;
 # at D <= 64 a backward
 # whose dK/dV launch splits next to a short dQ launch runs the combined dK/dV + dQ
 # kernel; dQ takes the pipelined kernel at D = 128 for short causal launches, and
@@ -48,6 +51,8 @@ def _defaults() -> tuple[str, ...]:
             names += [f"fa::fwd_pipe_kernel<32, {c}, 4, 1, {e}, 1>",
                       f"fa::fwd_pipe_kernel<64, {c}, 4, 1, {e}, 1>",
                       f"fa::fwd_pipe_kernel<128, {c}, 8, 1, {e}, 1>", f"fa::fwd_kernel<128, {c}, 4, 32, {e}>",
+                      f"fa::fwd_pipe_kernel<128, {c}, 4, 1, {e}, 1>",
+                      f"fa::fwd_pipe_kernel<128, {c}, 8, 1, {e}, 2>",
                       f"fa::dkdv_pipe_kernel<32, {c}, 4, {e}>", f"fa::dkdv_pipe_kernel<64, {c}, 4, {e}>",
                       f"fa::dkdv_pipe_kernel<128, {c}, 4, {e}>", f"fa::dkdv_pipe16_kernel<64, {c}, 4, {e}>",
                       f"fa::dkdv_pipe16_kernel<32, false, 4, {e}>",
@@ -67,6 +72,7 @@ def _defaults() -> tuple[str, ...]:
                 names += [f"fa::dq_pipe_kernel<128, true, 4, {e}, {t}>" for t in ("false", "true")]
                 names += [f"fa::dq_pipe16_kernel<64, true, 4, {e}, {t}>" for t in ("false", "true")]
         names.append(f"fa::fwd_pipe_kernel<32, true, 8, 1, {e}, 2>")
+        names += [f"fa::fwd_pipe_kernel<{d}, false, 8, 1, {e}, 2>" for d in (32, 64)]
         names.append(f"fa::fwd_pipe16_kernel<32, true, {e}, 2>")
         names += [f"fa::fwd_pipe16_kernel<{d}, {c}, {e}, 1>"
                   for d in (32, 64, 128) for c in ("false", "true")]
