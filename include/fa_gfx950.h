@@ -49,7 +49,7 @@
 extern "C" {
 #endif
 
-#define FA_ABI_VERSION 7
+#define FA_ABI_VERSION 8
 
 /* Error codes returned before any HIP call is made. */
 #define FA_OK 0
@@ -61,6 +61,7 @@ extern "C" {
 #define FA_ERR_BAD_SCALE (-5)          /* scale not finite or not > 0            */
 #define FA_ERR_BAD_TILING (-6)         /* no compiled kernel for this tiling     */
 #define FA_ERR_MISALIGNED (-7)         /* a tensor pointer is not 16-byte aligned */
+#define FA_ERR_BAD_STRIDE (-8)         /* a stride the kernels cannot address     */
 
 /* 16-bit storage type of the tensor elements: IEEE binary16 for the entry
  * points without a suffix, bfloat16 for the _bf16 ones. */
@@ -305,6 +306,44 @@ int fa_bwd_bf16(const fa_half_t* q, const fa_half_t* k, const fa_half_t* v,
                 int64_t B, int64_t Hq, int64_t Hkv, int64_t N_q, int64_t N_kv, int64_t D,
                 float scale, int causal, void* workspace, int64_t workspace_bytes,
                 void* stream);
+
+/* The forward and the whole backward on strided tensors of any head size D that
+ * is a multiple of 8 up to 128: what fa_fwd_ws and fa_bwd compute on contiguous
+ * copies zero-padded to the kernel width (the smallest of 32, 64 and 128 that
+ * holds D), without the copies. q, k, v and dO may be any [B, H, N, D] views
+ * whose last dimension is contiguous, such as the transposed projections of a
+ * model or the filled part of a key/value cache: `strides` holds the batch, head
+ * and row stride, in elements, of q (and dO, laid out as q), then of k and v. Each
+ * must be a multiple of 8 and not negative, head strides below 2^35, row strides
+ * at least D, and (rows + 4096) * row stride * 2 < 2^31 (FA_ERR_BAD_STRIDE,
+ * FA_ERR_TOO_LARGE). o, dq, dk, dv, lse and delta are contiguous. Workspaces:
+ * fa_fwd_workspace_bytes and fa_bwd_workspace_bytes of the kernel width. No
+ * counterpart in the reference, which copies its inputs with .contiguous()
+ * (attention.py:727, 841-843) and serves head sizes 32, 64 and 128 (657-661). */
+int fa_fwd_view(const fa_half_t* q, const fa_half_t* k, const fa_half_t* v,
+                fa_half_t* o, float* lse, const int64_t* strides,
+                int64_t B, int64_t Hq, int64_t Hkv, int64_t N_q, int64_t N_kv, int64_t D,
+                float scale, int causal, void* workspace, int64_t workspace_bytes,
+                void* stream);
+int fa_fwd_view_bf16(const fa_half_t* q, const fa_half_t* k, const fa_half_t* v,
+                     fa_half_t* o, float* lse, const int64_t* strides,
+                     int64_t B, int64_t Hq, int64_t Hkv, int64_t N_q, int64_t N_kv, int64_t D,
+                     float scale, int causal, void* workspace, int64_t workspace_bytes,
+                     void* stream);
+int fa_bwd_view(const fa_half_t* q, const fa_half_t* k, const fa_half_t* v,
+                const fa_half_t* o, const fa_half_t* dO, const float* lse,
+                float* delta, fa_half_t* dq, fa_half_t* dk, fa_half_t* dv,
+                const int64_t* strides,
+                int64_t B, int64_t Hq, int64_t Hkv, int64_t N_q, int64_t N_kv, int64_t D,
+                float scale, int causal, void* workspace, int64_t workspace_bytes,
+                void* stream);
+int fa_bwd_view_bf16(const fa_half_t* q, const fa_half_t* k, const fa_half_t* v,
+                     const fa_half_t* o, const fa_half_t* dO, const float* lse,
+                     float* delta, fa_half_t* dq, fa_half_t* dk, fa_half_t* dv,
+                     const int64_t* strides,
+                     int64_t B, int64_t Hq, int64_t Hkv, int64_t N_q, int64_t N_kv, int64_t D,
+                     float scale, int causal, void* workspace, int64_t workspace_bytes,
+                     void* stream);
 
 /* Forward that allocates nothing: fa_fwd_ws's computation with the split-KV
  * partials kept in a device array inside the library (64 MiB per GPU, held

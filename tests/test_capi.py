@@ -451,3 +451,42 @@ def test_native_binding_loads_and_takes_the_library_entry_points(lib):
         _native._module.attention(q, q, q, True, 0.125)
     with pytest.raises(RuntimeError, match="must be 4-D"):
         _native._module.attention(q[0], q[0], q[0], True, 0.125)
+
+
+def test_strided_entries_check_strides_and_head_size(lib):
+    """fa_fwd_view / fa_bwd_view take a head size that is a multiple of 8 up to
+    128 and strides the kernels can address, and reject the rest before any HIP
+    call; the scale is checked last, as in fa_fwd_ws."""
+    def fwd(strides=(4096, 2048, 64) * 2, D=64, scale=0.125, entry=lib.fa_fwd_view, q=P):
+        a = (ctypes.c_int64 * 6)(*strides) if strides else None
+        return entry(q, P, P, P, P, a, 1, 2, 2, 32, 32, D, scale, 0, None, 0, None)
+
+    def bwd(strides, dO=P):
+        a = (ctypes.c_int64 * 6)(*strides)
+        return lib.fa_bwd_view(*[P] * 4, dO, *[P] * 5, a, 1, 2, 2, 32, 32, 64, -1.0, 0, None, 0,
+                               None)
+
+    good = (4096, 2048, 64)
+    assert fwd(scale=-1.0) == _lib.FA_ERR_BAD_SCALE       # everything before is accepted
+    assert fwd(scale=-1.0, D=40) == _lib.FA_ERR_BAD_SCALE
+    assert fwd(scale=-1.0, strides=(0, 0, 64) * 2) == _lib.FA_ERR_BAD_SCALE  # broadcast heads
+    assert fwd(scale=-1.0, strides=good + (0, 8, 128)) == _lib.FA_ERR_BAD_SCALE
+    assert fwd(scale=-1.0, entry=lib.fa_fwd_view_bf16) == _lib.FA_ERR_BAD_SCALE
+    assert fwd(strides=None) == _lib.FA_ERR_NULL_POINTER
+    assert fwd(q=None) == _lib.FA_ERR_NULL_POINTER
+    assert fwd(q=P + 8) == _lib.FA_ERR_MISALIGNED
+    for D in (0, 4, 20, 136):
+        assert fwd(D=D) == _lib.FA_ERR_HEAD_DIM, D
+    for bad in ((4096, 2048, 63), (4096, 2047, 64), (4095, 2048, 64), (4096, 2048, 56),
+                (-8, 2048, 64), (4096, -8, 64), (4096, 1 << 35, 64)):
+        assert fwd(strides=bad + good) == _lib.FA_ERR_BAD_STRIDE, bad
+        assert "q and dO" in _lib.last_error()
+        assert fwd(strides=good + bad) == _lib.FA_ERR_BAD_STRIDE, bad
+        assert "k and v" in _lib.last_error()
+    row = (1 << 30) // (32 + 4096) // 8 * 8
+    assert fwd(strides=(0, 0, row) * 2, scale=-1.0) == _lib.FA_ERR_BAD_SCALE
+    assert fwd(strides=(0, 0, row + 8) * 2) == _lib.FA_ERR_TOO_LARGE
+    assert bwd(good * 2) == _lib.FA_ERR_BAD_SCALE
+    assert bwd(good + (4096, 2048, 0)) == _lib.FA_ERR_BAD_STRIDE
+    assert bwd(good * 2, dO=None) == _lib.FA_ERR_NULL_POINTER
+    assert bwd(good * 2, dO=P + 2) == _lib.FA_ERR_MISALIGNED

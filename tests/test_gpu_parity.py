@@ -32,7 +32,13 @@ from fa_testutil import (
     torch_reference_fp32,
 )
 from oracle import oracle
-from triton_flash_attention import _lib, _ops, explain_dispatch, scaled_dot_product_attention
+from triton_flash_attention import (
+    TritonAttention,
+    _lib,
+    _ops,
+    explain_dispatch,
+    scaled_dot_product_attention,
+)
 
 pytestmark = pytest.mark.gpu
 
@@ -2237,3 +2243,115 @@ def test_random_decode_envelope_matches_oracle(case):
     split-KV forward and split dQ in combination with padded head sizes,
     bf16 and custom scales, through the public API against the oracle."""
     test_random_envelope_matches_oracle(case)
+
+
+# ---------------------------------------------------------------------------
+# Strided operands and head sizes below the kernel width, read as they stand
+# ---------------------------------------------------------------------------
+def _laid_out(t, layout):
+    """A tensor of t's values whose strides are those of `layout`."""
+    B, H, N, D = t.shape
+    if layout == "heads":
+        return t.clone()
+    if layout == "tokens":       # a projection [B, N, H, D], transposed
+        return t.transpose(1, 2).contiguous().transpose(1, 2)
+    if layout == "fused":        # one of three in [B, N, 3, H, D]
+        x = torch.full((B, N, 3, H, D), float("nan"), dtype=t.dtype, device=t.device)
+        x[:, :, 1] = t.transpose(1, 2)
+        return x[:, :, 1].transpose(1, 2)
+    if layout == "cache":        # the filled part of a longer cache
+        x = torch.full((B, H, N + 37, D), float("nan"), dtype=t.dtype, device=t.device)
+        x[:, :, 5:N + 5] = t
+        return x[:, :, 5:N + 5]
+    if layout == "wide":         # leading columns of wider rows
+        x = torch.full((B, H, N, D + 24), float("nan"), dtype=t.dtype, device=t.device)
+        x[..., :D] = t
+        return x[..., :D]
+    if layout == "odd":          # rows at an odd stride: copied
+        x = torch.full((B, H, N, D + 3), float("nan"), dtype=t.dtype, device=t.device)
+        x[..., :D] = t
+        return x[..., :D]
+    if layout == "shifted":      # not 16-byte aligned: copied
+        x = torch.full((t.numel() + 4,), float("nan"), dtype=t.dtype, device=t.device)
+        x[4:] = t.flatten()
+        return x[4:].view(t.shape)
+    assert layout == "columns"   # columns apart: copied
+    return t.transpose(2, 3).contiguous().transpose(2, 3)
+
+
+LAYOUTS = ("heads", "tokens", "fused", "cache", "wide", "odd", "shifted", "columns")
+VIEW_CASES = [
+    # (B, Hq, Hkv, N_q, N_kv, D, causal)
+    (2, 4, 2, 129, 129, 64, True),        # combined dK/dV + dQ launch
+    (1, 8, 1, 1, 3000, 128, False),       # packed decoding, split keys
+    (2, 3, 3, 77, 300, 32, False),
+    (1, 4, 4, 260, 260, 128, True),
+    (2, 4, 4, 700, 700, 80, False),
+    (1, 8, 2, 515, 515, 96, True),        # split dK/dV
+    (1, 4, 4, 40, 4100, 40, False),       # split forward and dQ
+    (2, 2, 2, 65, 65, 8, True),
+    (1, 6, 3, 200, 333, 24, False),
+    (1, 2, 2, 150, 150, 120, True),
+    (16, 32, 32, 256, 256, 64, True),     # 16x16x32 dK/dV and dQ
+    (4, 32, 32, 900, 900, 24, False),     # the same at D = 32
+    (2, 32, 8, 16, 300, 104, False),      # classic short-query backward
+]
+
+
+@pytest.mark.parametrize("case", VIEW_CASES,
+                         ids=lambda c: f"H{c[1]}-{c[2]}Nq{c[3]}Nkv{c[4]}D{c[5]}"
+                                       f"{'c' if c[6] else 'b'}")
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+def test_strided_and_narrow_operands_match_contiguous_copies(case, dtype):
+    """Every layout, alone and mixed over q, k, v and dO, gives bit for bit what
+    the Python Function computes on contiguous, zero-padded copies: O, dQ, dK and
+    dV. The memory around the operands holds NaN, which no result may pick up."""
+    B, Hq, Hkv, N, Nkv, D, causal = case
+    g = torch.Generator().manual_seed(N + Nkv + D)
+    mk = lambda h, n, d: torch.randn((B, h, n, d), generator=g).to(dtype).to(DEV)
+    base = [mk(Hq, N, D), mk(Hkv, Nkv, D), mk(Hkv, Nkv, D), mk(Hq, N, D)]
+    leaves = [t.clone().requires_grad_() for t in base[:3]]
+    out = TritonAttention.apply(*leaves, causal, D ** -0.5)
+    want = [out.detach(), *torch.autograd.grad(out, leaves, base[3])]
+    mixes = [(x,) * 4 for x in LAYOUTS]
+    mixes += [tuple(LAYOUTS[(i + s * j) % len(LAYOUTS)] for j in range(4))
+              for i in range(len(LAYOUTS)) for s in (1, 3)]
+    for mix in mixes:
+        _note(f"{case} {dtype} {mix}")
+        q, k, v, do = (_laid_out(t, x) for t, x in zip(base, mix))
+        with torch.no_grad():
+            alone = scaled_dot_product_attention(q, k, v, is_causal=causal,
+                                                 enable_gqa=Hq != Hkv, backend="triton")
+        q, k, v = (t.detach().requires_grad_() for t in (q, k, v))
+        out = scaled_dot_product_attention(q, k, v, is_causal=causal, enable_gqa=Hq != Hkv,
+                                           backend="triton")
+        got = [out.detach(), *torch.autograd.grad(out, (q, k, v), do)]
+        torch.cuda.synchronize()
+        assert torch.equal(alone, want[0]), (mix, "o without autograd")
+        for name, a, b in zip(("o", "dq", "dk", "dv"), got, want):
+            assert a.is_contiguous() and torch.equal(a, b), (mix, name)
+
+
+def test_broadcast_operands_match_contiguous_copies():
+    """Heads and batches shared by stride 0, an expanded dO and N = 1 rows with an
+    arbitrary row stride."""
+    B, H, N, D = 3, 4, 200, 64
+    g = torch.Generator().manual_seed(5)
+    q = torch.randn((B, H, N, D), generator=g).half().to(DEV)
+    k1 = torch.randn((1, 1, N, D), generator=g).half().to(DEV)
+    k = k1.expand(B, H, N, D)
+    leaves = [q.clone().requires_grad_(), k1.clone().requires_grad_()]
+    for view in (True, False):
+        kk = leaves[1].expand(B, H, N, D)
+        kk = kk if view else kk.contiguous()
+        out = scaled_dot_product_attention(leaves[0], kk, kk, is_causal=True, backend="triton")
+        got = [out.detach(), *torch.autograd.grad(out.sum(), leaves)]
+        if view:
+            first = got
+    for a, b in zip(first, got):
+        assert torch.equal(a, b)
+    one = torch.randn((B, H, 9, D), generator=g).half().to(DEV)[:, :, 4:5]
+    o1 = scaled_dot_product_attention(one, k, k, backend="triton")
+    o2 = scaled_dot_product_attention(one.contiguous(), k.contiguous(), k.contiguous(),
+                                      backend="triton")
+    assert torch.equal(o1, o2)

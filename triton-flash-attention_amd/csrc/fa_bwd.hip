@@ -40,18 +40,23 @@ namespace fa {
 // --------------------------------------------------------------------------
 template <int D, class E = F16>
 __global__ __launch_bounds__(256) void preprocess_kernel(const half_t* __restrict__ o,
-                                                         const half_t* __restrict__ dO,
-                                                         float* __restrict__ delta,
-                                                         int64_t rows) {
+                                                         const half_t* __restrict__ dO, Layout dol,
+                                                         float* __restrict__ delta, int64_t rows,
+                                                         int H, int N, int cols) {
   constexpr int TPR = D / 8;  // threads per row, 8 halves each
   const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t row = gid / TPR;
   const int cc = (int)(gid - row * TPR);
   float acc = 0.f;
-  if (row < rows) {
-    const int64_t off = row * D + 8 * cc;
-    const half8 ov = *reinterpret_cast<const half8*>(o + off);
-    const half8 dv = *reinterpret_cast<const half8*>(dO + off);
+  if (row < rows && 8 * cc < cols) {
+    int64_t at = row * dol.row;  // rows of all heads one stride apart
+    if (dol.sh8 * 8ull != (uint64_t)N * dol.row || dol.sb != (int64_t)H * N * dol.row) {
+      const int head = (int)(row / N);
+      const int b = head / H;
+      at = (int64_t)dol.head(b, head - b * H) + (row - (int64_t)head * N) * dol.row;
+    }
+    const half8 ov = *reinterpret_cast<const half8*>(o + row * cols + 8 * cc);
+    const half8 dv = *reinterpret_cast<const half8*>(dO + at + 8 * cc);
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc = fmaf(elem_to_f32<E>(ov[i]), elem_to_f32<E>(dv[i]), acc);
   }
@@ -61,48 +66,51 @@ __global__ __launch_bounds__(256) void preprocess_kernel(const half_t* __restric
 }
 
 template <class E>
-hipError_t launch_preprocess_e(const half_t* o, const half_t* dO, float* delta, int64_t rows,
-                               int D, hipStream_t stream) {
+hipError_t launch_preprocess_e(const half_t* o, const half_t* dO, const Layout& dol, float* delta,
+                               int64_t rows, int64_t H, int64_t N, int D, int cols,
+                               hipStream_t stream) {
   const int64_t threads = rows * (D / 8);
   const int64_t blocks = (threads + 255) / 256;
   if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
+  const auto launch = [&](auto* kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, stream, o, dO, dol, delta, rows,
+                       (int)H, (int)N, cols);
+    return hipGetLastError();
+  };
   switch (D) {
-    case 32:
-      hipLaunchKernelGGL((preprocess_kernel<32, E>), dim3((unsigned)blocks), dim3(256), 0, stream,
-                         o, dO, delta, rows);
-      break;
-    case 64:
-      hipLaunchKernelGGL((preprocess_kernel<64, E>), dim3((unsigned)blocks), dim3(256), 0, stream,
-                         o, dO, delta, rows);
-      break;
-    case 128:
-      hipLaunchKernelGGL((preprocess_kernel<128, E>), dim3((unsigned)blocks), dim3(256), 0, stream,
-                         o, dO, delta, rows);
-      break;
-    default:
-      return hipErrorInvalidValue;
+    case 32: return launch(&preprocess_kernel<32, E>);
+    case 64: return launch(&preprocess_kernel<64, E>);
+    case 128: return launch(&preprocess_kernel<128, E>);
+    default: return hipErrorInvalidValue;
   }
-  return hipGetLastError();
 }
 
-hipError_t launch_preprocess(const half_t* o, const half_t* dO, float* delta, int64_t rows,
-                             int D, int dtype, hipStream_t stream) {
-  return dtype == kBF16 ? launch_preprocess_e<BF16>(o, dO, delta, rows, D, stream)
-                        : launch_preprocess_e<F16>(o, dO, delta, rows, D, stream);
+hipError_t launch_preprocess(const half_t* o, const half_t* dO, const Layout& dol, float* delta,
+                             int64_t B, int64_t H, int64_t N, int D, int cols, int dtype,
+                             hipStream_t stream) {
+  return dtype == kBF16
+             ? launch_preprocess_e<BF16>(o, dO, dol, delta, B * H * N, H, N, D, cols, stream)
+             : launch_preprocess_e<F16>(o, dO, dol, delta, B * H * N, H, N, D, cols, stream);
 }
 
 // --------------------------------------------------------------------------
 // dK/dV split reduction: out[i] = E(sum_s part[s][i]) in split order.
 // --------------------------------------------------------------------------
+// Value i of a plane of rows of 2^dshift floats is column i % 2^dshift of row
+// i / 2^dshift; the outputs keep the first columns that exist.
 template <class E = F16>
 __global__ __launch_bounds__(256) void split_reduce_kernel(const float* __restrict__ part,
                                                            half_t* __restrict__ dk,
                                                            half_t* __restrict__ dv,
-                                                           int64_t plane4, int nsplit) {
+                                                           int64_t plane4, int dshift, int d,
+                                                           int nsplit) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;  // float4 index in 2 planes
   if (i >= 2 * plane4) return;
   const bool is_v = i >= plane4;
   const int64_t j = is_v ? i - plane4 : i;
+  const int64_t row = (4 * j) >> dshift;
+  const int col = (int)(4 * j - (row << dshift));
+  if (col >= d) return;
   const float4v* src = reinterpret_cast<const float4v*>(part) + (is_v ? plane4 : 0) + j;
   float4v acc = src[0];
 #pragma unroll 8
@@ -110,15 +118,18 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(const float* __restri
   half4 h;
 #pragma unroll
   for (int e = 0; e < 4; ++e) h[e] = to_elem<E>(acc[e]);
-  *reinterpret_cast<half4*>((is_v ? dv : dk) + 4 * j) = h;
+  *reinterpret_cast<half4*>((is_v ? dv : dk) + row * d + col) = h;
 }
 
 template <class E>
 __global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict__ part,
                                                         half_t* __restrict__ out, int64_t elems4,
-                                                        int nsplit) {
+                                                        int dshift, int cols, int nsplit) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;  // float4 index
   if (i >= elems4) return;
+  const int64_t row = (4 * i) >> dshift;
+  const int col = (int)(4 * i - (row << dshift));
+  if (col >= cols) return;
   const float4v* src = reinterpret_cast<const float4v*>(part) + i;
   float4v acc = src[0];
 #pragma unroll 8
@@ -126,36 +137,29 @@ __global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict_
   half4 h;
 #pragma unroll
   for (int e = 0; e < 4; ++e) h[e] = to_elem<E>(acc[e]);
-  *reinterpret_cast<half4*>(out + 4 * i) = h;
+  *reinterpret_cast<half4*>(out + row * cols + col) = h;
 }
 
-hipError_t launch_split_sum(const float* part, half_t* out, int64_t elems, int nsplit, int dtype,
-                            hipStream_t stream) {
-  const int64_t elems4 = elems / 4;
+hipError_t launch_split_sum(const float* part, half_t* out, int64_t rows, int D, int cols,
+                            int nsplit, int dtype, hipStream_t stream) {
+  const int64_t elems4 = rows * D / 4;
   const int64_t blocks = (elems4 + 255) / 256;
-  if (elems % 4 != 0 || nsplit < 2 || blocks <= 0 || blocks > 0x7fffffff)
+  if (head_dim_index(D) < 0 || nsplit < 2 || blocks <= 0 || blocks > 0x7fffffff)
     return hipErrorInvalidValue;
-  if (dtype == kBF16)
-    hipLaunchKernelGGL(split_sum_kernel<BF16>, dim3((unsigned)blocks), dim3(256), 0, stream, part,
-                       out, elems4, nsplit);
-  else
-    hipLaunchKernelGGL(split_sum_kernel<F16>, dim3((unsigned)blocks), dim3(256), 0, stream, part,
-                       out, elems4, nsplit);
+  hipLaunchKernelGGL((dtype == kBF16 ? split_sum_kernel<BF16> : split_sum_kernel<F16>),
+                     dim3((unsigned)blocks), dim3(256), 0, stream, part, out, elems4, log2_of(D),
+                     cols, nsplit);
   return hipGetLastError();
 }
 
-
-hipError_t launch_split_reduce(const float* part, half_t* dk, half_t* dv, int64_t plane_elems,
-                               int nsplit, int dtype, hipStream_t stream) {
-  const int64_t plane4 = plane_elems / 4;
+hipError_t launch_split_reduce(const float* part, half_t* dk, half_t* dv, int64_t rows, int D,
+                               int d, int nsplit, int dtype, hipStream_t stream) {
+  const int64_t plane4 = rows * D / 4;
   const int64_t blocks = (2 * plane4 + 255) / 256;
-  if (plane_elems % 4 != 0 || blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidValue;
-  if (dtype == kBF16)
-    hipLaunchKernelGGL(split_reduce_kernel<BF16>, dim3((unsigned)blocks), dim3(256), 0, stream,
-                       part, dk, dv, plane4, nsplit);
-  else
-    hipLaunchKernelGGL(split_reduce_kernel<F16>, dim3((unsigned)blocks), dim3(256), 0, stream,
-                       part, dk, dv, plane4, nsplit);
+  if (head_dim_index(D) < 0 || blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((dtype == kBF16 ? split_reduce_kernel<BF16> : split_reduce_kernel<F16>),
+                     dim3((unsigned)blocks), dim3(256), 0, stream, part, dk, dv, plane4,
+                     log2_of(D), d, nsplit);
   return hipGetLastError();
 }
 
@@ -225,11 +229,10 @@ void dkdv_kernel(BwdArgs a) {
   const int G = a.group;
   const int N = a.N;      // queries
   const int Nkv = a.Nkv;  // keys
-  const uint32_t slab = (uint32_t)N * D * 2u;
-  const uint32_t kv_slab = (uint32_t)Nkv * D * 2u;
+  const uint32_t slab = a.ql.slab_bytes(N, a.d);
   const uint32_t aux_bytes = (uint32_t)N * 4u;
-  const rsrc_t rk = make_rsrc(a.k + (int64_t)kvh * Nkv * D, kv_slab);
-  const rsrc_t rv = make_rsrc(a.v + (int64_t)kvh * Nkv * D, kv_slab);
+  const rsrc_t rk = make_rsrc(a.k + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
+  const rsrc_t rv = make_rsrc(a.v + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
 
   const int k0 = kvtile * T::BKV;
   const int k0w = k0 + 32 * wave;
@@ -241,7 +244,7 @@ void dkdv_kernel(BwdArgs a) {
   half8 kf[D / 16], vf[D / 16];
 #pragma unroll
   for (int kk = 0; kk < D / 16; ++kk) {
-    const uint32_t off = (uint32_t)(krow * D + 16 * kk + 8 * g) * 2u;
+    const uint32_t off = elem_off(krow, a.kl.row, 16 * kk + 8 * g, a.d);
     kf[kk] = __builtin_bit_cast(half8, buf_load_b128(rk, off));
     vf[kk] = __builtin_bit_cast(half8, buf_load_b128(rv, off));
   }
@@ -267,15 +270,15 @@ void dkdv_kernel(BwdArgs a) {
   // Steps past the end load harmless data (rows past N read as zeros), so
   // every step issues the same number of DMA instructions.
   Dma dma;
-  dma.init(wave, lane);
+  dma.init(wave, lane, a.ql.row, a.d);
   auto issue_step = [&](int u, int slot) {
     const int st = s_lo + u;
     const int gi = min(st / ntq, G - 1);
     const int qt0 = q_begin + (st - gi * ntq) * QT;
     const int head = b * a.Hq + hkv * G + gi;
     half_t* base = lds + slot * T::STAGE;
-    dma.issue(make_rsrc_words(a.q + (int64_t)head * N * D, slab), qt0, base, wave);
-    dma.issue(make_rsrc_words(a.dO + (int64_t)head * N * D, slab), qt0, base + T::TILE, wave);
+    dma.issue(make_rsrc_words(a.q + a.ql.head(b, hkv * G + gi), slab), qt0, base, wave);
+    dma.issue(make_rsrc_words(a.dO + a.ql.head(b, hkv * G + gi), slab), qt0, base + T::TILE, wave);
     // Even waves fetch LSE[qt0 .. qt0+64), odd waves Delta (duplicates of the
     // same bytes are harmless); lane l -> float l of the 64-entry table.
     const bool is_lse = (wave & 1) == 0;
@@ -448,13 +451,13 @@ void dkdv_kernel(BwdArgs a) {
     }
     return;
   }
-  const rsrc_t rdk = make_rsrc(a.dk + (int64_t)kvh * Nkv * D, kv_slab);
-  const rsrc_t rdv = make_rsrc(a.dv + (int64_t)kvh * Nkv * D, kv_slab);
+  const rsrc_t rdk = make_rsrc(a.dk + (int64_t)kvh * Nkv * a.d, (uint32_t)(Nkv * a.d) * 2u);
+  const rsrc_t rdv = make_rsrc(a.dv + (int64_t)kvh * Nkv * a.d, (uint32_t)(Nkv * a.d) * 2u);
 #pragma unroll
   for (int db = 0; db < D / 32; ++db)
 #pragma unroll
     for (int jq = 0; jq < 4; ++jq) {
-      const uint32_t off = (uint32_t)(krow * D + 32 * db + 8 * jq + 4 * g) * 2u;
+      const uint32_t off = elem_off(krow, a.d, 32 * db + 8 * jq + 4 * g, a.d);
       buf_store_b64(rdk, off,
                     pack4<E>(dk[db][4 * jq] * scale, dk[db][4 * jq + 1] * scale,
                                dk[db][4 * jq + 2] * scale, dk[db][4 * jq + 3] * scale));
@@ -548,18 +551,16 @@ __global__ __launch_bounds__(64 * NW) void dq_kernel(BwdArgs a) {
   const int head = th.head;
   const int b = head / a.Hq;
   const int hq = head - b * a.Hq;
-  const int kvh = b * a.Hkv + hq / a.group;
+  const int hkv = hq / a.group;
   const int N = a.N;      // queries
   const int Nkv = a.Nkv;  // keys
-  const uint32_t slab = (uint32_t)N * D * 2u;
-  const uint32_t kv_slab = (uint32_t)Nkv * D * 2u;
   const uint32_t aux = (uint32_t)N * 4u;
-  const rsrc_t rq = make_rsrc(a.q + (int64_t)head * N * D, slab);
-  const rsrc_t rdo = make_rsrc(a.dO + (int64_t)head * N * D, slab);
+  const rsrc_t rq = make_rsrc(a.q + a.ql.head(b, hq), a.ql.slab_bytes(N, a.d));
+  const rsrc_t rdo = make_rsrc(a.dO + a.ql.head(b, hq), a.ql.slab_bytes(N, a.d));
   const rsrc_t rl = make_rsrc(a.lse + (int64_t)head * N, aux);
   const rsrc_t rd = make_rsrc(a.delta + (int64_t)head * N, aux);
-  const int4v rk = make_rsrc_words(a.k + (int64_t)kvh * Nkv * D, kv_slab);
-  const int4v rv = make_rsrc_words(a.v + (int64_t)kvh * Nkv * D, kv_slab);
+  const int4v rk = make_rsrc_words(a.k + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
+  const int4v rv = make_rsrc_words(a.v + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
 
   const int q0 = qtile * T::BQ;
   const int q0w = q0 + 32 * wave;
@@ -569,7 +570,7 @@ __global__ __launch_bounds__(64 * NW) void dq_kernel(BwdArgs a) {
   half8 qf[D / 16], dof[D / 16];
 #pragma unroll
   for (int kk = 0; kk < D / 16; ++kk) {
-    const uint32_t off = (uint32_t)(qrow * D + 16 * kk + 8 * g) * 2u;
+    const uint32_t off = elem_off(qrow, a.ql.row, 16 * kk + 8 * g, a.d);
     qf[kk] = __builtin_bit_cast(half8, buf_load_b128(rq, off));
     dof[kk] = __builtin_bit_cast(half8, buf_load_b128(rdo, off));
   }
@@ -590,7 +591,7 @@ __global__ __launch_bounds__(64 * NW) void dq_kernel(BwdArgs a) {
   const int ntiles = kv_hi > kv_lo ? (kv_hi - kv_lo + KT - 1) / KT : 0;
 
   Dma dma;
-  dma.init(wave, lane);
+  dma.init(wave, lane, a.kl.row, a.d);
   auto issue_tile = [&](int t, int slot) {
     const half_t* base = lds + slot * T::STAGE;
     dma.issue(rk, kv_lo + t * KT, base, wave);
@@ -702,7 +703,7 @@ __global__ __launch_bounds__(64 * NW) void dq_kernel(BwdArgs a) {
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-  const rsrc_t rdq = make_rsrc(a.dq + (int64_t)head * N * D, slab);
+  const rsrc_t rdq = make_rsrc(a.dq + (int64_t)head * N * a.d, (uint32_t)(N * a.d) * 2u);
   store_dq<D, E>(a, rdq, split, head, qrow, dq, a.scale);
 }
 

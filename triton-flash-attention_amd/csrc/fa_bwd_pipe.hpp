@@ -34,20 +34,22 @@ __device__ __forceinline__ void store_dq(const BwdArgs& a, const rsrc_t& rdq, in
   const int g = (int)(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) >> 5);
   const int64_t prow = ((int64_t)split * a.BH + head) * a.N + qrow;
   float* po = split_mode ? a.part + prow * D : nullptr;  // part is null in one-pass mode
+  with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-  for (int db = 0; db < D / 32; ++db)
+    for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-    for (int jq = 0; jq < 4; ++jq) {
-      float4v v;
+      for (int jq = 0; jq < 4; ++jq) {
+        float4v v;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = dq[db][4 * jq + e] * mul;
-      if (split_mode) {
-        if (qrow < a.N) *reinterpret_cast<float4v*>(po + 32 * db + 8 * jq + 4 * g) = v;
-      } else {
-        buf_store_b64(rdq, (uint32_t)(qrow * D + 32 * db + 8 * jq + 4 * g) * 2u,
-                      pack4<E>(v[0], v[1], v[2], v[3]));
+        for (int e = 0; e < 4; ++e) v[e] = dq[db][4 * jq + e] * mul;
+        const int col = 32 * db + 8 * jq + 4 * g;
+        if (split_mode) {
+          if (qrow < a.N) *reinterpret_cast<float4v*>(po + col) = v;
+        } else {
+          buf_store_b64(rdq, elem_off(qrow, cols, col, cols), pack4<E>(v[0], v[1], v[2], v[3]));
+        }
       }
-    }
+  });
 }
 
 template <int I, int N, typename F>
@@ -184,11 +186,10 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
   const int G = a.group;
   const int N = a.N;      // queries
   const int Nkv = a.Nkv;  // keys
-  const uint32_t slab = (uint32_t)N * D * 2u;
-  const uint32_t kv_slab = (uint32_t)Nkv * D * 2u;
+  const uint32_t slab = a.ql.slab_bytes(N, a.d);
   const uint32_t aux_bytes = (uint32_t)N * 4u;
-  const rsrc_t rk = make_rsrc(a.k + (int64_t)kvh * Nkv * D, kv_slab);
-  const rsrc_t rv = make_rsrc(a.v + (int64_t)kvh * Nkv * D, kv_slab);
+  const rsrc_t rk = make_rsrc(a.k + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
+  const rsrc_t rv = make_rsrc(a.v + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
 
   const int k0 = th.tile_rank * T::BKV;
   const int k0w = k0 + 32 * wave;
@@ -200,12 +201,14 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
   // the MFMA yields LSE' - s and P = exp2(-acc) needs no multiply-add.
   const float c = a.c;
   half8 kf[D / 16], vn[D / 16];
+  with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk) {
-    const uint32_t off = (uint32_t)(krow * D + 16 * kk + 8 * g) * 2u;
-    kf[kk] = __builtin_bit_cast(half8, buf_load_b128(rk, off));
-    vn[kk] = neg8(__builtin_bit_cast(half8, buf_load_b128(rv, off)));
-  }
+    for (int kk = 0; kk < D / 16; ++kk) {
+      const uint32_t off = elem_off(krow, a.kl.row, 16 * kk + 8 * g, cols);
+      kf[kk] = __builtin_bit_cast(half8, buf_load_b128(rk, off));
+      vn[kk] = neg8(__builtin_bit_cast(half8, buf_load_b128(rv, off)));
+    }
+  });
   wait_all_vm();
 #pragma unroll
   for (int kk = 0; kk < D / 16; ++kk)
@@ -241,59 +244,23 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
   const bool is_lse = (wave & 1) == 0;  // even waves fetch LSE, odd waves Delta
   auto set_head = [&]() {
     const int head = b * a.Hq + hkv * G + i_gi;
-    r_q = make_rsrc_words(a.q + (int64_t)head * N * D, slab);
-    r_do = make_rsrc_words(a.dO + (int64_t)head * N * D, slab);
+    r_q = make_rsrc_words(a.q + a.ql.head(b, hkv * G + i_gi), slab);
+    r_do = make_rsrc_words(a.dO + a.ql.head(b, hkv * G + i_gi), slab);
     r_aux = make_rsrc_words((is_lse ? a.lse : a.delta) + (int64_t)head * N, aux_bytes);
   };
   set_head();
 
   Dma dma;
-  dma.init(wave, lane);
+  dma.init(wave, lane, a.ql.row, a.d);
   const uint32_t lds0 = lds_addr(lds);
   const uint32_t aux_lane = (uint32_t)lane * 4u;
   const uint32_t aux_lds = 2u * T::TILE * 2u + (is_lse ? 0u : 64u * 4u);
   auto issue = [&](int slot) __attribute__((always_inline)) {
     const int row0 = i_left > 0 ? i_row : N;
-    const uint32_t vt = (uint32_t)row0 * (D * 2u) + dma.voff[0];
     const uint32_t va = (uint32_t)row0 * 4u + aux_lane;
     const uint32_t base = lds0 + (uint32_t)slot * (T::STAGE * 2u);
-    const uint32_t piece = (uint32_t)dma.piece0 * 1024u;
-    uint32_t saved;
-    if constexpr (Dma::PER_WAVE == 1) {
-      asm volatile(
-          "s_mov_b32 %0, m0\n\t"
-          "s_mov_b32 m0, %5\n\t"
-          "buffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
-          "s_mov_b32 m0, %6\n\t"
-          "buffer_load_dwordx4 %1, %4, 0 offen lds\n\t"
-          "s_mov_b32 m0, %8\n\t"
-          "buffer_load_dword %2, %7, 0 offen lds\n\t"
-          "s_mov_b32 m0, %0"
-          : "=&s"(saved)
-          : "v"(vt), "v"(va), "s"(r_q), "s"(r_do), "s"(base + piece),
-            "s"(base + T::TILE * 2u + piece), "s"(r_aux), "s"(base + aux_lds)
-          : "memory");
-    } else {
-      const uint32_t vt1 = (uint32_t)row0 * (D * 2u) + dma.voff[1];
-      asm volatile(
-          "s_mov_b32 %0, m0\n\t"
-          "s_mov_b32 m0, %6\n\t"
-          "buffer_load_dwordx4 %1, %4, 0 offen lds\n\t"
-          "s_mov_b32 m0, %7\n\t"
-          "buffer_load_dwordx4 %2, %4, 0 offen lds\n\t"
-          "s_mov_b32 m0, %8\n\t"
-          "buffer_load_dwordx4 %1, %5, 0 offen lds\n\t"
-          "s_mov_b32 m0, %9\n\t"
-          "buffer_load_dwordx4 %2, %5, 0 offen lds\n\t"
-          "s_mov_b32 m0, %11\n\t"
-          "buffer_load_dword %3, %10, 0 offen lds\n\t"
-          "s_mov_b32 m0, %0"
-          : "=&s"(saved)
-          : "v"(vt), "v"(vt1), "v"(va), "s"(r_q), "s"(r_do), "s"(base + piece),
-            "s"(base + piece + 1024u), "s"(base + T::TILE * 2u + piece),
-            "s"(base + T::TILE * 2u + piece + 1024u), "s"(r_aux), "s"(base + aux_lds)
-          : "memory");
-    }
+    issue_q_unit<T::TILE * 2>(dma, r_q, r_do, r_aux, row0, va, base + (uint32_t)dma.piece0 * 1024u,
+                              base + aux_lds);
     --i_left;
     i_row += T::QT;
     if (i_row >= N && i_left > 0) {
@@ -617,20 +584,22 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
     }
     return;
   }
-  const rsrc_t rdk = make_rsrc(a.dk + (int64_t)kvh * Nkv * D, kv_slab);
-  const rsrc_t rdv = make_rsrc(a.dv + (int64_t)kvh * Nkv * D, kv_slab);
+  const rsrc_t rdk = make_rsrc(a.dk + (int64_t)kvh * Nkv * a.d, (uint32_t)(Nkv * a.d) * 2u);
+  const rsrc_t rdv = make_rsrc(a.dv + (int64_t)kvh * Nkv * a.d, (uint32_t)(Nkv * a.d) * 2u);
+  with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-  for (int db = 0; db < D / 32; ++db)
+    for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-    for (int jq = 0; jq < 4; ++jq) {
-      const uint32_t off = (uint32_t)(krow * D + 32 * db + 8 * jq + 4 * g) * 2u;
-      buf_store_b64(rdk, off,
-                    pack4<E>(dk[db][4 * jq] * nscale, dk[db][4 * jq + 1] * nscale,
+      for (int jq = 0; jq < 4; ++jq) {
+        const uint32_t off = elem_off(krow, cols, 32 * db + 8 * jq + 4 * g, cols);
+        buf_store_b64(rdk, off,
+                      pack4<E>(dk[db][4 * jq] * nscale, dk[db][4 * jq + 1] * nscale,
                                dk[db][4 * jq + 2] * nscale, dk[db][4 * jq + 3] * nscale));
-      buf_store_b64(rdv, off,
-                    pack4<E>(dv[db][4 * jq], dv[db][4 * jq + 1], dv[db][4 * jq + 2],
+        buf_store_b64(rdv, off,
+                      pack4<E>(dv[db][4 * jq], dv[db][4 * jq + 1], dv[db][4 * jq + 2],
                                dv[db][4 * jq + 3]));
-    }
+      }
+  });
 }
 
 // --------------------------------------------------------------------------
@@ -718,18 +687,16 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
   const int head = th.head;
   const int b = head / a.Hq;
   const int hq = head - b * a.Hq;
-  const int kvh = b * a.Hkv + hq / a.group;
+  const int hkv = hq / a.group;
   const int N = a.N;      // queries
   const int Nkv = a.Nkv;  // keys
-  const uint32_t slab = (uint32_t)N * D * 2u;
-  const uint32_t kv_slab = (uint32_t)Nkv * D * 2u;
   const uint32_t aux = (uint32_t)N * 4u;
-  const rsrc_t rq = make_rsrc(a.q + (int64_t)head * N * D, slab);
-  const rsrc_t rdo = make_rsrc(a.dO + (int64_t)head * N * D, slab);
+  const rsrc_t rq = make_rsrc(a.q + a.ql.head(b, hq), a.ql.slab_bytes(N, a.d));
+  const rsrc_t rdo = make_rsrc(a.dO + a.ql.head(b, hq), a.ql.slab_bytes(N, a.d));
   const rsrc_t rl = make_rsrc(a.lse + (int64_t)head * N, aux);
   const rsrc_t rd = make_rsrc(a.delta + (int64_t)head * N, aux);
-  const int4v r_k = make_rsrc_words(a.k + (int64_t)kvh * Nkv * D, kv_slab);
-  const int4v r_v = make_rsrc_words(a.v + (int64_t)kvh * Nkv * D, kv_slab);
+  const int4v r_k = make_rsrc_words(a.k + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
+  const int4v r_v = make_rsrc_words(a.v + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
 
   const int q0 = qtile * T::BQ;
   const int q0w = q0 + 32 * wave;
@@ -738,26 +705,31 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
   // -fp16(c Q) and -dO as B operands (column = query ql, d = 16*kk + 8*g .. +7).
   const float c = a.c;
   half8 qf[D / 16], don[D / 16];
+  with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk) {
-    const uint32_t off = (uint32_t)(qrow * D + 16 * kk + 8 * g) * 2u;
-    qf[kk] = __builtin_bit_cast(half8, buf_load_b128(rq, off));
-    don[kk] = neg8(__builtin_bit_cast(half8, buf_load_b128(rdo, off)));
-  }
+    for (int kk = 0; kk < D / 16; ++kk) {
+      const uint32_t off = elem_off(qrow, a.ql.row, 16 * kk + 8 * g, cols);
+      qf[kk] = __builtin_bit_cast(half8, buf_load_b128(rq, off));
+      don[kk] = neg8(__builtin_bit_cast(half8, buf_load_b128(rdo, off)));
+    }
+  });
   const float lse = buf_load_f32(rl, (uint32_t)qrow * 4u);
   float delta;
   if (a.o != nullptr) {
     // Delta = rowsum(O * dO) of this lane's query (the halves g = 0, 1 hold
     // the two 8-wide halves of every 16-wide chunk of the row).
-    const rsrc_t ro = make_rsrc(a.o + (int64_t)head * N * D, slab);
+    const rsrc_t ro = make_rsrc(a.o + (int64_t)head * N * a.d, (uint32_t)(N * a.d) * 2u);
     float part = 0.f;
+    with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) {
-      const half8 ov = __builtin_bit_cast(
-          half8, buf_load_b128(ro, (uint32_t)(qrow * D + 16 * kk + 8 * g) * 2u));
+      for (int kk = 0; kk < D / 16; ++kk) {
+        const half8 ov = __builtin_bit_cast(
+            half8, buf_load_b128(ro, elem_off(qrow, cols, 16 * kk + 8 * g, cols)));
 #pragma unroll
-      for (int e = 0; e < 8; ++e) part = fmaf(elem_to_f32<E>(ov[e]), -elem_to_f32<E>(don[kk][e]), part);
-    }
+        for (int e = 0; e < 8; ++e)
+          part = fmaf(elem_to_f32<E>(ov[e]), -elem_to_f32<E>(don[kk][e]), part);
+      }
+    });
     delta = halves_sum(part);
     if (g == 0 && qrow < N && split == 0) a.delta_out[(int64_t)head * N + qrow] = delta;
   } else {
@@ -784,13 +756,14 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
   const int s0 = 2 * p0;
 
   Dma dma;
-  dma.init(wave, lane);
+  dma.init(wave, lane, a.kl.row, a.d);
   const uint32_t lds0 = lds_addr(lds);
   int i_row = kv_lo;  // first key row of the next unit to fetch
   auto issue = [&](int slot) __attribute__((always_inline)) {
     const int row0 = i_row < kv_hi ? i_row : Nkv;  // past the range: zeros
-    issue_kv_unit<T::TILE * 2>(dma, r_k, r_v, (uint32_t)row0 * (D * 2u),
-                               lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
+    issue_kv_unit<T::TILE * 2>(
+        dma, r_k, r_v, row0,
+        lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
     i_row += T::KT;
   };
 #pragma unroll
@@ -1047,7 +1020,7 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
   if constexpr (kAgprAcc) agpr_acc_drain();
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-  const rsrc_t rdq = make_rsrc(a.dq + (int64_t)head * N * D, slab);
+  const rsrc_t rdq = make_rsrc(a.dq + (int64_t)head * N * a.d, (uint32_t)(N * a.d) * 2u);
   store_dq<D, E>(a, rdq, split, head, qrow, dq, -a.scale);  // accumulated -dS
 }
 

@@ -60,18 +60,16 @@ __device__ __forceinline__ void dq_pipe16_body(const BwdArgs& a, const unsigned 
   const int head = th.head;
   const int b = head / a.Hq;
   const int hq = head - b * a.Hq;
-  const int kvh = b * a.Hkv + hq / a.group;
+  const int hkv = hq / a.group;
   const int N = a.N;      // queries
   const int Nkv = a.Nkv;  // keys
-  const uint32_t slab = (uint32_t)N * D * 2u;
-  const uint32_t kv_slab = (uint32_t)Nkv * D * 2u;
   const uint32_t aux = (uint32_t)N * 4u;
-  const rsrc_t rq = make_rsrc(a.q + (int64_t)head * N * D, slab);
-  const rsrc_t rdo = make_rsrc(a.dO + (int64_t)head * N * D, slab);
+  const rsrc_t rq = make_rsrc(a.q + a.ql.head(b, hq), a.ql.slab_bytes(N, a.d));
+  const rsrc_t rdo = make_rsrc(a.dO + a.ql.head(b, hq), a.ql.slab_bytes(N, a.d));
   const rsrc_t rl = make_rsrc(a.lse + (int64_t)head * N, aux);
   const rsrc_t rd = make_rsrc(a.delta + (int64_t)head * N, aux);
-  const int4v r_k = make_rsrc_words(a.k + (int64_t)kvh * Nkv * D, kv_slab);
-  const int4v r_v = make_rsrc_words(a.v + (int64_t)kvh * Nkv * D, kv_slab);
+  const int4v r_k = make_rsrc_words(a.k + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
+  const int4v r_v = make_rsrc_words(a.v + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
 
   const int q0 = qtile * T::BQ;
   const int q0w = q0 + 32 * wave;
@@ -81,32 +79,36 @@ __device__ __forceinline__ void dq_pipe16_body(const BwdArgs& a, const unsigned 
   // d = 32 kd + 8 sg .. +7. Rows past N read as zeros (buffer range check).
   const float c = a.c;
   half8 qf[2][KD], don[2][KD];
+  with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb)
+    for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
-    for (int kd = 0; kd < KD; ++kd) {
-      const uint32_t off = (uint32_t)((qrow0 + 16 * qb) * D + 32 * kd + 8 * sg) * 2u;
-      qf[qb][kd] = __builtin_bit_cast(half8, buf_load_b128(rq, off));
-      don[qb][kd] = neg8(__builtin_bit_cast(half8, buf_load_b128(rdo, off)));
-    }
+      for (int kd = 0; kd < KD; ++kd) {
+        const uint32_t off = elem_off(qrow0 + 16 * qb, a.ql.row, 32 * kd + 8 * sg, cols);
+        qf[qb][kd] = __builtin_bit_cast(half8, buf_load_b128(rq, off));
+        don[qb][kd] = neg8(__builtin_bit_cast(half8, buf_load_b128(rdo, off)));
+      }
+  });
   float lse[2], delta[2];
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb) lse[qb] = buf_load_f32(rl, (uint32_t)(qrow0 + 16 * qb) * 4u);
   if (a.o != nullptr) {
     // Delta = rowsum(O * dO) of each of the lane's two queries; the lanes
     // l, l^16, l^32, l^48 hold the four quarters of every 32-wide chunk.
-    const rsrc_t ro = make_rsrc(a.o + (int64_t)head * N * D, slab);
+    const rsrc_t ro = make_rsrc(a.o + (int64_t)head * N * a.d, (uint32_t)(N * a.d) * 2u);
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
       float part = 0.f;
+      with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-      for (int kd = 0; kd < KD; ++kd) {
-        const half8 ov = __builtin_bit_cast(
-            half8, buf_load_b128(ro, (uint32_t)((qrow0 + 16 * qb) * D + 32 * kd + 8 * sg) * 2u));
+        for (int kd = 0; kd < KD; ++kd) {
+          const half8 ov = __builtin_bit_cast(
+              half8, buf_load_b128(ro, elem_off(qrow0 + 16 * qb, cols, 32 * kd + 8 * sg, cols)));
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          part = fmaf(elem_to_f32<E>(ov[e]), -elem_to_f32<E>(don[qb][kd][e]), part);
-      }
+          for (int e = 0; e < 8; ++e)
+            part = fmaf(elem_to_f32<E>(ov[e]), -elem_to_f32<E>(don[qb][kd][e]), part);
+        }
+      });
       delta[qb] = quarters_sum(part);
       const int qr = qrow0 + 16 * qb;
       if (G == 0 && qr < N && split == 0) a.delta_out[(int64_t)head * N + qr] = delta[qb];
@@ -138,13 +140,14 @@ __device__ __forceinline__ void dq_pipe16_body(const BwdArgs& a, const unsigned 
   const int s0 = 2 * p0;
 
   Dma dma;
-  dma.init(wave, lane);
+  dma.init(wave, lane, a.kl.row, a.d);
   const uint32_t lds0 = lds_addr(lds);
   int i_row = kv_lo;  // first key row of the next unit to fetch
   auto issue = [&](int slot) __attribute__((always_inline)) {
     const int row0 = i_row < kv_hi ? i_row : Nkv;  // past the range: zeros
-    issue_kv_unit<T::TILE * 2>(dma, r_k, r_v, (uint32_t)row0 * (D * 2u),
-                               lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
+    issue_kv_unit<T::TILE * 2>(
+        dma, r_k, r_v, row0,
+        lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
     i_row += T::KT;
   };
 #pragma unroll
@@ -184,30 +187,27 @@ __device__ __forceinline__ void dq_pipe16_body(const BwdArgs& a, const unsigned 
 
   // Row reads of K and V (A operands of S^T and dP^T): key row 16 kb + c16,
   // 16-byte chunk 4 kd + sg.
-  int r_off[2][KD];
+  // (Both tables: rows 16 apart have the same chunk order, so a key block or half
+  // only adds a constant.)
+  int r_off[KD];
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-    for (int kd = 0; kd < KD; ++kd)
-      r_off[kb][kd] = swz_offset<D>(16 * kb + rows16<D>(c16), 4 * kd + sg);
+  for (int kd = 0; kd < KD; ++kd) r_off[kd] = swz_offset<D>(rows16<D>(c16), 4 * kd + sg);
   // Transposing reads of K (A operand of dQ^T += K^T dS'^T): in 16-lane group
   // G, source lane i addresses key row 16 h + 4 gq + i / 4, columns
   // 16 dd + 4 (i % 4) .. +3, and lane i receives keys 16 h + 4 gq + 0..3 of
   // column (d) 16 dd + i (ds_read_b64_tr_b16).
-  int t_off[DD][2];
+  int t_off[DD];
 #pragma unroll
-  for (int dd = 0; dd < DD; ++dd)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int row = 16 * h + 4 * gq + (c16 >> 2);
-      const int col = 16 * dd + 4 * (c16 & 3);
-      t_off[dd][h] = row * D + 8 * swz_chunk<D>(row, col >> 3) + (col & 7);
-    }
+  for (int dd = 0; dd < DD; ++dd) {
+    const int row = 4 * gq + (c16 >> 2);
+    const int col = 16 * dd + 4 * (c16 & 3);
+    t_off[dd] = row * D + 8 * swz_chunk<D>(row, col >> 3) + (col & 7);
+  }
   auto trk = [&](const half_t* base, int dd) {
     const half4 lo = __builtin_bit_cast(
-        half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(base + t_off[dd][0])));
+        half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(base + t_off[dd])));
     const half4 hi = __builtin_bit_cast(
-        half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(base + t_off[dd][1])));
+        half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(base + t_off[dd] + 16 * D)));
     half8 v;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -250,8 +250,8 @@ __device__ __forceinline__ void dq_pipe16_body(const BwdArgs& a, const unsigned 
 #pragma unroll
     for (int kd = 0; kd < KD; ++kd) {
       const half_t* first = lds + s0 * T::STAGE;
-      const half8 ok = *reinterpret_cast<const half8*>(first + r_off[kb][kd]);
-      const half8 ov = *reinterpret_cast<const half8*>(first + T::TILE + r_off[kb][kd]);
+      const half8 ok = *reinterpret_cast<const half8*>(first + 16 * kb * D + r_off[kd]);
+      const half8 ov = *reinterpret_cast<const half8*>(first + T::TILE + 16 * kb * D + r_off[kd]);
 #pragma unroll
       for (int qb = 0; qb < 2; ++qb) {
         s_cur[kb][qb] = mma16<E>(ok, qf[qb][kd], s_cur[kb][qb]);
@@ -338,8 +338,8 @@ __device__ __forceinline__ void dq_pipe16_body(const BwdArgs& a, const unsigned 
       constexpr int kind = t % 3, q = t / 3;
       constexpr int kb = q / KD, kd = q % KD;
       if constexpr (kind == 0) return trk(p, q);
-      else if constexpr (kind == 1) return *reinterpret_cast<const half8*>(n + r_off[kb][kd]);
-      else return *reinterpret_cast<const half8*>(n + T::TILE + r_off[kb][kd]);
+      else if constexpr (kind == 1) return *reinterpret_cast<const half8*>(n + 16 * kb * D + r_off[kd]);
+      else return *reinterpret_cast<const half8*>(n + T::TILE + 16 * kb * D + r_off[kd]);
     };
     auto load_op = [&](auto t_c) -> half8 { return load_op_at(t_c, prv, nxt); };
     float4v s_nx[2][2], dp_nx[2][2];
@@ -444,25 +444,27 @@ __device__ __forceinline__ void dq_pipe16_body(const BwdArgs& a, const unsigned 
   // Epilogue: lane holds d = 16 dd + 4 G + j of query 16 qb + c16 (scaled by
   // -scale: the accumulator holds -dS K).
   const float mul = -a.scale;
-  const rsrc_t rdq = make_rsrc(a.dq + (int64_t)head * N * D, slab);
+  const rsrc_t rdq = make_rsrc(a.dq + (int64_t)head * N * a.d, (uint32_t)(N * a.d) * 2u);
   const bool split_mode = a.nsplit > 1;
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb) {
     const int qr = qrow0 + 16 * qb;
     const int64_t prow = ((int64_t)split * a.BH + head) * a.N + qr;
     float* po = split_mode ? a.part + prow * D : nullptr;  // part is null in one-pass mode
+    with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-    for (int dd = 0; dd < DD; ++dd) {
-      float4v v;
+      for (int dd = 0; dd < DD; ++dd) {
+        float4v v;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = dq[dd][qb][e] * mul;
-      if (split_mode) {
-        if (qr < a.N) *reinterpret_cast<float4v*>(po + 16 * dd + 4 * G) = v;
-      } else {
-        buf_store_b64(rdq, (uint32_t)(qr * D + 16 * dd + 4 * G) * 2u,
-                      pack4<E>(v[0], v[1], v[2], v[3]));
+        for (int e = 0; e < 4; ++e) v[e] = dq[dd][qb][e] * mul;
+        const int col = 16 * dd + 4 * G;
+        if (split_mode) {
+          if (qr < a.N) *reinterpret_cast<float4v*>(po + col) = v;
+        } else {
+          buf_store_b64(rdq, elem_off(qr, cols, col, cols), pack4<E>(v[0], v[1], v[2], v[3]));
+        }
       }
-    }
+    });
   }
 }
 
@@ -513,11 +515,10 @@ __device__ __forceinline__ void dkdv_pipe16_body(const BwdArgs& a, const unsigne
   const int QG = a.group;
   const int N = a.N;      // queries
   const int Nkv = a.Nkv;  // keys
-  const uint32_t slab = (uint32_t)N * D * 2u;
-  const uint32_t kv_slab = (uint32_t)Nkv * D * 2u;
+  const uint32_t slab = a.ql.slab_bytes(N, a.d);
   const uint32_t aux_bytes = (uint32_t)N * 4u;
-  const rsrc_t rk = make_rsrc(a.k + (int64_t)kvh * Nkv * D, kv_slab);
-  const rsrc_t rv = make_rsrc(a.v + (int64_t)kvh * Nkv * D, kv_slab);
+  const rsrc_t rk = make_rsrc(a.k + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
+  const rsrc_t rv = make_rsrc(a.v + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
 
   const int k0 = th.tile_rank * T::BKV;
   const int k0w = k0 + 32 * wave;
@@ -528,14 +529,16 @@ __device__ __forceinline__ void dkdv_pipe16_body(const BwdArgs& a, const unsigne
   // (attention.py:435). Rows past N_kv read as zeros.
   const float c = a.c;
   half8 kf[2][KD], vn[2][KD];
+  with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-    for (int kd = 0; kd < KD; ++kd) {
-      const uint32_t off = (uint32_t)((krow0 + 16 * kb) * D + 32 * kd + 8 * sg) * 2u;
-      kf[kb][kd] = __builtin_bit_cast(half8, buf_load_b128(rk, off));
-      vn[kb][kd] = neg8(__builtin_bit_cast(half8, buf_load_b128(rv, off)));
-    }
+      for (int kd = 0; kd < KD; ++kd) {
+        const uint32_t off = elem_off(krow0 + 16 * kb, a.kl.row, 32 * kd + 8 * sg, cols);
+        kf[kb][kd] = __builtin_bit_cast(half8, buf_load_b128(rk, off));
+        vn[kb][kd] = neg8(__builtin_bit_cast(half8, buf_load_b128(rv, off)));
+      }
+  });
   wait_all_vm();
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb)
@@ -566,59 +569,23 @@ __device__ __forceinline__ void dkdv_pipe16_body(const BwdArgs& a, const unsigne
   const bool is_lse = (wave & 1) == 0;  // even waves fetch LSE, odd waves Delta
   auto set_head = [&]() {
     const int head = b * a.Hq + hkv * QG + i_gi;
-    r_q = make_rsrc_words(a.q + (int64_t)head * N * D, slab);
-    r_do = make_rsrc_words(a.dO + (int64_t)head * N * D, slab);
+    r_q = make_rsrc_words(a.q + a.ql.head(b, hkv * QG + i_gi), slab);
+    r_do = make_rsrc_words(a.dO + a.ql.head(b, hkv * QG + i_gi), slab);
     r_aux = make_rsrc_words((is_lse ? a.lse : a.delta) + (int64_t)head * N, aux_bytes);
   };
   set_head();
 
   Dma dma;
-  dma.init(wave, lane);
+  dma.init(wave, lane, a.ql.row, a.d);
   const uint32_t lds0 = lds_addr(lds);
   const uint32_t aux_lane = (uint32_t)lane * 4u;
   const uint32_t aux_lds = 2u * T::TILE * 2u + (is_lse ? 0u : 64u * 4u);
   auto issue = [&](int slot) __attribute__((always_inline)) {
     const int row0 = i_left > 0 ? i_row : N;
-    const uint32_t vt = (uint32_t)row0 * (D * 2u) + dma.voff[0];
     const uint32_t va = (uint32_t)row0 * 4u + aux_lane;
     const uint32_t base = lds0 + (uint32_t)slot * (T::STAGE * 2u);
-    const uint32_t piece = (uint32_t)dma.piece0 * 1024u;
-    uint32_t saved;
-    if constexpr (Dma::PER_WAVE == 1) {
-      asm volatile(
-          "s_mov_b32 %0, m0\n\t"
-          "s_mov_b32 m0, %5\n\t"
-          "buffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
-          "s_mov_b32 m0, %6\n\t"
-          "buffer_load_dwordx4 %1, %4, 0 offen lds\n\t"
-          "s_mov_b32 m0, %8\n\t"
-          "buffer_load_dword %2, %7, 0 offen lds\n\t"
-          "s_mov_b32 m0, %0"
-          : "=&s"(saved)
-          : "v"(vt), "v"(va), "s"(r_q), "s"(r_do), "s"(base + piece),
-            "s"(base + T::TILE * 2u + piece), "s"(r_aux), "s"(base + aux_lds)
-          : "memory");
-    } else {
-      const uint32_t vt1 = (uint32_t)row0 * (D * 2u) + dma.voff[1];
-      asm volatile(
-          "s_mov_b32 %0, m0\n\t"
-          "s_mov_b32 m0, %6\n\t"
-          "buffer_load_dwordx4 %1, %4, 0 offen lds\n\t"
-          "s_mov_b32 m0, %7\n\t"
-          "buffer_load_dwordx4 %2, %4, 0 offen lds\n\t"
-          "s_mov_b32 m0, %8\n\t"
-          "buffer_load_dwordx4 %1, %5, 0 offen lds\n\t"
-          "s_mov_b32 m0, %9\n\t"
-          "buffer_load_dwordx4 %2, %5, 0 offen lds\n\t"
-          "s_mov_b32 m0, %11\n\t"
-          "buffer_load_dword %3, %10, 0 offen lds\n\t"
-          "s_mov_b32 m0, %0"
-          : "=&s"(saved)
-          : "v"(vt), "v"(vt1), "v"(va), "s"(r_q), "s"(r_do), "s"(base + piece),
-            "s"(base + piece + 1024u), "s"(base + T::TILE * 2u + piece),
-            "s"(base + T::TILE * 2u + piece + 1024u), "s"(r_aux), "s"(base + aux_lds)
-          : "memory");
-    }
+    issue_q_unit<T::TILE * 2>(dma, r_q, r_do, r_aux, row0, va, base + (uint32_t)dma.piece0 * 1024u,
+                              base + aux_lds);
     --i_left;
     i_row += T::QT;
     if (i_row >= N && i_left > 0) {
@@ -643,30 +610,27 @@ __device__ __forceinline__ void dkdv_pipe16_body(const BwdArgs& a, const unsigne
 
   // Row reads of Q and dO (A operands of S and dP): query row 16 qb + c16,
   // 16-byte chunk 4 kd + sg.
-  int r_off[2][KD];
+  // (Both tables: rows 16 apart have the same chunk order, so a query block or half
+  // only adds a constant.)
+  int r_off[KD];
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-    for (int kd = 0; kd < KD; ++kd)
-      r_off[qb][kd] = swz_offset<D>(16 * qb + rows16<D>(c16), 4 * kd + sg);
+  for (int kd = 0; kd < KD; ++kd) r_off[kd] = swz_offset<D>(rows16<D>(c16), 4 * kd + sg);
   // Transposing reads of dO and Q (A operands of dV^T and dK^T): in 16-lane
   // group G, source lane i addresses query row 16 h + 4 gq + i / 4, columns
   // 16 dd + 4 (i % 4) .. +3; lane i receives queries 16 h + 4 gq + 0..3 of
   // column (d) 16 dd + i.
-  int t_off[DD][2];
+  int t_off[DD];
 #pragma unroll
-  for (int dd = 0; dd < DD; ++dd)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int row = 16 * h + 4 * gq + (c16 >> 2);
-      const int col = 16 * dd + 4 * (c16 & 3);
-      t_off[dd][h] = row * D + 8 * swz_chunk<D>(row, col >> 3) + (col & 7);
-    }
+  for (int dd = 0; dd < DD; ++dd) {
+    const int row = 4 * gq + (c16 >> 2);
+    const int col = 16 * dd + 4 * (c16 & 3);
+    t_off[dd] = row * D + 8 * swz_chunk<D>(row, col >> 3) + (col & 7);
+  }
   auto trq = [&](const half_t* base, int dd) {
     const half4 lo = __builtin_bit_cast(
-        half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(base + t_off[dd][0])));
+        half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(base + t_off[dd])));
     const half4 hi = __builtin_bit_cast(
-        half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(base + t_off[dd][1])));
+        half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(base + t_off[dd] + 16 * D)));
     half8 v;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -720,8 +684,8 @@ __device__ __forceinline__ void dkdv_pipe16_body(const BwdArgs& a, const unsigne
     for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
       for (int kd = 0; kd < KD; ++kd) {
-        const half8 oq = *reinterpret_cast<const half8*>(first + r_off[qb][kd]);
-        const half8 od = *reinterpret_cast<const half8*>(first + T::TILE + r_off[qb][kd]);
+        const half8 oq = *reinterpret_cast<const half8*>(first + 16 * qb * D + r_off[kd]);
+        const half8 od = *reinterpret_cast<const half8*>(first + T::TILE + 16 * qb * D + r_off[kd]);
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
           s_cur[qb][kb] = mma16<E>(oq, kf[kb][kd], s_cur[qb][kb]);
@@ -792,8 +756,8 @@ __device__ __forceinline__ void dkdv_pipe16_body(const BwdArgs& a, const unsigne
       constexpr int qb = q / KD, kd = q % KD;
       if constexpr (kind == 0) return trq(p + T::TILE, q);
       else if constexpr (kind == 1) return trq(p, q);
-      else if constexpr (kind == 2) return *reinterpret_cast<const half8*>(n + r_off[qb][kd]);
-      else return *reinterpret_cast<const half8*>(n + T::TILE + r_off[qb][kd]);
+      else if constexpr (kind == 2) return *reinterpret_cast<const half8*>(n + 16 * qb * D + r_off[kd]);
+      else return *reinterpret_cast<const half8*>(n + T::TILE + 16 * qb * D + r_off[kd]);
     };
     auto load_op = [&](auto t_c) -> half8 { return load_op_at(t_c, prv, nxt); };
     const half_t* nxt2 = lds + ((SLOT + 2) % NS) * T::STAGE;
@@ -948,18 +912,21 @@ __device__ __forceinline__ void dkdv_pipe16_body(const BwdArgs& a, const unsigne
     }
     return;
   }
-  const rsrc_t rdk = make_rsrc(a.dk + (int64_t)kvh * Nkv * D, kv_slab);
-  const rsrc_t rdv = make_rsrc(a.dv + (int64_t)kvh * Nkv * D, kv_slab);
+  const rsrc_t rdk = make_rsrc(a.dk + (int64_t)kvh * Nkv * a.d, (uint32_t)(Nkv * a.d) * 2u);
+  const rsrc_t rdv = make_rsrc(a.dv + (int64_t)kvh * Nkv * a.d, (uint32_t)(Nkv * a.d) * 2u);
+  with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-    for (int dd = 0; dd < DD; ++dd) {
-      const uint32_t off = (uint32_t)((krow0 + 16 * kb) * D + 16 * dd + 4 * G) * 2u;
-      buf_store_b64(rdk, off,
-                    pack4<E>(dk[dd][kb][0] * nscale, dk[dd][kb][1] * nscale,
-                             dk[dd][kb][2] * nscale, dk[dd][kb][3] * nscale));
-      buf_store_b64(rdv, off, pack4<E>(dv[dd][kb][0], dv[dd][kb][1], dv[dd][kb][2], dv[dd][kb][3]));
-    }
+      for (int dd = 0; dd < DD; ++dd) {
+        const uint32_t off = elem_off(krow0 + 16 * kb, cols, 16 * dd + 4 * G, cols);
+        buf_store_b64(rdk, off,
+                      pack4<E>(dk[dd][kb][0] * nscale, dk[dd][kb][1] * nscale,
+                               dk[dd][kb][2] * nscale, dk[dd][kb][3] * nscale));
+        buf_store_b64(rdv, off,
+                      pack4<E>(dv[dd][kb][0], dv[dd][kb][1], dv[dd][kb][2], dv[dd][kb][3]));
+      }
+  });
 }
 
 }  // namespace fa

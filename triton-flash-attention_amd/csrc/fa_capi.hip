@@ -412,19 +412,83 @@ int check_scale(float scale) {
   return FA_OK;
 }
 
-fa::BwdArgs bwd_args(const fa_half_t* q, const fa_half_t* k, const fa_half_t* v,
-                     const fa_half_t* dO, const float* lse, const float* delta, int64_t B,
+const fa::half_t* elems(const fa_half_t* p) { return reinterpret_cast<const fa::half_t*>(p); }
+fa::half_t* elems(fa_half_t* p) { return reinterpret_cast<fa::half_t*>(p); }
+
+// The layout of a contiguous [B, H, N, D] tensor.
+fa::Layout packed(int64_t H, int64_t N, int64_t D) {
+  return {H * N * D, (uint32_t)(N * D / 8), (int)D};
+}
+
+// The input tensors of a call, their layouts (q and dO, k and v) and head size, at
+// most the kernel width the call runs at.
+struct Inputs {
+  const fa_half_t *q, *k, *v, *dO;
+  fa::Layout ql, kl;
+  int d;
+};
+
+// Contiguous inputs of the kernel width D (dO null in the forward).
+Inputs contiguous_inputs(const fa_half_t* q, const fa_half_t* k, const fa_half_t* v,
+                         const fa_half_t* dO, int64_t Hq, int64_t Hkv, int64_t N, int64_t Nkv,
+                         int64_t D) {
+  return {q, k, v, dO, packed(Hq, N, D), packed(Hkv, Nkv, D), (int)D};
+}
+
+// A layout from the batch, head and row stride (elements) a strided entry point was
+// given for `what`, tensors of `rows` rows of D columns.
+int view_layout(const char* name, const char* what, const int64_t* strides, int64_t rows,
+                int64_t D, fa::Layout* out) {
+  const int64_t sb = strides[0], sh = strides[1], row = strides[2];
+  if (sb % 8 || sh % 8 || row % 8 || sb < 0 || sh < 0 || sh / 8 > UINT32_MAX)
+    return fail(FA_ERR_BAD_STRIDE, "%s: the strides of %s (%lld, %lld, %lld) must be multiples of "
+                "8 elements and not negative, the head stride below 2^35", name, what,
+                (long long)sb, (long long)sh, (long long)row);
+  if (row < D)
+    return fail(FA_ERR_BAD_STRIDE, "%s: the row stride %lld of %s is smaller than their %lld "
+                "columns", name, (long long)row, what, (long long)D);
+  // rows are addressed with 32-bit byte offsets from their head
+  if (row >= ((int64_t)1 << 30) || (rows + 4096) * row * 2 >= ((int64_t)1 << 31))
+    return fail(FA_ERR_TOO_LARGE, "%s: %lld rows of %s at stride %lld exceed the 32-bit "
+                "addressing", name, (long long)rows, what, (long long)row);
+  *out = {sb, (uint32_t)(sh / 8), (int)row};
+  return FA_OK;
+}
+
+// The inputs of a strided entry point: `strides` holds the batch, head and row stride
+// of q (and dO), then of k and v.
+int view_inputs(const char* name, const fa_half_t* q, const fa_half_t* k, const fa_half_t* v,
+                const fa_half_t* dO, const int64_t* strides, int64_t N, int64_t Nkv, int64_t D,
+                Inputs* out) {
+  if (!strides) return fail(FA_ERR_NULL_POINTER, "%s: null pointer", name);
+  *out = {q, k, v, dO, {}, {}, (int)D};
+  const int rc = view_layout(name, "q and dO", strides, N, D, &out->ql);
+  return rc ? rc : view_layout(name, "k and v", strides + 3, Nkv, D, &out->kl);
+}
+
+// The kernel width that holds head size D (a multiple of 8), or a negative code.
+int64_t view_width(const char* name, int64_t D) {
+  if (D < 8 || D % 8 || D > 128)
+    return fail(FA_ERR_HEAD_DIM, "%s: the head size must be a multiple of 8 up to 128; got %lld",
+                name, (long long)D);
+  return D <= 32 ? 32 : D <= 64 ? 64 : 128;
+}
+
+fa::BwdArgs bwd_args(const Inputs& in, const float* lse, const float* delta, int64_t B,
                      int64_t Hq, int64_t Hkv, int64_t N, int64_t Nkv, float scale) {
   fa::BwdArgs a;
-  a.q = reinterpret_cast<const fa::half_t*>(q);
-  a.k = reinterpret_cast<const fa::half_t*>(k);
-  a.v = reinterpret_cast<const fa::half_t*>(v);
-  a.dO = reinterpret_cast<const fa::half_t*>(dO);
+  a.q = elems(in.q);
+  a.k = elems(in.k);
+  a.v = elems(in.v);
+  a.dO = elems(in.dO);
+  a.ql = in.ql;
+  a.kl = in.kl;
   a.lse = lse;
   a.delta = delta;
   a.dq = nullptr;
   a.dk = nullptr;
   a.dv = nullptr;
+  a.d = in.d;
   a.N = (int)N;
   a.Nkv = (int)Nkv;
   a.Hq = (int)Hq;
@@ -821,15 +885,15 @@ const char* fa_last_error(void) { return g_last_error; }
 
 // Argument checks of the forward entry points (no HIP call); on success *var
 // is the selected tiling and *need the split workspace bytes (0: one pass).
-static int fwd_check(int dt, const char* name, const fa_half_t* q, const fa_half_t* k,
-                     const fa_half_t* v, fa_half_t* o, float* lse, int64_t B, int64_t Hq,
-                     int64_t Hkv, int64_t N, int64_t Nkv, int64_t D, float scale, int causal,
-                     const fa::Variant** var, int64_t* need) {
-  if (!q || !k || !v || !o || !lse) return fail(FA_ERR_NULL_POINTER, "%s: null pointer", name);
+static int fwd_check(int dt, const char* name, const Inputs& in, fa_half_t* o, float* lse,
+                     int64_t B, int64_t Hq, int64_t Hkv, int64_t N, int64_t Nkv, int64_t D,
+                     float scale, int causal, const fa::Variant** var, int64_t* need) {
+  if (!in.q || !in.k || !in.v || !o || !lse)
+    return fail(FA_ERR_NULL_POINTER, "%s: null pointer", name);
   int rc = check_common(B, Hq, Hkv, N, D);
   if (rc) return rc;
   if ((rc = check_kv_length(Nkv, D))) return rc;
-  if ((rc = check_aligned(name, {q, k, v, o, lse}))) return rc;
+  if ((rc = check_aligned(name, {in.q, in.k, in.v, o, lse}))) return rc;
   if ((rc = check_scale(scale))) return rc;
   *var = select_fwd(fa::head_dim_index(D), causal, N, Nkv, B * Hq, Hq / Hkv, dt);
   if (!*var) return fail(FA_ERR_BAD_TILING, "%s: no kernel for the selected tiling", name);
@@ -838,20 +902,23 @@ static int fwd_check(int dt, const char* name, const fa_half_t* q, const fa_half
   return FA_OK;
 }
 
-static int fwd_impl(int dt, const char* name, const fa_half_t* q, const fa_half_t* k,
-                    const fa_half_t* v, fa_half_t* o, float* lse, int64_t B, int64_t Hq,
-                    int64_t Hkv, int64_t N, int64_t Nkv, int64_t D, float scale, int causal,
-                    void* stream, void* workspace = nullptr, int64_t workspace_bytes = 0) {
+static int fwd_launch_impl(int dt, const char* name, const Inputs& in, fa_half_t* o, float* lse,
+                           int64_t B, int64_t Hq, int64_t Hkv, int64_t N, int64_t Nkv, int64_t D,
+                           float scale, int causal, void* stream, void* workspace,
+                           int64_t workspace_bytes) {
   const fa::Variant* var = nullptr;
   int64_t need = 0;
-  int rc = fwd_check(dt, name, q, k, v, o, lse, B, Hq, Hkv, N, Nkv, D, scale, causal, &var, &need);
+  int rc = fwd_check(dt, name, in, o, lse, B, Hq, Hkv, N, Nkv, D, scale, causal, &var, &need);
   if (rc) return rc;
   fa::FwdArgs a;
-  a.q = reinterpret_cast<const fa::half_t*>(q);
-  a.k = reinterpret_cast<const fa::half_t*>(k);
-  a.v = reinterpret_cast<const fa::half_t*>(v);
-  a.o = reinterpret_cast<fa::half_t*>(o);
+  a.q = elems(in.q);
+  a.k = elems(in.k);
+  a.v = elems(in.v);
+  a.ql = in.ql;
+  a.kl = in.kl;
+  a.o = elems(o);
   a.lse = lse;
+  a.d = in.d;
   a.N = (int)N;
   a.Nkv = (int)Nkv;
   a.Hq = (int)Hq;
@@ -881,8 +948,34 @@ static int fwd_impl(int dt, const char* name, const fa_half_t* q, const fa_half_
   a.part = static_cast<float*>(workspace);
   hipError_t e = fn(a, s);
   if (e != hipSuccess) return launch_result(e, name);
-  return launch_result(fa::launch_fwd_combine(a.part, a.o, lse, B * Hq * N, (int)D, sp.nsplit, dt, s),
-                       name);
+  return launch_result(
+      fa::launch_fwd_combine(a.part, a.o, lse, B * Hq * N, (int)D, a.d, sp.nsplit, dt, s), name);
+}
+
+// The forward on contiguous tensors of the kernel width.
+static int fwd_impl(int dt, const char* name, const fa_half_t* q, const fa_half_t* k,
+                    const fa_half_t* v, fa_half_t* o, float* lse, int64_t B, int64_t Hq,
+                    int64_t Hkv, int64_t N, int64_t Nkv, int64_t D, float scale, int causal,
+                    void* stream, void* workspace = nullptr, int64_t workspace_bytes = 0) {
+  return fwd_launch_impl(dt, name, contiguous_inputs(q, k, v, nullptr, Hq, Hkv, N, Nkv, D), o, lse,
+                         B, Hq, Hkv, N, Nkv, D, scale, causal, stream, workspace, workspace_bytes);
+}
+
+// The forward on strided tensors of any head size the kernels hold.
+static int fwd_view_impl(int dt, const char* name, const fa_half_t* q, const fa_half_t* k,
+                         const fa_half_t* v, fa_half_t* o, float* lse, const int64_t* strides,
+                         int64_t B, int64_t Hq, int64_t Hkv, int64_t N, int64_t Nkv, int64_t D,
+                         float scale, int causal, void* workspace,
+                         int64_t workspace_bytes, void* stream) {
+  const int64_t W = view_width(name, D);
+  if (W < 0) return (int)W;
+  int rc = check_common(B, Hq, Hkv, N, W);
+  if (rc) return rc;
+  if ((rc = check_kv_length(Nkv, W))) return rc;
+  Inputs in;
+  if ((rc = view_inputs(name, q, k, v, nullptr, strides, N, Nkv, D, &in))) return rc;
+  return fwd_launch_impl(dt, name, in, o, lse, B, Hq, Hkv, N, Nkv, W, scale, causal, stream,
+                         workspace, workspace_bytes);
 }
 
 int64_t fa_fwd_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t N_q, int64_t N_kv,
@@ -946,10 +1039,10 @@ static int preprocess_impl(int dt, const char* name, const fa_half_t* o, const f
   int rc = check_common(B, Hq, 1, N, D);
   if (rc) return rc;
   if ((rc = check_aligned(name, {o, dO, delta}))) return rc;
-  return launch_result(fa::launch_preprocess(reinterpret_cast<const fa::half_t*>(o),
-                                          reinterpret_cast<const fa::half_t*>(dO), delta,
-                                          B * Hq * N, (int)D, dt, static_cast<hipStream_t>(stream)),
-                    name);
+  return launch_result(
+      fa::launch_preprocess(elems(o), elems(dO), packed(Hq, N, D), delta, B, Hq, N, (int)D, (int)D,
+                            dt, static_cast<hipStream_t>(stream)),
+      name);
 }
 
 static int dkdv_impl(int dt, const char* name, const fa_half_t* q, const fa_half_t* k,
@@ -965,9 +1058,10 @@ static int dkdv_impl(int dt, const char* name, const fa_half_t* q, const fa_half
   if ((rc = check_scale(scale))) return rc;
   const fa::Variant* var = select_dkdv(fa::head_dim_index(D), causal, B, Hq, Hkv, N, Nkv, dt);
   if (!var) return fail(FA_ERR_BAD_TILING, "%s: no kernel for the selected tiling", name);
-  fa::BwdArgs a = bwd_args(q, k, v, dO, lse, delta, B, Hq, Hkv, N, Nkv, scale);
-  a.dk = reinterpret_cast<fa::half_t*>(dk);
-  a.dv = reinterpret_cast<fa::half_t*>(dv);
+  fa::BwdArgs a = bwd_args(contiguous_inputs(q, k, v, dO, Hq, Hkv, N, Nkv, D), lse, delta, B, Hq,
+                           Hkv, N, Nkv, scale);
+  a.dk = elems(dk);
+  a.dv = elems(dv);
   auto fn = reinterpret_cast<fa::bwd_launch_fn>(var->fn[dt][fa::head_dim_index(D)][causal ? 1 : 0]);
   return launch_result(fn(a, static_cast<hipStream_t>(stream)), name);
 }
@@ -994,23 +1088,23 @@ int64_t fa_bwd_dkdv_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t 
   return dkdv_workspace_impl("fa_bwd_dkdv_workspace_bytes", B, Hq, Hkv, N, N, D, causal);
 }
 
-static int dkdv_ws_impl(int dt, const char* name, const fa_half_t* q, const fa_half_t* k,
-                        const fa_half_t* v, const fa_half_t* dO, const float* lse,
-                        const float* delta, fa_half_t* dk, fa_half_t* dv, int64_t B, int64_t Hq,
-                        int64_t Hkv, int64_t N, int64_t Nkv, int64_t D, float scale, int causal,
-                        void* workspace, int64_t workspace_bytes, void* stream) {
-  if (!q || !k || !v || !dO || !lse || !delta || !dk || !dv)
+static int dkdv_ws_launch_impl(int dt, const char* name, const Inputs& in, const float* lse,
+                               const float* delta, fa_half_t* dk, fa_half_t* dv, int64_t B,
+                               int64_t Hq, int64_t Hkv, int64_t N, int64_t Nkv, int64_t D,
+                               float scale, int causal, void* workspace, int64_t workspace_bytes,
+                               void* stream) {
+  if (!in.q || !in.k || !in.v || !in.dO || !lse || !delta || !dk || !dv)
     return fail(FA_ERR_NULL_POINTER, "%s: null pointer", name);
   int rc = check_common(B, Hq, Hkv, N, D);
   if (rc) return rc;
   if ((rc = check_kv_length(Nkv, D))) return rc;
-  if ((rc = check_aligned(name, {q, k, v, dO, lse, delta, dk, dv}))) return rc;
+  if ((rc = check_aligned(name, {in.q, in.k, in.v, in.dO, lse, delta, dk, dv}))) return rc;
   if ((rc = check_scale(scale))) return rc;
   const fa::Variant* var = select_dkdv(fa::head_dim_index(D), causal, B, Hq, Hkv, N, Nkv, dt);
   if (!var) return fail(FA_ERR_BAD_TILING, "%s: no kernel for the selected tiling", name);
-  fa::BwdArgs a = bwd_args(q, k, v, dO, lse, delta, B, Hq, Hkv, N, Nkv, scale);
-  a.dk = reinterpret_cast<fa::half_t*>(dk);
-  a.dv = reinterpret_cast<fa::half_t*>(dv);
+  fa::BwdArgs a = bwd_args(in, lse, delta, B, Hq, Hkv, N, Nkv, scale);
+  a.dk = elems(dk);
+  a.dv = elems(dv);
   const int nsplit = dkdv_split(*var, B, Hq, Hkv, N, Nkv, causal);
   const int64_t need = split_workspace_bytes(nsplit, B, Hkv, Nkv, D);
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -1027,8 +1121,18 @@ static int dkdv_ws_impl(int dt, const char* name, const fa_half_t* q, const fa_h
   a.part = static_cast<float*>(workspace);
   hipError_t e = fn(a, s);
   if (e != hipSuccess) return launch_result(e, name);
-  return launch_result(fa::launch_split_reduce(a.part, a.dk, a.dv, B * Hkv * Nkv * D, nsplit, dt, s),
-                    name);
+  return launch_result(
+      fa::launch_split_reduce(a.part, a.dk, a.dv, B * Hkv * Nkv, (int)D, a.d, nsplit, dt, s), name);
+}
+
+static int dkdv_ws_impl(int dt, const char* name, const fa_half_t* q, const fa_half_t* k,
+                        const fa_half_t* v, const fa_half_t* dO, const float* lse,
+                        const float* delta, fa_half_t* dk, fa_half_t* dv, int64_t B, int64_t Hq,
+                        int64_t Hkv, int64_t N, int64_t Nkv, int64_t D, float scale, int causal,
+                        void* workspace, int64_t workspace_bytes, void* stream) {
+  return dkdv_ws_launch_impl(dt, name, contiguous_inputs(q, k, v, dO, Hq, Hkv, N, Nkv, D), lse,
+                             delta, dk, dv, B, Hq, Hkv, N, Nkv, D, scale, causal, workspace,
+                             workspace_bytes, stream);
 }
 
 static int dq_impl(int dt, const char* name, const fa_half_t* q, const fa_half_t* k,
@@ -1044,29 +1148,30 @@ static int dq_impl(int dt, const char* name, const fa_half_t* q, const fa_half_t
   if ((rc = check_scale(scale))) return rc;
   const fa::Variant* var = select_dq(fa::head_dim_index(D), causal, N, B * Hq, dt);
   if (!var) return fail(FA_ERR_BAD_TILING, "%s: no kernel for the selected tiling", name);
-  fa::BwdArgs a = bwd_args(q, k, v, dO, lse, delta, B, Hq, Hkv, N, Nkv, scale);
-  a.dq = reinterpret_cast<fa::half_t*>(dq);
+  fa::BwdArgs a = bwd_args(contiguous_inputs(q, k, v, dO, Hq, Hkv, N, Nkv, D), lse, delta, B, Hq,
+                           Hkv, N, Nkv, scale);
+  a.dq = elems(dq);
   auto fn = reinterpret_cast<fa::bwd_launch_fn>(var->fn[dt][fa::head_dim_index(D)][causal ? 1 : 0]);
   return launch_result(fn(a, static_cast<hipStream_t>(stream)), name);
 }
 
-static int dq_delta_impl(int dt, const char* name, const fa_half_t* q, const fa_half_t* k,
-                         const fa_half_t* v, const fa_half_t* o, const fa_half_t* dO,
-                         const float* lse, float* delta, fa_half_t* dq, int64_t B, int64_t Hq,
-                         int64_t Hkv, int64_t N, int64_t Nkv, int64_t D, float scale, int causal,
-                         void* stream, void* workspace = nullptr, int64_t workspace_bytes = 0) {
-  if (!q || !k || !v || !o || !dO || !lse || !delta || !dq)
+static int dq_delta_launch_impl(int dt, const char* name, const Inputs& in, const fa_half_t* o,
+                                const float* lse, float* delta, fa_half_t* dq, int64_t B,
+                                int64_t Hq, int64_t Hkv, int64_t N, int64_t Nkv, int64_t D,
+                                float scale, int causal, void* stream, void* workspace,
+                                int64_t workspace_bytes) {
+  if (!in.q || !in.k || !in.v || !o || !in.dO || !lse || !delta || !dq)
     return fail(FA_ERR_NULL_POINTER, "%s: null pointer", name);
   int rc = check_common(B, Hq, Hkv, N, D);
   if (rc) return rc;
   if ((rc = check_kv_length(Nkv, D))) return rc;
-  if ((rc = check_aligned(name, {q, k, v, o, dO, lse, delta, dq}))) return rc;
+  if ((rc = check_aligned(name, {in.q, in.k, in.v, o, in.dO, lse, delta, dq}))) return rc;
   if ((rc = check_scale(scale))) return rc;
   const fa::Variant* var = select_dq(fa::head_dim_index(D), causal, N, B * Hq, dt);
   if (!var) return fail(FA_ERR_BAD_TILING, "%s: no kernel for the selected tiling", name);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  fa::BwdArgs a = bwd_args(q, k, v, dO, lse, delta, B, Hq, Hkv, N, Nkv, scale);
-  a.dq = reinterpret_cast<fa::half_t*>(dq);
+  fa::BwdArgs a = bwd_args(in, lse, delta, B, Hq, Hkv, N, Nkv, scale);
+  a.dq = elems(dq);
   // Split mode (few work-groups, a workspace given): fp32 partial dQ per key range, then summed.
   const FwdSplit sp = dq_split(*var, B, Hq, N, Nkv, causal);
   const int64_t need = dq_workspace_bytes(sp, B, Hq, N, D);
@@ -1082,18 +1187,28 @@ static int dq_delta_impl(int dt, const char* name, const fa_half_t* q, const fa_
     a.part = static_cast<float*>(workspace);
   }
   if (var->flags & fa::kFusesDelta) {
-    a.o = reinterpret_cast<const fa::half_t*>(o);
+    a.o = elems(o);
     a.delta_out = delta;
   } else {
-    hipError_t e = fa::launch_preprocess(reinterpret_cast<const fa::half_t*>(o),
-                                         reinterpret_cast<const fa::half_t*>(dO), delta,
-                                         B * Hq * N, (int)D, dt, s);
+    hipError_t e =
+        fa::launch_preprocess(elems(o), elems(in.dO), in.ql, delta, B, Hq, N, (int)D, in.d, dt, s);
     if (e != hipSuccess) return launch_result(e, name);
   }
   auto fn = reinterpret_cast<fa::bwd_launch_fn>(var->fn[dt][fa::head_dim_index(D)][causal ? 1 : 0]);
   hipError_t e = fn(a, s);
   if (e != hipSuccess || !split) return launch_result(e, name);
-  return launch_result(fa::launch_split_sum(a.part, a.dq, B * Hq * N * D, sp.nsplit, dt, s), name);
+  return launch_result(
+      fa::launch_split_sum(a.part, a.dq, B * Hq * N, (int)D, a.d, sp.nsplit, dt, s), name);
+}
+
+static int dq_delta_impl(int dt, const char* name, const fa_half_t* q, const fa_half_t* k,
+                         const fa_half_t* v, const fa_half_t* o, const fa_half_t* dO,
+                         const float* lse, float* delta, fa_half_t* dq, int64_t B, int64_t Hq,
+                         int64_t Hkv, int64_t N, int64_t Nkv, int64_t D, float scale, int causal,
+                         void* stream, void* workspace = nullptr, int64_t workspace_bytes = 0) {
+  return dq_delta_launch_impl(dt, name, contiguous_inputs(q, k, v, dO, Hq, Hkv, N, Nkv, D), o, lse,
+                              delta, dq, B, Hq, Hkv, N, Nkv, D, scale, causal, stream, workspace,
+                              workspace_bytes);
 }
 
 int64_t fa_bwd_dq_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t N_q, int64_t N_kv,
@@ -1203,18 +1318,18 @@ int64_t fa_bwd_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t N_q, 
   return bytes;
 }
 
-static int bwd_impl(int dt, const char* name, const fa_half_t* q, const fa_half_t* k,
-                    const fa_half_t* v, const fa_half_t* o, const fa_half_t* dO,
-                    const float* lse, float* delta, fa_half_t* dq, fa_half_t* dk, fa_half_t* dv,
-                    int64_t B, int64_t Hq, int64_t Hkv, int64_t N, int64_t Nkv, int64_t D,
-                    float scale, int causal, void* workspace, int64_t workspace_bytes,
-                    void* stream) {
-  if (!q || !k || !v || !o || !dO || !lse || !delta || !dq || !dk || !dv)
+static int bwd_launch_impl(int dt, const char* name, const Inputs& in, const fa_half_t* o,
+                           const float* lse, float* delta, fa_half_t* dq, fa_half_t* dk,
+                           fa_half_t* dv, int64_t B, int64_t Hq, int64_t Hkv, int64_t N,
+                           int64_t Nkv, int64_t D, float scale, int causal, void* workspace,
+                           int64_t workspace_bytes, void* stream) {
+  if (!in.q || !in.k || !in.v || !o || !in.dO || !lse || !delta || !dq || !dk || !dv)
     return fail(FA_ERR_NULL_POINTER, "%s: null pointer", name);
   int rc = check_common(B, Hq, Hkv, N, D);
   if (rc) return rc;
   if ((rc = check_kv_length(Nkv, D))) return rc;
-  if ((rc = check_aligned(name, {q, k, v, o, dO, lse, delta, dq, dk, dv}))) return rc;
+  if ((rc = check_aligned(name, {in.q, in.k, in.v, o, in.dO, lse, delta, dq, dk, dv})))
+    return rc;
   if ((rc = check_scale(scale))) return rc;
   BwdPlan p;
   if (!plan_bwd(dt, B, Hq, Hkv, N, Nkv, D, causal, &p))
@@ -1229,29 +1344,56 @@ static int bwd_impl(int dt, const char* name, const fa_half_t* q, const fa_half_
   }
   if (p.pair && ws != nullptr) {
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const auto* o16 = reinterpret_cast<const fa::half_t*>(o);
-    const auto* do16 = reinterpret_cast<const fa::half_t*>(dO);
-    hipError_t e = fa::launch_preprocess(o16, do16, delta, B * Hq * N, (int)D, dt, s);
+    hipError_t e = fa::launch_preprocess(elems(o), elems(in.dO), in.ql, delta, B, Hq, N, (int)D, in.d, dt, s);
     if (e != hipSuccess) return launch_result(e, name);
-    fa::BwdArgs ad = bwd_args(q, k, v, dO, lse, delta, B, Hq, Hkv, N, Nkv, scale);
-    ad.dk = reinterpret_cast<fa::half_t*>(dk);
-    ad.dv = reinterpret_cast<fa::half_t*>(dv);
+    fa::BwdArgs ad = bwd_args(in, lse, delta, B, Hq, Hkv, N, Nkv, scale);
+    ad.dk = elems(dk);
+    ad.dv = elems(dv);
     ad.nsplit = p.dkdv_nsplit;
     ad.part = reinterpret_cast<float*>(ws + p.dkdv_offset);
-    fa::BwdArgs aq = bwd_args(q, k, v, dO, lse, delta, B, Hq, Hkv, N, Nkv, scale);
-    aq.dq = reinterpret_cast<fa::half_t*>(dq);
+    fa::BwdArgs aq = bwd_args(in, lse, delta, B, Hq, Hkv, N, Nkv, scale);
+    aq.dq = elems(dq);
     e = fa::bwd_pair_launcher(dt, fa::head_dim_index(D), causal)(ad, aq, s);
     if (e != hipSuccess) return launch_result(e, name);
-    return launch_result(
-        fa::launch_split_reduce(ad.part, ad.dk, ad.dv, B * Hkv * Nkv * D, p.dkdv_nsplit, dt, s),
-        name);
+    return launch_result(fa::launch_split_reduce(ad.part, ad.dk, ad.dv, B * Hkv * Nkv, (int)D, in.d,
+                                                 p.dkdv_nsplit, dt, s),
+                         name);
   }
-  rc = dq_delta_impl(dt, name, q, k, v, o, dO, lse, delta, dq, B, Hq, Hkv, N, Nkv, D, scale,
-                     causal, stream, p.dq_bytes > 0 ? ws : nullptr, p.dq_bytes);
+  rc = dq_delta_launch_impl(dt, name, in, o, lse, delta, dq, B, Hq, Hkv, N, Nkv, D, scale, causal,
+                            stream, p.dq_bytes > 0 ? ws : nullptr, p.dq_bytes);
   if (rc) return rc;
-  return dkdv_ws_impl(dt, name, q, k, v, dO, lse, delta, dk, dv, B, Hq, Hkv, N, Nkv, D, scale,
-                      causal, p.dkdv_bytes > 0 && ws ? ws + p.dkdv_offset : nullptr,
-                      p.dkdv_bytes, stream);
+  return dkdv_ws_launch_impl(dt, name, in, lse, delta, dk, dv, B, Hq, Hkv, N, Nkv, D, scale, causal,
+                             p.dkdv_bytes > 0 && ws ? ws + p.dkdv_offset : nullptr, p.dkdv_bytes,
+                             stream);
+}
+
+static int bwd_impl(int dt, const char* name, const fa_half_t* q, const fa_half_t* k,
+                    const fa_half_t* v, const fa_half_t* o, const fa_half_t* dO,
+                    const float* lse, float* delta, fa_half_t* dq, fa_half_t* dk, fa_half_t* dv,
+                    int64_t B, int64_t Hq, int64_t Hkv, int64_t N, int64_t Nkv, int64_t D,
+                    float scale, int causal, void* workspace, int64_t workspace_bytes,
+                    void* stream) {
+  return bwd_launch_impl(dt, name, contiguous_inputs(q, k, v, dO, Hq, Hkv, N, Nkv, D), o, lse,
+                         delta, dq, dk, dv, B, Hq, Hkv, N, Nkv, D, scale, causal, workspace,
+                         workspace_bytes, stream);
+}
+
+// The whole backward on strided q, k, v, dO of any head size the kernels hold.
+static int bwd_view_impl(int dt, const char* name, const fa_half_t* q, const fa_half_t* k,
+                         const fa_half_t* v, const fa_half_t* o, const fa_half_t* dO,
+                         const float* lse, float* delta, fa_half_t* dq, fa_half_t* dk,
+                         fa_half_t* dv, const int64_t* strides, int64_t B, int64_t Hq, int64_t Hkv,
+                         int64_t N, int64_t Nkv, int64_t D, float scale, int causal,
+                         void* workspace, int64_t workspace_bytes, void* stream) {
+  const int64_t W = view_width(name, D);
+  if (W < 0) return (int)W;
+  int rc = check_common(B, Hq, Hkv, N, W);
+  if (rc) return rc;
+  if ((rc = check_kv_length(Nkv, W))) return rc;
+  Inputs in;
+  if ((rc = view_inputs(name, q, k, v, dO, strides, N, Nkv, D, &in))) return rc;
+  return bwd_launch_impl(dt, name, in, o, lse, delta, dq, dk, dv, B, Hq, Hkv, N, Nkv, W, scale,
+                         causal, workspace, workspace_bytes, stream);
 }
 
 int fa_bwd(const fa_half_t* q, const fa_half_t* k, const fa_half_t* v, const fa_half_t* o,
@@ -1359,8 +1501,8 @@ int fa_fwd_noalloc(const fa_half_t* q, const fa_half_t* k, const fa_half_t* v, f
   const char* name = "fa_fwd_noalloc";
   const fa::Variant* var = nullptr;
   int64_t need = 0;
-  int rc = fwd_check(fa::kF16, name, q, k, v, o, lse, B, Hq, Hkv, N_q, N_kv, D, scale, causal,
-                     &var, &need);
+  int rc = fwd_check(fa::kF16, name, contiguous_inputs(q, k, v, nullptr, Hq, Hkv, N_q, N_kv, D), o,
+                     lse, B, Hq, Hkv, N_q, N_kv, D, scale, causal, &var, &need);
   if (rc) return rc;
   if (need > kNoallocScratchBytes)
     return fail(FA_ERR_TOO_LARGE, "%s: this shape's split-KV partials need %lld bytes, more than "
@@ -1437,6 +1579,41 @@ int fa_bwd_dq_delta_kv_bf16(const fa_half_t* q, const fa_half_t* k, const fa_hal
                             void* stream) {
   return dq_delta_impl(fa::kBF16, "fa_bwd_dq_delta_kv_bf16", q, k, v, o, dO, lse, delta, dq, B,
                        Hq, Hkv, N_q, N_kv, D, scale, causal, stream);
+}
+
+// ---- strided tensors, head sizes up to the kernel width ------------------
+int fa_fwd_view(const fa_half_t* q, const fa_half_t* k, const fa_half_t* v, fa_half_t* o,
+                float* lse, const int64_t* strides, int64_t B, int64_t Hq, int64_t Hkv,
+                int64_t N_q, int64_t N_kv, int64_t D, float scale, int causal,
+                void* workspace, int64_t workspace_bytes, void* stream) {
+  return fwd_view_impl(fa::kF16, "fa_fwd_view", q, k, v, o, lse, strides, B, Hq, Hkv, N_q, N_kv, D,
+                       scale, causal, workspace, workspace_bytes, stream);
+}
+int fa_fwd_view_bf16(const fa_half_t* q, const fa_half_t* k, const fa_half_t* v, fa_half_t* o,
+                     float* lse, const int64_t* strides, int64_t B, int64_t Hq, int64_t Hkv,
+                     int64_t N_q, int64_t N_kv, int64_t D, float scale, int causal,
+                     void* workspace, int64_t workspace_bytes, void* stream) {
+  return fwd_view_impl(fa::kBF16, "fa_fwd_view_bf16", q, k, v, o, lse, strides, B, Hq, Hkv, N_q,
+                       N_kv, D, scale, causal, workspace, workspace_bytes, stream);
+}
+int fa_bwd_view(const fa_half_t* q, const fa_half_t* k, const fa_half_t* v, const fa_half_t* o,
+                const fa_half_t* dO, const float* lse, float* delta, fa_half_t* dq, fa_half_t* dk,
+                fa_half_t* dv, const int64_t* strides, int64_t B, int64_t Hq, int64_t Hkv,
+                int64_t N_q, int64_t N_kv, int64_t D, float scale, int causal,
+                void* workspace, int64_t workspace_bytes, void* stream) {
+  return bwd_view_impl(fa::kF16, "fa_bwd_view", q, k, v, o, dO, lse, delta, dq, dk, dv, strides, B,
+                       Hq, Hkv, N_q, N_kv, D, scale, causal, workspace, workspace_bytes,
+                       stream);
+}
+int fa_bwd_view_bf16(const fa_half_t* q, const fa_half_t* k, const fa_half_t* v,
+                     const fa_half_t* o, const fa_half_t* dO, const float* lse, float* delta,
+                     fa_half_t* dq, fa_half_t* dk, fa_half_t* dv, const int64_t* strides,
+                     int64_t B, int64_t Hq, int64_t Hkv, int64_t N_q, int64_t N_kv, int64_t D,
+                     float scale, int causal, void* workspace,
+                     int64_t workspace_bytes, void* stream) {
+  return bwd_view_impl(fa::kBF16, "fa_bwd_view_bf16", q, k, v, o, dO, lse, delta, dq, dk, dv,
+                       strides, B, Hq, Hkv, N_q, N_kv, D, scale, causal, workspace,
+                       workspace_bytes, stream);
 }
 
 int fa_get_tiling(int kernel, int64_t D, int causal, int* out4) {

@@ -9,6 +9,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace fa {
 
 typedef _Float16 half_t;
@@ -31,6 +33,25 @@ constexpr int kRsrcWord3 = 0x00020000;
 __device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
                                            kRsrcWord3);
+}
+
+// A byte offset past every buffer (they hold less than 2^31 bytes), also after
+// the byte offset of a row (below 2^31) is added.
+constexpr uint32_t kOutOfRange = 0x80000000u;
+
+// Byte offset of column `col` of row `row`, rows `stride` elements apart; out of
+// range (reads zero, stores nothing) for the columns from `cols` on.
+__device__ __forceinline__ uint32_t elem_off(int row, int stride, int col, int cols) {
+  return col < cols ? (uint32_t)(row * stride + col) * 2u : kOutOfRange;
+}
+
+// f(cols) with the columns that exist of the kernel width D: an integral constant
+// where that is all of them, so that elem_off's test folds away and a row's chunks
+// differ by immediate offsets.
+template <int D, class F>
+__device__ __forceinline__ void with_cols(int d, F&& f) {
+  if (d == D) f(std::integral_constant<int, D>{});
+  else f(d);
 }
 
 __device__ __forceinline__ u32x4 buf_load_b128(rsrc_t r, uint32_t byte_off) {
@@ -333,38 +354,6 @@ __device__ __forceinline__ half8 read_row(const half_t* tile, int row, int k0, i
   return *reinterpret_cast<const half8*>(tile + swz_offset<D>(row, c));
 }
 
-// Global -> registers -> LDS staging of an R x D tile (16-byte chunks;
-// consecutive threads take consecutive chunks of a row, so global reads
-// coalesce and LDS writes are conflict-free).
-template <int D, int R, int NT>
-struct Stager {
-  static constexpr int DC = D / 8;
-  static constexpr int CHUNKS = R * DC;
-  static constexpr int PER_T = (CHUNKS + NT - 1) / NT;
-  u32x4 reg[PER_T];
-
-  __device__ __forceinline__ void load(rsrc_t r, int row0, int tid) {
-#pragma unroll
-    for (int i = 0; i < PER_T; ++i) {
-      const int ci = tid + i * NT;
-      if (CHUNKS % NT == 0 || ci < CHUNKS) {
-        const int row = ci / DC, c = ci - row * DC;
-        reg[i] = buf_load_b128(r, (uint32_t)((row0 + row) * D + 8 * c) * 2u);
-      }
-    }
-  }
-  __device__ __forceinline__ void store(half_t* tile, int tid) const {
-#pragma unroll
-    for (int i = 0; i < PER_T; ++i) {
-      const int ci = tid + i * NT;
-      if (CHUNKS % NT == 0 || ci < CHUNKS) {
-        const int row = ci / DC, c = ci - row * DC;
-        *reinterpret_cast<u32x4*>(tile + swz_offset<D>(row, c)) = reg[i];
-      }
-    }
-  }
-};
-
 // ---------------------------------------------------------------------------
 // Global -> LDS direct (DMA) staging with buffer_load_dwordx4 ... lds.
 // One wave instruction writes 1 KiB of LDS contiguously (lane l at M0 + 16 l),
@@ -445,9 +434,13 @@ struct DmaStager {
 
   // Per-lane byte offsets inside the tile's global rows (loop-invariant).
   uint32_t voff[PER_WAVE];
-  int piece0;  // first 1 KiB piece of this wave
+  int piece0;          // first 1 KiB piece of this wave
+  uint32_t row_bytes;  // from one global row to the next
 
-  __device__ __forceinline__ void init(int wave, int lane) {
+  // Global rows `stride` elements apart, of which the first `cols` columns exist;
+  // the chunks past them read zeros.
+  __device__ __forceinline__ void init(int wave, int lane, int stride, int cols) {
+    row_bytes = (uint32_t)stride * 2u;
     piece0 = INSTR >= NW ? wave * PER_WAVE : wave % INSTR;
 #pragma unroll
     for (int i = 0; i < PER_WAVE; ++i) {
@@ -455,13 +448,13 @@ struct DmaStager {
       const int row = byte / (D * 2);
       const int pc = (byte % (D * 2)) / 16;
       const int c = swz_chunk<D>(row, pc);  // XOR swizzle is an involution
-      voff[i] = (uint32_t)(row * D + 8 * c) * 2u;
+      voff[i] = elem_off(row, stride, 8 * c, cols);
     }
   }
   // Tile rows [row0, row0 + R) of the buffer -> LDS tile at `tile`.
   __device__ __forceinline__ void issue(int4v rsrc, int row0, const half_t* tile, int) const {
     const uint32_t base = lds_addr(tile) + (uint32_t)piece0 * 1024u;
-    const uint32_t roff = (uint32_t)row0 * D * 2u;
+    const uint32_t roff = (uint32_t)row0 * row_bytes;
 #pragma unroll
     for (int i = 0; i < PER_WAVE; ++i) dma_b128(rsrc, roff + voff[i], base + 1024u * i);
   }
@@ -469,11 +462,12 @@ struct DmaStager {
 
 // The K rows and the V rows of one key unit -> LDS tiles at byte address
 // `base` (K) and base + TILE_BYTES (V), this wave's one or two 1 KiB pieces of
-// each, in one asm block. `row_off` is the unit's first row as a byte offset.
+// each, in one asm block. `row0` is the unit's first row.
 template <int TILE_BYTES, class Dma>
-__device__ __forceinline__ void issue_kv_unit(const Dma& dma, int4v r_k, int4v r_v,
-                                              uint32_t row_off, uint32_t base) {
+__device__ __forceinline__ void issue_kv_unit(const Dma& dma, int4v r_k, int4v r_v, int row0,
+                                              uint32_t base) {
   static_assert(Dma::PER_WAVE == 1 || Dma::PER_WAVE == 2, "one or two tile pieces per wave");
+  const uint32_t row_off = (uint32_t)row0 * dma.row_bytes;
   const uint32_t vt = row_off + dma.voff[0];
   uint32_t saved;
   if constexpr (Dma::PER_WAVE == 1) {
@@ -503,6 +497,52 @@ __device__ __forceinline__ void issue_kv_unit(const Dma& dma, int4v r_k, int4v r
         : "=&s"(saved)
         : "v"(vt), "v"(vt1), "s"(r_k), "s"(r_v), "s"(base), "s"(base + 1024u),
           "s"(base + TILE_BYTES), "s"(base + TILE_BYTES + 1024u)
+        : "memory");
+  }
+}
+
+// The same for one query unit of dK/dV: the Q and dO rows, and this wave's 256
+// bytes of LSE or Delta (byte offset aux_off of r_aux -> LDS address aux_lds).
+template <int TILE_BYTES, class Dma>
+__device__ __forceinline__ void issue_q_unit(const Dma& dma, int4v r_q, int4v r_do, int4v r_aux,
+                                             int row0, uint32_t aux_off, uint32_t base,
+                                             uint32_t aux_lds) {
+  static_assert(Dma::PER_WAVE == 1 || Dma::PER_WAVE == 2, "one or two tile pieces per wave");
+  const uint32_t row_off = (uint32_t)row0 * dma.row_bytes;
+  const uint32_t vt = row_off + dma.voff[0];
+  uint32_t saved;
+  if constexpr (Dma::PER_WAVE == 1) {
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %6\n\t"
+        "buffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
+        "s_mov_b32 m0, %7\n\t"
+        "buffer_load_dwordx4 %1, %4, 0 offen lds\n\t"
+        "s_mov_b32 m0, %8\n\t"
+        "buffer_load_dword %2, %5, 0 offen lds\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "v"(vt), "v"(aux_off), "s"(r_q), "s"(r_do), "s"(r_aux), "s"(base),
+          "s"(base + TILE_BYTES), "s"(aux_lds)
+        : "memory");
+  } else {
+    const uint32_t vt1 = row_off + dma.voff[1];
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %7\n\t"
+        "buffer_load_dwordx4 %1, %4, 0 offen lds\n\t"
+        "s_mov_b32 m0, %8\n\t"
+        "buffer_load_dwordx4 %2, %4, 0 offen lds\n\t"
+        "s_mov_b32 m0, %9\n\t"
+        "buffer_load_dwordx4 %1, %5, 0 offen lds\n\t"
+        "s_mov_b32 m0, %10\n\t"
+        "buffer_load_dwordx4 %2, %5, 0 offen lds\n\t"
+        "s_mov_b32 m0, %11\n\t"
+        "buffer_load_dword %3, %6, 0 offen lds\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "v"(vt), "v"(vt1), "v"(aux_off), "s"(r_q), "s"(r_do), "s"(r_aux), "s"(base),
+          "s"(base + 1024u), "s"(base + TILE_BYTES), "s"(base + TILE_BYTES + 1024u), "s"(aux_lds)
         : "memory");
   }
 }

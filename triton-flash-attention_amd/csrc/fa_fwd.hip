@@ -77,20 +77,22 @@ __device__ __forceinline__ void store_fwd_output(const FwdArgs& a, const rsrc_t&
   const int64_t prow = ((int64_t)split * a.BH + head) * a.N + qrow;
   float* po = split_mode ? a.part + prow * D : nullptr;  // part is null in one-pass mode
   const bool row_ok = qrow < a.N;
+  with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-  for (int db = 0; db < D / 32; ++db)
+    for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-    for (int jq = 0; jq < 4; ++jq) {
-      float4v v;
+      for (int jq = 0; jq < 4; ++jq) {
+        float4v v;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = o[db][4 * jq + e] * inv;
-      if (split_mode) {
-        if (row_ok) *reinterpret_cast<float4v*>(po + 32 * db + 8 * jq + 4 * g) = v;
-      } else {
-        buf_store_b64(ro, (uint32_t)(qrow * D + 32 * db + 8 * jq + 4 * g) * 2u,
-                      pack4<E>(v[0], v[1], v[2], v[3]));
+        for (int e = 0; e < 4; ++e) v[e] = o[db][4 * jq + e] * inv;
+        const int col = 32 * db + 8 * jq + 4 * g;
+        if (split_mode) {
+          if (row_ok) *reinterpret_cast<float4v*>(po + col) = v;
+        } else {
+          buf_store_b64(ro, elem_off(qrow, cols, col, cols), pack4<E>(v[0], v[1], v[2], v[3]));
+        }
       }
-    }
+  });
   if (g == 0 && row_ok) {
     const float lse = seen ? m + log2_fast(lt) : -INFINITY;
     if (split_mode) a.part[(int64_t)a.nsplit * a.BH * a.N * D + prow] = lse;
@@ -131,15 +133,13 @@ __global__ __launch_bounds__(64 * NW) void fwd_kernel(FwdArgs a) {
   const int head = th.head * P + wave % P;  // wave-uniform
   const int b = head / a.Hq;
   const int hq = head - b * a.Hq;
-  const int kvh = b * a.Hkv + hq / a.group;
+  const int hkv = hq / a.group;
   const int N = a.N;      // queries
   const int Nkv = a.Nkv;  // keys
-  const uint32_t slab = (uint32_t)N * D * 2u;
-  const uint32_t kv_slab = (uint32_t)Nkv * D * 2u;
-  const rsrc_t rq = make_rsrc(a.q + (int64_t)head * N * D, slab);
-  const rsrc_t ro = make_rsrc(a.o + (int64_t)head * N * D, slab);
-  const int4v rk = make_rsrc_words(a.k + (int64_t)kvh * Nkv * D, kv_slab);
-  const int4v rv = make_rsrc_words(a.v + (int64_t)kvh * Nkv * D, kv_slab);
+  const rsrc_t rq = make_rsrc(a.q + a.ql.head(b, hq), a.ql.slab_bytes(N, a.d));
+  const rsrc_t ro = make_rsrc(a.o + (int64_t)head * N * a.d, (uint32_t)(N * a.d) * 2u);
+  const int4v rk = make_rsrc_words(a.k + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
+  const int4v rv = make_rsrc_words(a.v + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
 
   const int bm = T::BM / P;  // query rows per head
   const int q0 = qtile * bm;
@@ -155,16 +155,19 @@ __global__ __launch_bounds__(64 * NW) void fwd_kernel(FwdArgs a) {
   // Q^T operand fragments: lane (query ql, k-half g), d = 16*kk + 8*g .. +7.
   // Completed before the first DMA so no later wait on them drains the ring.
   half8 qf[D / 16];
+  with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk)
-    qf[kk] = __builtin_bit_cast(half8, buf_load_b128(rq, (uint32_t)(qrow * D + 16 * kk + 8 * g) * 2u));
+    for (int kk = 0; kk < D / 16; ++kk)
+      qf[kk] = __builtin_bit_cast(
+          half8, buf_load_b128(rq, elem_off(qrow, a.ql.row, 16 * kk + 8 * g, cols)));
+  });
   wait_all_vm();
 
   // DMA prologue: tiles 0 .. AHEAD-1 into ring slots 0 .. AHEAD-1. Every
   // step then issues exactly one tile (past the end the loads read zeros or
   // unused rows), so the in-flight count is the same at every wait.
   Dma dma;
-  dma.init(wave, lane);
+  dma.init(wave, lane, a.kl.row, a.d);
   auto issue_tile = [&](int t, int slot) {
     const half_t* base = lds + slot * T::STAGE;
     dma.issue(rk, kv_lo + t * BN, base, wave);
@@ -482,15 +485,13 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
   const int head = head_blk * P + wave % P;  // wave-uniform
   const int b = head / a.Hq;
   const int hq = head - b * a.Hq;
-  const int kvh = b * a.Hkv + hq / a.group;
+  const int hkv = hq / a.group;
   const int N = a.N;      // queries
   const int Nkv = a.Nkv;  // keys
-  const uint32_t slab = (uint32_t)N * D * 2u;
-  const uint32_t kv_slab = (uint32_t)Nkv * D * 2u;
-  const rsrc_t rq = make_rsrc(a.q + (int64_t)head * N * D, slab);
-  const rsrc_t ro = make_rsrc(a.o + (int64_t)head * N * D, slab);
-  const int4v r_k = make_rsrc_words(a.k + (int64_t)kvh * Nkv * D, kv_slab);
-  const int4v r_v = make_rsrc_words(a.v + (int64_t)kvh * Nkv * D, kv_slab);
+  const rsrc_t rq = make_rsrc(a.q + a.ql.head(b, hq), a.ql.slab_bytes(N, a.d));
+  const rsrc_t ro = make_rsrc(a.o + (int64_t)head * N * a.d, (uint32_t)(N * a.d) * 2u);
+  const int4v r_k = make_rsrc_words(a.k + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
+  const int4v r_v = make_rsrc_words(a.v + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
 
   const int bm = T::BM / P;  // query rows per head
   const int q0 = qtile * bm;
@@ -499,9 +500,12 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
 
   // Q^T operand fragments: lane (query ql, k-half g), d = 16*kk + 8*g .. +7.
   half8 qf[D / 16];
+  with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk)
-    qf[kk] = __builtin_bit_cast(half8, buf_load_b128(rq, (uint32_t)(qrow * D + 16 * kk + 8 * g) * 2u));
+    for (int kk = 0; kk < D / 16; ++kk)
+      qf[kk] = __builtin_bit_cast(
+          half8, buf_load_b128(rq, elem_off(qrow, a.ql.row, 16 * kk + 8 * g, cols)));
+  });
   wait_all_vm();
 
   const int kv_end = CAUSAL ? min(Nkv, q0 + bm) : Nkv;
@@ -523,13 +527,14 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
   const int s0 = UPS * p0;
 
   Dma dma;
-  dma.init(wave, lane);
+  dma.init(wave, lane, a.kl.row, a.d);
   const uint32_t lds0 = lds_addr(lds);
   int i_row = kv_lo;  // first key row of the next unit to fetch
   auto issue = [&](int slot) __attribute__((always_inline)) {
     const int row0 = i_row < kv_hi ? i_row : Nkv;  // past the range: zeros
-    issue_kv_unit<T::TILE * 2>(dma, r_k, r_v, (uint32_t)row0 * (D * 2u),
-                               lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
+    issue_kv_unit<T::TILE * 2>(
+        dma, r_k, r_v, row0,
+        lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
     i_row += T::KT;
   };
 #pragma unroll
@@ -866,15 +871,13 @@ __device__ __forceinline__ void fwd_pipe16_body(const FwdArgs& a, int split, int
   const int head = head_blk * P + wave % P;  // wave-uniform
   const int b = head / a.Hq;
   const int hq = head - b * a.Hq;
-  const int kvh = b * a.Hkv + hq / a.group;
+  const int hkv = hq / a.group;
   const int N = a.N;      // queries
   const int Nkv = a.Nkv;  // keys
-  const uint32_t slab = (uint32_t)N * D * 2u;
-  const uint32_t kv_slab = (uint32_t)Nkv * D * 2u;
-  const rsrc_t rq = make_rsrc(a.q + (int64_t)head * N * D, slab);
-  const rsrc_t ro = make_rsrc(a.o + (int64_t)head * N * D, slab);
-  const int4v r_k = make_rsrc_words(a.k + (int64_t)kvh * Nkv * D, kv_slab);
-  const int4v r_v = make_rsrc_words(a.v + (int64_t)kvh * Nkv * D, kv_slab);
+  const rsrc_t rq = make_rsrc(a.q + a.ql.head(b, hq), a.ql.slab_bytes(N, a.d));
+  const rsrc_t ro = make_rsrc(a.o + (int64_t)head * N * a.d, (uint32_t)(N * a.d) * 2u);
+  const int4v r_k = make_rsrc_words(a.k + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
+  const int4v r_v = make_rsrc_words(a.v + a.kl.head(b, hkv), a.kl.slab_bytes(Nkv, a.d));
 
   const int bm = BM / P;  // query rows per head
   const int q0 = qtile * bm;
@@ -883,12 +886,14 @@ __device__ __forceinline__ void fwd_pipe16_body(const FwdArgs& a, int split, int
 
   // Q^T operand fragments: column = query 16 qb + c16, d = 32 kd + 8 sg .. +7.
   half8 qf[QB][KD];
+  with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-  for (int qb = 0; qb < QB; ++qb)
+    for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
-    for (int kd = 0; kd < KD; ++kd)
-      qf[qb][kd] = __builtin_bit_cast(
-          half8, buf_load_b128(rq, (uint32_t)((qrow0 + 16 * qb) * D + 32 * kd + 8 * sg) * 2u));
+      for (int kd = 0; kd < KD; ++kd)
+        qf[qb][kd] = __builtin_bit_cast(
+            half8, buf_load_b128(rq, elem_off(qrow0 + 16 * qb, a.ql.row, 32 * kd + 8 * sg, cols)));
+  });
   wait_all_vm();
 
   const int kv_end = CAUSAL ? min(Nkv, q0 + bm) : Nkv;
@@ -901,13 +906,14 @@ __device__ __forceinline__ void fwd_pipe16_body(const FwdArgs& a, int split, int
   const int s0 = p0;
 
   Dma dma;
-  dma.init(wave, lane);
+  dma.init(wave, lane, a.kl.row, a.d);
   const uint32_t lds0 = lds_addr(lds);
   int i_row = kv_lo;  // first key row of the next unit to fetch
   auto issue = [&](int slot) __attribute__((always_inline)) {
     const int row0 = i_row < kv_hi ? i_row : Nkv;  // past the range: zeros
-    issue_kv_unit<T::TILE * 2>(dma, r_k, r_v, (uint32_t)row0 * (D * 2u),
-                               lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
+    issue_kv_unit<T::TILE * 2>(
+        dma, r_k, r_v, row0,
+        lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
     i_row += T::KT;
   };
 #pragma unroll
@@ -1201,18 +1207,20 @@ __device__ __forceinline__ void fwd_pipe16_body(const FwdArgs& a, int split, int
     const bool row_ok = qrow < N;
     const int64_t prow = ((int64_t)split * a.BH + head) * N + qrow;
     float* po = split_mode ? a.part + prow * D : nullptr;  // part is null in one-pass mode
+    with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-    for (int dd = 0; dd < DD; ++dd) {
-      float4v v;
+      for (int dd = 0; dd < DD; ++dd) {
+        float4v v;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = o[dd][qb][e] * inv;
-      if (split_mode) {
-        if (row_ok) *reinterpret_cast<float4v*>(po + 16 * dd + 4 * G) = v;
-      } else {
-        buf_store_b64(ro, (uint32_t)(qrow * D + 16 * dd + 4 * G) * 2u,
-                      pack4<E>(v[0], v[1], v[2], v[3]));
+        for (int e = 0; e < 4; ++e) v[e] = o[dd][qb][e] * inv;
+        const int col = 16 * dd + 4 * G;
+        if (split_mode) {
+          if (row_ok) *reinterpret_cast<float4v*>(po + col) = v;
+        } else {
+          buf_store_b64(ro, elem_off(qrow, cols, col, cols), pack4<E>(v[0], v[1], v[2], v[3]));
+        }
       }
-    }
+    });
     if (G == 0 && row_ok) {
       const float lse = seen ? m[qb] + log2_fast(lt) : -INFINITY;
       if (split_mode) a.part[(int64_t)a.nsplit * a.BH * N * D + prow] = lse;
@@ -1422,12 +1430,13 @@ template <int D, class E>
 __global__ __launch_bounds__(256) void fwd_combine_kernel(const float* __restrict__ part,
                                                           half_t* __restrict__ o,
                                                           float* __restrict__ lse, int64_t rows,
-                                                          int nsplit) {
+                                                          int cols, int nsplit) {
   constexpr int CPR = D / 4;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= rows * CPR) return;
   const int64_t row = i / CPR;
   const int c = (int)(i - row * CPR);
+  if (4 * c >= cols) return;
   const float* plse = part + (int64_t)nsplit * rows * D;
   float ls[kMaxFwdSplitKv];
   float4v v[kMaxFwdSplitKv];
@@ -1457,31 +1466,31 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const float* __restric
   half4 h;
 #pragma unroll
   for (int e = 0; e < 4; ++e) h[e] = to_elem<E>(acc[e] * inv);
-  *reinterpret_cast<half4*>(o + row * D + 4 * c) = h;
+  *reinterpret_cast<half4*>(o + row * cols + 4 * c) = h;
   if (c == 0) lse[row] = mx + log2_fast(wsum);
 }
 
 template <int D, class E>
-hipError_t fwd_combine_launch(const float* part, half_t* o, float* lse, int64_t rows, int nsplit,
-                              hipStream_t stream) {
+hipError_t fwd_combine_launch(const float* part, half_t* o, float* lse, int64_t rows, int cols,
+                              int nsplit, hipStream_t stream) {
   const int64_t blocks = (rows * (D / 4) + 255) / 256;
   if (nsplit < 2 || nsplit > kMaxFwdSplitKv || blocks <= 0 || blocks > 0x7fffffff)
     return hipErrorInvalidValue;
   hipLaunchKernelGGL((fwd_combine_kernel<D, E>), dim3((unsigned)blocks), dim3(256), 0, stream,
-                     part, o, lse, rows, nsplit);
+                     part, o, lse, rows, cols, nsplit);
   return hipGetLastError();
 }
 
 hipError_t launch_fwd_combine(const float* part, half_t* o, float* lse, int64_t rows, int D,
-                              int nsplit, int dtype, hipStream_t stream) {
+                              int cols, int nsplit, int dtype, hipStream_t stream) {
   const bool bf = dtype == kBF16;
   switch (D) {
-    case 32: return bf ? fwd_combine_launch<32, BF16>(part, o, lse, rows, nsplit, stream)
-                       : fwd_combine_launch<32, F16>(part, o, lse, rows, nsplit, stream);
-    case 64: return bf ? fwd_combine_launch<64, BF16>(part, o, lse, rows, nsplit, stream)
-                       : fwd_combine_launch<64, F16>(part, o, lse, rows, nsplit, stream);
-    case 128: return bf ? fwd_combine_launch<128, BF16>(part, o, lse, rows, nsplit, stream)
-                        : fwd_combine_launch<128, F16>(part, o, lse, rows, nsplit, stream);
+    case 32: return bf ? fwd_combine_launch<32, BF16>(part, o, lse, rows, cols, nsplit, stream)
+                       : fwd_combine_launch<32, F16>(part, o, lse, rows, cols, nsplit, stream);
+    case 64: return bf ? fwd_combine_launch<64, BF16>(part, o, lse, rows, cols, nsplit, stream)
+                       : fwd_combine_launch<64, F16>(part, o, lse, rows, cols, nsplit, stream);
+    case 128: return bf ? fwd_combine_launch<128, BF16>(part, o, lse, rows, cols, nsplit, stream)
+                        : fwd_combine_launch<128, F16>(part, o, lse, rows, cols, nsplit, stream);
     default: return hipErrorInvalidValue;
   }
 }

@@ -27,19 +27,50 @@ struct FwdJobs {
   int job[kMaxJobs];
 };
 
+// How input tensors [B, H, N, columns] lie in memory: the columns of a row are
+// consecutive; batches lie `sb` elements apart, heads 8 * `sh8` and rows `row`
+// (all multiples of 8, row >= columns: the kernels move 16-byte chunks). The two
+// tensors that a kernel reads side by side (k and v, q and dO) have one layout, so
+// that they share a work-group's address arithmetic and, in the loop, an offset
+// register; the head stride is held in 32 bits. Each work-group does this
+// arithmetic before its first load: with a layout and 64-bit strides for each of the
+// four tensors the dK/dV launch of B2 H16, 64 queries against 16384 keys (D = 64),
+// 4096 work-groups of two units each, took 76.8 us instead of 72.3, and with two
+// offset registers its bf16 causal build spilled.
+struct Layout {
+  int64_t sb;
+  uint32_t sh8;
+  int row;
+
+  // Elements from the tensor's first to the first of head h of batch b.
+  __host__ __device__ uint64_t head(uint32_t b, uint32_t h) const {
+    return (uint64_t)b * (uint64_t)sb + ((uint64_t)h * sh8 << 3);
+  }
+  // Bytes from a head's first element past its last one, of n rows of `cols`
+  // columns: a buffer of that size reads zeros for rows >= n.
+  __host__ __device__ uint32_t slab_bytes(int n, int cols) const {
+    return ((uint32_t)(n - 1) * (uint32_t)row + (uint32_t)cols) * 2u;
+  }
+};
+
 // Arguments of one forward launch (the values _attn_fwd receives at
-// attention.py:690-718, minus strides: every tensor is contiguous).
+// attention.py:690-718). The kernel of width D serves any head size d <= D that
+// is a multiple of 8: columns past it read as zeros (their 16-byte chunks take
+// an out-of-range offset) and are not stored.
 struct FwdArgs {
   const half_t* q;
   const half_t* k;
   const half_t* v;
-  half_t* o;
+  Layout ql;       // of q
+  Layout kl;       // of k and v
+  half_t* o;       // contiguous [B, Hq, N, d]
   float* lse;
   int N;           // query sequence length
   int Nkv;         // key/value sequence length (== N for self-attention)
   int Hq, Hkv;     // query heads, key/value heads
   int group;       // Hq / Hkv
   int BH;          // B * Hq
+  int d;           // columns of q, k, v and o
   int num_tiles;   // filled in by the launcher
   float c;         // scale * log2(e)
   // Split-KV mode (nsplit > 1): work-group split s covers keys
@@ -69,11 +100,14 @@ struct BwdArgs {
   const half_t* k;
   const half_t* v;
   const half_t* dO;
+  Layout ql;       // of q and dO
+  Layout kl;       // of k and v
   const float* lse;
   const float* delta;
-  half_t* dq;
-  half_t* dk;
-  half_t* dv;
+  half_t* dq;      // contiguous [B, Hq, N, d]
+  half_t* dk;      // contiguous [B, Hkv, Nkv, d]
+  half_t* dv;      // contiguous [B, Hkv, Nkv, d]
+  int d;           // columns of every tensor (see FwdArgs)
   int N;           // query sequence length
   int Nkv;         // key/value sequence length (== N for self-attention)
   int Hq, Hkv, group;
@@ -95,7 +129,7 @@ struct BwdArgs {
   int split_keys;
   // Fused Delta (dQ kernels whose variant has kFusesDelta): when o is set the
   // kernel computes Delta = rowsum(O * dO) itself and writes it to delta_out
-  // instead of reading delta.
+  // instead of reading delta. o is contiguous [B, Hq, N, d].
   const half_t* o;
   float* delta_out;
 };
@@ -173,23 +207,35 @@ bwd_pair_launch_fn bwd_pair_launcher(int dtype, int di, int causal);
 // Waves per work-group of the combined launch (both kinds' tiling).
 int bwd_pair_waves();
 
-// Sum of the nsplit fp32 partial planes into fp16 dK, dV (fixed order).
+// Sum of the nsplit fp32 partial planes (`rows` rows of D values each for dK, then
+// dV) into 16-bit dK, dV of d columns (fixed order).
 // dtype: kF16 or kBF16 (the element type of the 16-bit tensors).
-hipError_t launch_split_reduce(const float* part, half_t* dk, half_t* dv, int64_t plane_elems,
-                               int nsplit, int dtype, hipStream_t stream);
+hipError_t launch_split_reduce(const float* part, half_t* dk, half_t* dv, int64_t rows, int D,
+                               int d, int nsplit, int dtype, hipStream_t stream);
 
-hipError_t launch_preprocess(const half_t* o, const half_t* dO, float* delta, int64_t rows,
-                             int D, int dtype, hipStream_t stream);
+// Delta of o (contiguous) and dO, B x H heads of N rows of cols columns, by the
+// kernel of width D.
+hipError_t launch_preprocess(const half_t* o, const half_t* dO, const Layout& dol, float* delta,
+                             int64_t B, int64_t H, int64_t N, int D, int cols, int dtype,
+                             hipStream_t stream);
 
-// Sum of nsplit fp32 partial planes of `elems` values into 16-bit `out`.
-hipError_t launch_split_sum(const float* part, half_t* out, int64_t elems, int nsplit, int dtype,
-                            hipStream_t stream);
+// Sum of nsplit fp32 partial planes of `rows` rows of D values into 16-bit `out` of
+// `cols` columns.
+hipError_t launch_split_sum(const float* part, half_t* out, int64_t rows, int D, int cols,
+                            int nsplit, int dtype, hipStream_t stream);
 
 // Merge of the forward's nsplit partials (FwdArgs::part) into O (16-bit) and
 // base-2 LSE, rows = B * Hq * N: O = sum_s w_s O_s / sum_s w_s with
 // w_s = exp2(lse_s - max_s lse_s), LSE = max + log2(sum_s w_s).
+// The partials have D columns, o the first `cols` of them.
 hipError_t launch_fwd_combine(const float* part, half_t* o, float* lse, int64_t rows, int D,
-                              int nsplit, int dtype, hipStream_t stream);
+                              int cols, int nsplit, int dtype, hipStream_t stream);
+
+inline int log2_of(int x) {
+  int s = 0;
+  while ((1 << s) < x) ++s;
+  return s;
+}
 
 inline int head_dim_index(int64_t D) {
   return D == 32 ? 0 : D == 64 ? 1 : D == 128 ? 2 : -1;

@@ -5,15 +5,21 @@
 // attention.py:673-771) runs its forward and backward in Python. At small
 // shapes that costs more than the kernels: the Python Function's bookkeeping
 // and the backward's trip through the autograd engine into Python take ~90 us
-// per fwd+bwd on top of the op layer. This binding makes the same library
-// calls from a C++ torch::autograd::Function: fa_fwd_kv (or fa_fwd_ws when the
-// forward splits its keys) and fa_bwd, with the same arguments, the same
-// workspaces and on torch's current stream, so its results are identical bit
-// for bit. forward() serves calls that need no gradient the same way (the op
-// layer's flash_fwd, without the Python around it). Both serve the plain case
-// only: a positive scale and one kernel head size (32, 64 or 128) for q, k and
-// v; attention.py keeps the Python path for the rest (negative or zero scales,
-// padded head sizes, forward-mode AD).
+// per fwd+bwd on top of the op layer. This binding makes the same kernel
+// launches from a C++ torch::autograd::Function, through fa_fwd_view and
+// fa_bwd_view, with the same workspaces and on torch's current stream, so its
+// results are identical bit for bit. forward() serves calls that need no
+// gradient the same way (the op layer's flash_fwd, without the Python around
+// it). Both serve positive scales and one head size, a multiple of 8, for q, k
+// and v; attention.py keeps the Python path for the rest (negative or zero
+// scales, other head sizes, forward-mode AD).
+//
+// The kernels read strided q, k, v and dO and head sizes below their width as
+// they stand. A model's transposed projections, slices of a fused projection
+// and the filled part of a key/value cache are thus passed on without a copy
+// (B1 Hq32 Hkv8 N3001 D128: the three copies took 34 us beside an 82 us forward;
+// one query against a 3001-token part of a cache, 16 beside 23). operand() says
+// which tensors qualify; the others are copied.
 //
 // The library's entry points come from the copy Python has already loaded
 // (init() takes their addresses), so one libfa_gfx950.so serves both paths.
@@ -22,27 +28,26 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <stdexcept>
 #include <string>
 
 namespace {
 
-using FwdKv = int (*)(const void*, const void*, const void*, void*, void*, int64_t, int64_t,
-                      int64_t, int64_t, int64_t, int64_t, float, int, void*);
-using FwdWs = int (*)(const void*, const void*, const void*, void*, void*, int64_t, int64_t,
-                      int64_t, int64_t, int64_t, int64_t, float, int, void*, int64_t, void*);
+using FwdView = int (*)(const void*, const void*, const void*, void*, void*, const int64_t*,
+                        int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, float, int, void*,
+                        int64_t, void*);
+using BwdView = int (*)(const void*, const void*, const void*, const void*, const void*,
+                        const void*, void*, void*, void*, void*, const int64_t*, int64_t, int64_t,
+                        int64_t, int64_t, int64_t, int64_t, float, int, void*, int64_t, void*);
 using WsBytes = int64_t (*)(int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int);
-using Bwd = int (*)(const void*, const void*, const void*, const void*, const void*,
-                    const void*, void*, void*, void*, void*, int64_t, int64_t, int64_t, int64_t,
-                    int64_t, int64_t, float, int, void*, int64_t, void*);
 using LastError = const char* (*)();
 
 // Entry points; index 0 = fp16, 1 = bf16.
 struct Entries {
-  FwdKv fwd_kv[2] = {nullptr, nullptr};
-  FwdWs fwd_ws[2] = {nullptr, nullptr};
-  Bwd bwd[2] = {nullptr, nullptr};
+  FwdView fwd[2] = {nullptr, nullptr};
+  BwdView bwd[2] = {nullptr, nullptr};
   WsBytes fwd_ws_bytes = nullptr;
   WsBytes bwd_ws_bytes = nullptr;
   LastError last_error = nullptr;
@@ -50,8 +55,8 @@ struct Entries {
 Entries g;
 
 bool ready() {
-  return g.fwd_kv[0] && g.fwd_kv[1] && g.fwd_ws[0] && g.fwd_ws[1] && g.bwd[0] && g.bwd[1] &&
-         g.fwd_ws_bytes && g.bwd_ws_bytes && g.last_error;
+  return g.fwd[0] && g.fwd[1] && g.bwd[0] && g.bwd[1] && g.fwd_ws_bytes && g.bwd_ws_bytes &&
+         g.last_error;
 }
 
 // The library's error as the Python binding words it (_lib.FlashAttentionError).
@@ -79,6 +84,49 @@ at::Tensor aligned(const at::Tensor& t) {
              : c.clone(at::MemoryFormat::Contiguous);
 }
 
+// An input as the kernels read it: rows of consecutive columns, batches, heads and
+// rows `stride` elements apart.
+struct Operand {
+  at::Tensor t;
+  int64_t stride[3];
+};
+
+// Whether the kernels can read t [B, H, N, columns] as it stands: consecutive,
+// 16-byte aligned rows that do not overlap, within 32-bit byte offsets of their
+// head (the library's bounds, fa_capi.hip view_inputs). A dimension of one element
+// has no stride to speak of.
+bool readable(const at::Tensor& t) {
+  if (t.is_neg() || t.stride(3) != 1 || reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0)
+    return false;
+  for (int i = 0; i < 3; ++i)
+    if (t.size(i) > 1 && t.stride(i) % 8 != 0) return false;
+  if (t.size(1) > 1 && t.stride(1) >= (int64_t{1} << 35)) return false;
+  const int64_t n = t.size(2), row = t.stride(2);
+  return n == 1 || (row >= t.size(3) && row < (int64_t{1} << 30) &&
+                    (n + 4096) * row * 2 < (int64_t{1} << 31));
+}
+
+Operand as_operand(const at::Tensor& t) {
+  Operand o{t, {t.stride(0), t.stride(1), t.stride(2)}};
+  // strides of one-element dimensions as a packed tensor has them
+  if (t.size(2) == 1) o.stride[2] = t.size(3);
+  if (t.size(1) == 1) o.stride[1] = t.size(2) * o.stride[2];
+  if (t.size(0) == 1) o.stride[0] = t.size(1) * o.stride[1];
+  return o;
+}
+
+Operand operand(const at::Tensor& t) {
+  return as_operand(readable(t) ? t : aligned(t.resolve_neg()));
+}
+
+// Two operands that a kernel reads side by side need one layout: where theirs
+// differ, the strided ones are copied.
+void pair_up(Operand& a, Operand& b) {
+  if (std::equal(a.stride, a.stride + 3, b.stride)) return;
+  a = as_operand(aligned(a.t));
+  b = as_operand(aligned(b.t));
+}
+
 void* stream_of(const at::Tensor& t) {
   return static_cast<void*>(c10::hip::getCurrentHIPStream(t.device().index()).stream());
 }
@@ -91,6 +139,8 @@ at::Tensor workspace(int64_t bytes, const at::Tensor& like) {
 
 struct Dims {
   int64_t B, Hq, Hkv, N, Nkv, D;
+  // The kernel width that holds the head size (it sizes the workspaces).
+  int64_t width() const { return D <= 32 ? 32 : D <= 64 ? 64 : 128; }
 };
 
 Dims dims_of(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
@@ -105,8 +155,8 @@ Dims dims_of(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
   return {q.size(0), q.size(1), k.size(1), q.size(2), k.size(2), q.size(3)};
 }
 
-// The forward launch (the op layer's flash_fwd): O and the base-2 LSE of
-// aligned q, k, v on the current stream of their device.
+// The forward launch (the op layer's flash_fwd): O and the base-2 LSE of q, k, v
+// (as the kernels read them) on the current stream of their device.
 struct Forward {
   at::Tensor q, k, v, o, lse;
 };
@@ -115,22 +165,21 @@ Forward run_forward(const at::Tensor& query, const at::Tensor& key, const at::Te
                     bool causal, double scale) {
   const Dims d = dims_of(query, key, value);
   const int e = elem_index(query);
-  Forward f{aligned(query), aligned(key), aligned(value), at::Tensor(), at::Tensor()};
-  c10::DeviceGuard guard(f.q.device());
-  f.o = at::empty_like(f.q);
-  f.lse = at::empty({d.B, d.Hq, d.N}, f.q.options().dtype(at::kFloat));
+  c10::DeviceGuard guard(query.device());
+  const Operand q = operand(query);
+  Operand k = operand(key), v = operand(value);
+  pair_up(k, v);
+  Forward f{q.t, k.t, v.t, at::Tensor(), at::Tensor()};
+  const int64_t strides[6] = {q.stride[0], q.stride[1], q.stride[2],
+                              k.stride[0], k.stride[1], k.stride[2]};
+  f.o = at::empty({d.B, d.Hq, d.N, d.D}, q.t.options());
+  f.lse = at::empty({d.B, d.Hq, d.N}, q.t.options().dtype(at::kFloat));
   const int c = causal ? 1 : 0;
-  const float s = static_cast<float>(scale);
-  const int64_t ws_bytes = g.fwd_ws_bytes(d.B, d.Hq, d.Hkv, d.N, d.Nkv, d.D, c);
-  const at::Tensor ws = workspace(ws_bytes, f.q);
-  void* stream = stream_of(f.q);
-  if (ws_bytes > 0)
-    check(g.fwd_ws[e](f.q.data_ptr(), f.k.data_ptr(), f.v.data_ptr(), f.o.data_ptr(),
-                      f.lse.data_ptr(), d.B, d.Hq, d.Hkv, d.N, d.Nkv, d.D, s, c, ws.data_ptr(),
-                      ws_bytes, stream));
-  else
-    check(g.fwd_kv[e](f.q.data_ptr(), f.k.data_ptr(), f.v.data_ptr(), f.o.data_ptr(),
-                      f.lse.data_ptr(), d.B, d.Hq, d.Hkv, d.N, d.Nkv, d.D, s, c, stream));
+  const int64_t ws_bytes = g.fwd_ws_bytes(d.B, d.Hq, d.Hkv, d.N, d.Nkv, d.width(), c);
+  const at::Tensor ws = workspace(ws_bytes, q.t);
+  check(g.fwd[e](q.t.data_ptr(), k.t.data_ptr(), v.t.data_ptr(), f.o.data_ptr(), f.lse.data_ptr(),
+                 strides, d.B, d.Hq, d.Hkv, d.N, d.Nkv, d.D, static_cast<float>(scale), c,
+                 ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, stream_of(q.t)));
   return f;
 }
 
@@ -146,25 +195,35 @@ class FlashAttention : public torch::autograd::Function<FlashAttention> {
     return f.o;
   }
 
+  // The strides are read from the saved tensors as they come back (a saved-tensor
+  // hook may return them laid out otherwise than they were packed).
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
                                                  torch::autograd::variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    const at::Tensor &q = saved[0], &k = saved[1], &v = saved[2], &o = saved[3], &lse = saved[4];
+    const Dims d = dims_of(saved[0], saved[1], saved[2]);
+    const int e = elem_index(saved[0]);
+    c10::DeviceGuard guard(saved[0].device());
+    Operand q = operand(saved[0]), k = operand(saved[1]), v = operand(saved[2]);
+    Operand dO = operand(grads[0]);
+    pair_up(k, v);
+    pair_up(q, dO);
+    const at::Tensor o = aligned(saved[3]), lse = aligned(saved[4]);
     const bool causal = ctx->saved_data["causal"].toBool();
     const float s = static_cast<float>(ctx->saved_data["scale"].toDouble());
-    const Dims d = dims_of(q, k, v);
-    const int e = elem_index(q);
-    const at::Tensor dO = aligned(grads[0]);
-    c10::DeviceGuard guard(q.device());
+    const int64_t strides[6] = {q.stride[0], q.stride[1], q.stride[2],
+                                k.stride[0], k.stride[1], k.stride[2]};
     const int c = causal ? 1 : 0;
-    const int64_t ws_bytes = g.bwd_ws_bytes(d.B, d.Hq, d.Hkv, d.N, d.Nkv, d.D, c);
-    at::Tensor delta = at::empty({d.B, d.Hq, d.N}, q.options().dtype(at::kFloat));
-    at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
-    const at::Tensor ws = workspace(ws_bytes, q);
-    check(g.bwd[e](q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dO.data_ptr(),
-                   lse.data_ptr(), delta.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-                   d.B, d.Hq, d.Hkv, d.N, d.Nkv, d.D, s, c,
-                   ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, stream_of(q)));
+    const int64_t ws_bytes = g.bwd_ws_bytes(d.B, d.Hq, d.Hkv, d.N, d.Nkv, d.width(), c);
+    const auto like = q.t.options();
+    at::Tensor delta = at::empty({d.B, d.Hq, d.N}, like.dtype(at::kFloat));
+    at::Tensor dq = at::empty({d.B, d.Hq, d.N, d.D}, like);
+    at::Tensor dk = at::empty({d.B, d.Hkv, d.Nkv, d.D}, like);
+    at::Tensor dv = at::empty({d.B, d.Hkv, d.Nkv, d.D}, like);
+    const at::Tensor ws = workspace(ws_bytes, q.t);
+    check(g.bwd[e](q.t.data_ptr(), k.t.data_ptr(), v.t.data_ptr(), o.data_ptr(),
+                   dO.t.data_ptr(), lse.data_ptr(), delta.data_ptr(), dq.data_ptr(),
+                   dk.data_ptr(), dv.data_ptr(), strides, d.B, d.Hq, d.Hkv, d.N, d.Nkv, d.D, s, c,
+                   ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, stream_of(q.t)));
     return {dq, dk, dv, at::Tensor(), at::Tensor()};
   }
 };
@@ -184,19 +243,16 @@ at::Tensor forward_only(const at::Tensor& query, const at::Tensor& key, const at
   return run_forward(query, key, value, causal, scale).o;
 }
 
-// Takes the entry points' addresses: fa_fwd_kv, fa_fwd_kv_bf16, fa_fwd_ws,
-// fa_fwd_ws_bf16, fa_bwd, fa_bwd_bf16, fa_fwd_workspace_bytes,
-// fa_bwd_workspace_bytes, fa_last_error.
-void init(int64_t fwd_kv, int64_t fwd_kv_bf16, int64_t fwd_ws, int64_t fwd_ws_bf16, int64_t bwd,
-          int64_t bwd_bf16, int64_t fwd_ws_bytes, int64_t bwd_ws_bytes, int64_t last_error) {
+// Takes the entry points' addresses: fa_fwd_view, fa_fwd_view_bf16, fa_bwd_view,
+// fa_bwd_view_bf16, fa_fwd_workspace_bytes, fa_bwd_workspace_bytes, fa_last_error.
+void init(int64_t fwd, int64_t fwd_bf16, int64_t bwd, int64_t bwd_bf16, int64_t fwd_ws_bytes,
+          int64_t bwd_ws_bytes, int64_t last_error) {
   auto fn = [](int64_t a) { return reinterpret_cast<void*>(static_cast<uintptr_t>(a)); };
   Entries e;
-  e.fwd_kv[0] = reinterpret_cast<FwdKv>(fn(fwd_kv));
-  e.fwd_kv[1] = reinterpret_cast<FwdKv>(fn(fwd_kv_bf16));
-  e.fwd_ws[0] = reinterpret_cast<FwdWs>(fn(fwd_ws));
-  e.fwd_ws[1] = reinterpret_cast<FwdWs>(fn(fwd_ws_bf16));
-  e.bwd[0] = reinterpret_cast<Bwd>(fn(bwd));
-  e.bwd[1] = reinterpret_cast<Bwd>(fn(bwd_bf16));
+  e.fwd[0] = reinterpret_cast<FwdView>(fn(fwd));
+  e.fwd[1] = reinterpret_cast<FwdView>(fn(fwd_bf16));
+  e.bwd[0] = reinterpret_cast<BwdView>(fn(bwd));
+  e.bwd[1] = reinterpret_cast<BwdView>(fn(bwd_bf16));
   e.fwd_ws_bytes = reinterpret_cast<WsBytes>(fn(fwd_ws_bytes));
   e.bwd_ws_bytes = reinterpret_cast<WsBytes>(fn(bwd_ws_bytes));
   e.last_error = reinterpret_cast<LastError>(fn(last_error));
@@ -207,7 +263,7 @@ void init(int64_t fwd_kv, int64_t fwd_kv_bf16, int64_t fwd_ws, int64_t fwd_ws_bf
 }  // namespace
 
 PYBIND11_MODULE(_fa_native, m) {
-  m.doc() = "C++ autograd binding of libfa_gfx950.so (fa_fwd_kv / fa_fwd_ws and fa_bwd)";
+  m.doc() = "C++ autograd binding of libfa_gfx950.so (fa_fwd_view and fa_bwd_view)";
   m.def("init", &init);
   m.def("ready", &ready);
   m.def("attention", &attention);

@@ -14,7 +14,7 @@ from pathlib import Path
 
 from ._build import LIB_PATH
 
-ABI_VERSION = 7
+ABI_VERSION = 8
 
 FA_OK = 0
 FA_ERR_NULL_POINTER = -1
@@ -24,6 +24,7 @@ FA_ERR_TOO_LARGE = -4
 FA_ERR_BAD_SCALE = -5
 FA_ERR_BAD_TILING = -6
 FA_ERR_MISALIGNED = -7
+FA_ERR_BAD_STRIDE = -8
 
 KERNEL_FWD = 0
 KERNEL_DKDV = 1
@@ -92,6 +93,11 @@ SIGNATURES["fa_bwd"] = (
     (_P,) * 10 + (_I64, _I64, _I64, _I64, _I64, _I64, _F32, _INT, _P, _I64, _P),
 )
 SIGNATURES["fa_bwd_bf16"] = SIGNATURES["fa_bwd"]
+# Strided tensors: the tensors, their strides, sizes, workspace, its size, stream.
+_view = (_P,) + (_I64,) * 6 + (_F32, _INT, _P, _I64, _P)
+SIGNATURES["fa_fwd_view"] = SIGNATURES["fa_fwd_view_bf16"] = (_INT, (_P,) * 5 + _view)
+SIGNATURES["fa_bwd_view"] = SIGNATURES["fa_bwd_view_bf16"] = (_INT, (_P,) * 10 + _view)
+del _view
 # Forward without allocation (device-resident scratch): fa_fwd_kv's arguments.
 SIGNATURES["fa_fwd_noalloc"] = SIGNATURES["fa_fwd_kv"]
 SIGNATURES["fa_fwd_noalloc_max_workspace_bytes"] = (_I64, ())

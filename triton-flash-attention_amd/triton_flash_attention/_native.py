@@ -1,9 +1,10 @@
 """Loader of the C++ autograd binding (``_fa_native.so``, csrc/fa_native.cpp).
 
 The binding runs the public API's training path (forward + backward through
-the autograd engine) in C++ with the same library calls as the Python
+the autograd engine) in C++ with the same kernel launches as the Python
 ``TritonAttention`` Function, so its results are identical bit for bit; it
-only saves host time. It is built in-tree next to libfa_gfx950.so
+saves host time, and the copies the Python Function makes of strided inputs and
+of head sizes between the kernels' widths. It is built in-tree next to libfa_gfx950.so
 (``_build.build_native``) and takes the entry points of the copy of the
 library that ``_lib`` has loaded. If it is missing or fails to load, the
 public API uses the Python Function (the same kernels); ``status()`` says why.
@@ -22,9 +23,8 @@ NAME = "_fa_native"
 PATH = Path(__file__).resolve().parent / f"{NAME}.so"
 
 # Entry points handed to init(), in its argument order.
-ENTRY_POINTS = ("fa_fwd_kv", "fa_fwd_kv_bf16", "fa_fwd_ws", "fa_fwd_ws_bf16", "fa_bwd",
-                "fa_bwd_bf16", "fa_fwd_workspace_bytes", "fa_bwd_workspace_bytes",
-                "fa_last_error")
+ENTRY_POINTS = ("fa_fwd_view", "fa_fwd_view_bf16", "fa_bwd_view", "fa_bwd_view_bf16",
+                "fa_fwd_workspace_bytes", "fa_bwd_workspace_bytes", "fa_last_error")
 
 _module = None
 _error: str | None = None
@@ -75,6 +75,7 @@ def forward(query, key, value, causal: bool, scale: float):
 
 def attention(query, key, value, causal: bool, scale: float):
     """O = attention(query, key, value), differentiable, through the binding.
-    The caller guarantees the served case: contiguous fp16/bf16 GPU tensors,
-    one head size for q, k, v among 32, 64, 128, and a positive scale."""
+    The caller guarantees the served case: fp16/bf16 GPU tensors (any strides:
+    what the kernels cannot read as it stands is copied), one head size for q, k
+    and v that is a multiple of 8 up to 128, and a positive scale."""
     return _module.attention(query, key, value, bool(causal), float(scale))

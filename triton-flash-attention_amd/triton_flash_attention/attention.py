@@ -30,9 +30,10 @@ the reference's first-rule reason (ref 639-642, "the custom kernel currently
 specializes in self-attention") so that callers matching on it keep working,
 followed by the rule that decided here. Head sizes other than the kernels'
 32, 64 and 128, and a value head size other than the query/key one, are served
-up to 128: :class:`TritonAttention` zero-pads the operands to the smallest
-kernel width that holds both sizes (zero columns add exact zeros to every dot
-product) and slices the results back.
+up to 128 by the smallest kernel width that holds both sizes (zero columns add
+exact zeros to every dot product): the kernels read one size that is a multiple of
+8 as it stands; for the others, and in :class:`TritonAttention`, the operands are
+zero-padded and the results sliced back.
 
 The backend keeps the reference's name "triton" so existing call sites
 (``backend="triton"``) run unchanged; it now means "the custom fused kernel".
@@ -319,13 +320,26 @@ class TritonAttention(torch.autograd.Function):
 
 
 def _native_serves(query: torch.Tensor, value: torch.Tensor, softmax_scale: float) -> bool:
-    """Whether the C++ binding (``_native``) runs this call: it makes
-    TritonAttention's launches (or, without autograd, the forward's) for a
-    positive scale and one kernel head size for q, k and v; padded head sizes,
+    """Whether the C++ binding (``_native``) runs this call at the head sizes'
+    own kernel: it makes TritonAttention's launches (or, without autograd, the
+    forward's) for a positive scale and one kernel head size for q, k and v;
     negative or zero scales and forward-mode AD stay in Python."""
     head_dim = query.shape[-1]
     return (head_dim in _SUPPORTED_HEAD_DIMS and value.shape[-1] == head_dim
-            and not _forward_ad_active() and _kernel_scale(softmax_scale)[1] == "plain"
+            and _native_scale(softmax_scale))
+
+
+def _native_narrow(query: torch.Tensor, value: torch.Tensor, softmax_scale: float) -> bool:
+    """The same for another head size (one for q, k and v): the kernel of the
+    next width reads the columns that exist, without padded copies, where they
+    fill whole 16-byte chunks."""
+    head_dim = query.shape[-1]
+    return (head_dim not in _SUPPORTED_HEAD_DIMS and value.shape[-1] == head_dim
+            and head_dim % 8 == 0 and _native_scale(softmax_scale))
+
+
+def _native_scale(softmax_scale: float) -> bool:
+    return (not _forward_ad_active() and _kernel_scale(softmax_scale)[1] == "plain"
             and _native.available())
 
 
@@ -470,17 +484,19 @@ def scaled_dot_product_attention(
             query, key, value, is_causal=is_causal, scale=scale, enable_gqa=enable_gqa
         )
 
+    differentiable = (torch.is_grad_enabled() and (
+        query.requires_grad or key.requires_grad or value.requires_grad)) or _forward_ad_active()
+    if (_native_serves(query, value, softmax_scale)
+            or _native_narrow(query, value, softmax_scale)):
+        # TritonAttention's launches (or only the forward's) from C++: less host
+        # time, and strided inputs are read as they stand.
+        run = _native.attention if differentiable else _native.forward
+        return run(query, key, value, is_causal, softmax_scale)
     query, key, value = query.contiguous(), key.contiguous(), value.contiguous()
-    if (torch.is_grad_enabled() and (query.requires_grad or key.requires_grad
-                                     or value.requires_grad)) or _forward_ad_active():
-        if _native_serves(query, value, softmax_scale):
-            # The same library calls as TritonAttention, from C++ (less host time).
-            return _native.attention(query, key, value, is_causal, softmax_scale)
+    if differentiable:
         return TritonAttention.apply(query, key, value, is_causal, softmax_scale)
     # No gradient can flow (inference, or under torch.no_grad()): the same
     # forward launch without the autograd Function's bookkeeping.
-    if _native_serves(query, value, softmax_scale):
-        return _native.forward(query, key, value, is_causal, softmax_scale)
     output = _padded_forward(query, key, value, is_causal, softmax_scale)[3]
     return _unpad_output(output, value.shape[-1])
 
