@@ -195,29 +195,6 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
   const int k0w = k0 + 32 * wave;
   const int krow = k0w + ql;
 
-  // -fp16(c K) and -V as B operands (column = key ql, d = 16*kk + 8*g .. +7).
-  // The scaled key operand is the reference's k_scaled (attention.py:435):
-  // c K in fp32 rounded to fp16. With the S accumulator started from LSE',
-  // the MFMA yields LSE' - s and P = exp2(-acc) needs no multiply-add.
-  const float c = a.c;
-  half8 kf[D / 16], vn[D / 16];
-  with_cols<D>(a.d, [&](auto cols) {
-#pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) {
-      const uint32_t off = elem_off(krow, a.kl.row, 16 * kk + 8 * g, cols);
-      kf[kk] = __builtin_bit_cast(half8, buf_load_b128(rk, off));
-      vn[kk] = neg8(__builtin_bit_cast(half8, buf_load_b128(rv, off)));
-    }
-  });
-  wait_all_vm();
-#pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) kf[kk][e] = to_elem<E>(-c * elem_to_f32<E>(kf[kk][e]));
-  // Opaque from here on, so that the operands are not recomputed inside the loop.
-#pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk) asm volatile("" : "+v"(kf[kk]), "+v"(vn[kk]));
-
   const int q_begin = CAUSAL ? k0 : 0;  // k0 is a multiple of 32
   // Under the causal mask a key tile past the last query (N < Nkv) sees no
   // query: it takes no unit (every chunk gets none, as the chunks past the
@@ -269,8 +246,36 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
       set_head();
     }
   };
+  // The units the first step needs, then the register operands, so that both
+  // latencies run at once; the units in flight over the first barrier follow the
+  // wait.
 #pragma unroll
-  for (int u = 0; u < T::AHEAD; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
+  for (int u = 0; u < 3; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
+  // -fp16(c K) and -V as B operands (column = key ql, d = 16*kk + 8*g .. +7).
+  // The scaled key operand is the reference's k_scaled (attention.py:435):
+  // c K in fp32 rounded to fp16. With the S accumulator started from LSE',
+  // the MFMA yields LSE' - s and P = exp2(-acc) needs no multiply-add.
+  const float c = a.c;
+  half8 kf[D / 16], vn[D / 16];
+  with_cols<D>(a.d, [&](auto cols) {
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk) {
+      const uint32_t off = elem_off(krow, a.kl.row, 16 * kk + 8 * g, cols);
+      kf[kk] = __builtin_bit_cast(half8, buf_load_b128(rk, off));
+      vn[kk] = neg8(__builtin_bit_cast(half8, buf_load_b128(rv, off)));
+    }
+  });
+  wait_all_vm();
+#pragma unroll
+  for (int kk = 0; kk < D / 16; ++kk)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) kf[kk][e] = to_elem<E>(-c * elem_to_f32<E>(kf[kk][e]));
+  // Opaque from here on, so that the operands are not recomputed inside the loop.
+#pragma unroll
+  for (int kk = 0; kk < D / 16; ++kk) asm volatile("" : "+v"(kf[kk]), "+v"(vn[kk]));
+
+#pragma unroll
+  for (int u = 3; u < T::AHEAD; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
 
   // The slot read as "unit -1" holds zeros (its P and dS' are zero too);
   // the +inf table of fully masked units.
@@ -702,6 +707,34 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
   const int q0w = q0 + 32 * wave;
   const int qrow = q0w + ql;
 
+  const int kv_end = CAUSAL ? min(Nkv, q0 + T::BQ) : Nkv;
+  // This work-group's keys [kv_lo, kv_hi): all of [0, kv_end) unless split.
+  const int kv_lo = split * a.split_keys;
+  const int kv_hi = min(kv_end, kv_lo + a.split_keys);
+  const int nunits = kv_hi > kv_lo ? (kv_hi - kv_lo + T::KT - 1) / T::KT : 0;
+  const int npad = (nunits + NS - 1) / NS * NS;
+  // The units end in the ring's last slot: the first ring turn starts at step
+  // p0 (slot s0), so at most one padding unit runs and the loop over whole
+  // turns has no branches between its steps.
+  const int p0 = __builtin_amdgcn_readfirstlane((npad - nunits) / 2);
+  const int s0 = 2 * p0;
+
+  Dma dma;
+  dma.init(wave, lane, a.kl.row, a.d);
+  const uint32_t lds0 = lds_addr(lds);
+  int i_row = kv_lo;  // first key row of the next unit to fetch
+  auto issue = [&](int slot) __attribute__((always_inline)) {
+    const int row0 = i_row < kv_hi ? i_row : Nkv;  // past the range: zeros
+    issue_kv_unit<T::TILE * 2>(
+        dma, r_k, r_v, row0,
+        lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
+    i_row += T::KT;
+  };
+  // The units the first step needs, then the register operands, so that both
+  // latencies run at once; the units in flight over the first barrier follow the
+  // wait.
+#pragma unroll
+  for (int u = 0; u < 3; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
   // -fp16(c Q) and -dO as B operands (column = query ql, d = 16*kk + 8*g .. +7).
   const float c = a.c;
   half8 qf[D / 16], don[D / 16];
@@ -743,31 +776,8 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
 #pragma unroll
   for (int kk = 0; kk < D / 16; ++kk) asm volatile("" : "+v"(qf[kk]), "+v"(don[kk]));
 
-  const int kv_end = CAUSAL ? min(Nkv, q0 + T::BQ) : Nkv;
-  // This work-group's keys [kv_lo, kv_hi): all of [0, kv_end) unless split.
-  const int kv_lo = split * a.split_keys;
-  const int kv_hi = min(kv_end, kv_lo + a.split_keys);
-  const int nunits = kv_hi > kv_lo ? (kv_hi - kv_lo + T::KT - 1) / T::KT : 0;
-  const int npad = (nunits + NS - 1) / NS * NS;
-  // The units end in the ring's last slot: the first ring turn starts at step
-  // p0 (slot s0), so at most one padding unit runs and the loop over whole
-  // turns has no branches between its steps.
-  const int p0 = __builtin_amdgcn_readfirstlane((npad - nunits) / 2);
-  const int s0 = 2 * p0;
-
-  Dma dma;
-  dma.init(wave, lane, a.kl.row, a.d);
-  const uint32_t lds0 = lds_addr(lds);
-  int i_row = kv_lo;  // first key row of the next unit to fetch
-  auto issue = [&](int slot) __attribute__((always_inline)) {
-    const int row0 = i_row < kv_hi ? i_row : Nkv;  // past the range: zeros
-    issue_kv_unit<T::TILE * 2>(
-        dma, r_k, r_v, row0,
-        lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
-    i_row += T::KT;
-  };
 #pragma unroll
-  for (int u = 0; u < T::AHEAD; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
+  for (int u = 3; u < T::AHEAD; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
 
   // The slot read as "unit -1" holds zeros (its dS' is zero too).
   {

@@ -75,6 +75,32 @@ __device__ __forceinline__ void dq_pipe16_body(const BwdArgs& a, const unsigned 
   const int q0w = q0 + 32 * wave;
   const int qrow0 = q0w + c16;  // query of block qb: qrow0 + 16 qb
 
+  const int kv_end = CAUSAL ? min(Nkv, q0 + T::BQ) : Nkv;
+  // This work-group's keys [kv_lo, kv_hi): all of [0, kv_end) unless split.
+  const int kv_lo = split * a.split_keys;
+  const int kv_hi = min(kv_end, kv_lo + a.split_keys);
+  const int nunits = kv_hi > kv_lo ? (kv_hi - kv_lo + T::KT - 1) / T::KT : 0;
+  const int npad = (nunits + NS - 1) / NS * NS;
+  // The units end in the ring's last slot (rotated start, as in dq_pipe_body).
+  const int p0 = __builtin_amdgcn_readfirstlane((npad - nunits) / 2);
+  const int s0 = 2 * p0;
+
+  Dma dma;
+  dma.init(wave, lane, a.kl.row, a.d);
+  const uint32_t lds0 = lds_addr(lds);
+  int i_row = kv_lo;  // first key row of the next unit to fetch
+  auto issue = [&](int slot) __attribute__((always_inline)) {
+    const int row0 = i_row < kv_hi ? i_row : Nkv;  // past the range: zeros
+    issue_kv_unit<T::TILE * 2>(
+        dma, r_k, r_v, row0,
+        lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
+    i_row += T::KT;
+  };
+  // The units the first step needs, then the register operands, so that both
+  // latencies run at once; the units in flight over the first barrier follow the
+  // wait.
+#pragma unroll
+  for (int u = 0; u < 3; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
   // -fp16(c Q) and -dO as B operands: column = query 16 qb + c16,
   // d = 32 kd + 8 sg .. +7. Rows past N read as zeros (buffer range check).
   const float c = a.c;
@@ -129,29 +155,8 @@ __device__ __forceinline__ void dq_pipe16_body(const BwdArgs& a, const unsigned 
 #pragma unroll
     for (int kd = 0; kd < KD; ++kd) asm volatile("" : "+v"(qf[qb][kd]), "+v"(don[qb][kd]));
 
-  const int kv_end = CAUSAL ? min(Nkv, q0 + T::BQ) : Nkv;
-  // This work-group's keys [kv_lo, kv_hi): all of [0, kv_end) unless split.
-  const int kv_lo = split * a.split_keys;
-  const int kv_hi = min(kv_end, kv_lo + a.split_keys);
-  const int nunits = kv_hi > kv_lo ? (kv_hi - kv_lo + T::KT - 1) / T::KT : 0;
-  const int npad = (nunits + NS - 1) / NS * NS;
-  // The units end in the ring's last slot (rotated start, as in dq_pipe_body).
-  const int p0 = __builtin_amdgcn_readfirstlane((npad - nunits) / 2);
-  const int s0 = 2 * p0;
-
-  Dma dma;
-  dma.init(wave, lane, a.kl.row, a.d);
-  const uint32_t lds0 = lds_addr(lds);
-  int i_row = kv_lo;  // first key row of the next unit to fetch
-  auto issue = [&](int slot) __attribute__((always_inline)) {
-    const int row0 = i_row < kv_hi ? i_row : Nkv;  // past the range: zeros
-    issue_kv_unit<T::TILE * 2>(
-        dma, r_k, r_v, row0,
-        lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
-    i_row += T::KT;
-  };
 #pragma unroll
-  for (int u = 0; u < T::AHEAD; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
+  for (int u = 3; u < T::AHEAD; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
 
   // The slot read as "unit -1" holds zeros (its dS' is zero too).
   {
@@ -524,33 +529,6 @@ __device__ __forceinline__ void dkdv_pipe16_body(const BwdArgs& a, const unsigne
   const int k0w = k0 + 32 * wave;
   const int krow0 = k0w + c16;  // key of block kb: krow0 + 16 kb
 
-  // -fp16(c K) and -V as B operands (column = key 16 kb + c16, d = 32 kd +
-  // 8 sg .. +7); the scaled key operand is the reference's k_scaled
-  // (attention.py:435). Rows past N_kv read as zeros.
-  const float c = a.c;
-  half8 kf[2][KD], vn[2][KD];
-  with_cols<D>(a.d, [&](auto cols) {
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int kd = 0; kd < KD; ++kd) {
-        const uint32_t off = elem_off(krow0 + 16 * kb, a.kl.row, 32 * kd + 8 * sg, cols);
-        kf[kb][kd] = __builtin_bit_cast(half8, buf_load_b128(rk, off));
-        vn[kb][kd] = neg8(__builtin_bit_cast(half8, buf_load_b128(rv, off)));
-      }
-  });
-  wait_all_vm();
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-    for (int kd = 0; kd < KD; ++kd)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) kf[kb][kd][e] = to_elem<E>(-c * elem_to_f32<E>(kf[kb][kd][e]));
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-    for (int kd = 0; kd < KD; ++kd) asm volatile("" : "+v"(kf[kb][kd]), "+v"(vn[kb][kd]));
-
   const int q_begin = CAUSAL ? k0 : 0;  // k0 is a multiple of 32
   const int ntq = max(1, (N - q_begin + T::QT - 1) / T::QT);
   const int total_units = CAUSAL && q_begin >= N ? 0 : QG * ntq;  // as in dkdv_pipe_body
@@ -594,8 +572,40 @@ __device__ __forceinline__ void dkdv_pipe16_body(const BwdArgs& a, const unsigne
       set_head();
     }
   };
+  // The units the first step needs, then the register operands, so that both
+  // latencies run at once; the units in flight over the first barrier follow the
+  // wait.
 #pragma unroll
-  for (int u = 0; u < T::AHEAD; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
+  for (int u = 0; u < 3; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
+  // -fp16(c K) and -V as B operands (column = key 16 kb + c16, d = 32 kd +
+  // 8 sg .. +7); the scaled key operand is the reference's k_scaled
+  // (attention.py:435). Rows past N_kv read as zeros.
+  const float c = a.c;
+  half8 kf[2][KD], vn[2][KD];
+  with_cols<D>(a.d, [&](auto cols) {
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int kd = 0; kd < KD; ++kd) {
+        const uint32_t off = elem_off(krow0 + 16 * kb, a.kl.row, 32 * kd + 8 * sg, cols);
+        kf[kb][kd] = __builtin_bit_cast(half8, buf_load_b128(rk, off));
+        vn[kb][kd] = neg8(__builtin_bit_cast(half8, buf_load_b128(rv, off)));
+      }
+  });
+  wait_all_vm();
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+    for (int kd = 0; kd < KD; ++kd)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) kf[kb][kd][e] = to_elem<E>(-c * elem_to_f32<E>(kf[kb][kd][e]));
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+    for (int kd = 0; kd < KD; ++kd) asm volatile("" : "+v"(kf[kb][kd]), "+v"(vn[kb][kd]));
+
+#pragma unroll
+  for (int u = 3; u < T::AHEAD; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
 
   // The slot read as "unit -1" holds zeros (its P and dS' are zero too);
   // the +inf table of fully masked units.

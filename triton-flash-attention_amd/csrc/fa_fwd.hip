@@ -498,16 +498,6 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
   const int q0w = q0 + 32 * (wave / P);
   const int qrow = q0w + ql;
 
-  // Q^T operand fragments: lane (query ql, k-half g), d = 16*kk + 8*g .. +7.
-  half8 qf[D / 16];
-  with_cols<D>(a.d, [&](auto cols) {
-#pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk)
-      qf[kk] = __builtin_bit_cast(
-          half8, buf_load_b128(rq, elem_off(qrow, a.ql.row, 16 * kk + 8 * g, cols)));
-  });
-  wait_all_vm();
-
   const int kv_end = CAUSAL ? min(Nkv, q0 + bm) : Nkv;
   // This work-group's keys: all of [0, kv_end) unless split; with two key
   // groups, the first ceil(units / 2) units go to group 0, the rest to group
@@ -537,8 +527,22 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
         lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
     i_row += T::KT;
   };
+  // The units the first step needs, then the Q^T operand fragments (lane: query ql,
+  // k-half g, d = 16*kk + 8*g .. +7), so that both latencies run at once; the units
+  // in flight over the first barrier follow the wait.
 #pragma unroll
-  for (int u = 0; u < T::AHEAD; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
+  for (int u = 0; u < T::AHEAD - T::IN_FLIGHT; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
+  half8 qf[D / 16];
+  with_cols<D>(a.d, [&](auto cols) {
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk)
+      qf[kk] = __builtin_bit_cast(
+          half8, buf_load_b128(rq, elem_off(qrow, a.ql.row, 16 * kk + 8 * g, cols)));
+  });
+  wait_all_vm();
+#pragma unroll
+  for (int u = T::AHEAD - T::IN_FLIGHT; u < T::AHEAD; ++u)
+    issue(s0 + u < NS ? s0 + u : s0 + u - NS);
 
   // The V tile read as "unit -1" holds zeros (its P is zero too).
   {
@@ -884,18 +888,6 @@ __device__ __forceinline__ void fwd_pipe16_body(const FwdArgs& a, int split, int
   const int q0w = q0 + 16 * QB * (wave / P);
   const int qrow0 = q0w + c16;  // query of block qb: qrow0 + 16 qb
 
-  // Q^T operand fragments: column = query 16 qb + c16, d = 32 kd + 8 sg .. +7.
-  half8 qf[QB][KD];
-  with_cols<D>(a.d, [&](auto cols) {
-#pragma unroll
-    for (int qb = 0; qb < QB; ++qb)
-#pragma unroll
-      for (int kd = 0; kd < KD; ++kd)
-        qf[qb][kd] = __builtin_bit_cast(
-            half8, buf_load_b128(rq, elem_off(qrow0 + 16 * qb, a.ql.row, 32 * kd + 8 * sg, cols)));
-  });
-  wait_all_vm();
-
   const int kv_end = CAUSAL ? min(Nkv, q0 + bm) : Nkv;
   const int kv_lo = split * a.split_keys;
   const int kv_hi = min(kv_end, kv_lo + a.split_keys);
@@ -916,8 +908,23 @@ __device__ __forceinline__ void fwd_pipe16_body(const FwdArgs& a, int split, int
         lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
     i_row += T::KT;
   };
+  // The first units, the Q^T operand fragments (column = query 16 qb + c16, d =
+  // 32 kd + 8 sg .. +7), the other units (as in fwd_pipe_body).
 #pragma unroll
-  for (int u = 0; u < T::AHEAD; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
+  for (int u = 0; u < T::AHEAD - T::IN_FLIGHT; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
+  half8 qf[QB][KD];
+  with_cols<D>(a.d, [&](auto cols) {
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+      for (int kd = 0; kd < KD; ++kd)
+        qf[qb][kd] = __builtin_bit_cast(
+            half8, buf_load_b128(rq, elem_off(qrow0 + 16 * qb, a.ql.row, 32 * kd + 8 * sg, cols)));
+  });
+  wait_all_vm();
+#pragma unroll
+  for (int u = T::AHEAD - T::IN_FLIGHT; u < T::AHEAD; ++u)
+    issue(s0 + u < NS ? s0 + u : s0 + u - NS);
 
   // The V tile read as "unit -1" holds zeros (its P is zero too).
   {
