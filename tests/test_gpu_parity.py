@@ -2355,3 +2355,43 @@ def test_broadcast_operands_match_contiguous_copies():
     o2 = scaled_dot_product_attention(one.contiguous(), k.contiguous(), k.contiguous(),
                                       backend="triton")
     assert torch.equal(o1, o2)
+
+
+# (B, Hq, Hkv, N_q, N_kv, D): rows per key/value head up to the kernel's 16 and past
+# it, key counts around its 32-key units, its four waves and its key ranges
+DECODE_KERNEL_CASES = [
+    (1, 1, 1, 1, 1, 64), (1, 3, 1, 5, 31, 128), (2, 16, 1, 1, 32, 32), (2, 4, 4, 16, 33, 64),
+    (1, 6, 2, 5, 97, 40), (3, 8, 2, 4, 127, 128), (1, 8, 4, 8, 129, 32), (2, 10, 2, 3, 1000, 96),
+    (1, 4, 2, 8, 2048, 128), (1, 4, 2, 8, 2049, 128), (1, 8, 2, 1, 2561, 64), (2, 4, 1, 4, 5003, 32),
+    (1, 17, 1, 1, 600, 64), (1, 4, 2, 9, 600, 128), (130, 1, 1, 2, 2100, 64),
+]
+
+
+@pytest.mark.parametrize("case", DECODE_KERNEL_CASES,
+                         ids=lambda c: f"B{c[0]}H{c[1]}-{c[2]}Nq{c[3]}Nkv{c[4]}D{c[5]}")
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+def test_decoding_kernel_matches_float64(case, dtype):
+    """The decoding kernel (all rows of a key/value head in one block, keys split
+    over waves and ranges) against 64-bit attention: O within the rounding of P and O
+    (rel-L2 at most 2^-9 + 2^-9 in bf16, 2^-12 + 2^-12 in fp16, round to nearest),
+    LSE within 1e-5; inputs x4 as well, whose row maxima move. Keys and values are
+    the filled part of a cache with NaN around it."""
+    B, Hq, Hkv, N, Nkv, D = case
+    _note(f"decoding kernel {case} {dtype}")
+    g = torch.Generator().manual_seed(Nkv + N + D)
+    for mult in (1.0, 4.0):
+        mk = lambda h, n: (torch.randn((B, h, n, D), generator=g) * mult).to(dtype).to(DEV)
+        q, k, v = mk(Hq, N), mk(Hkv, Nkv), mk(Hkv, Nkv)
+        kc, vc = (_laid_out(t, "cache") for t in (k, v))
+        with torch.no_grad():
+            o = scaled_dot_product_attention(q, kc, vc, enable_gqa=Hq != Hkv, backend="triton")
+        kd, vd = (t.double().repeat_interleave(Hq // Hkv, 1) for t in (k, v))
+        s = (q.double() @ kd.transpose(-1, -2).contiguous()) * D ** -0.5
+        ref = torch.softmax(s, -1) @ vd
+        rel = float((o.double() - ref).norm() / ref.norm())
+        assert rel <= (2 ** -8 if dtype == torch.bfloat16 else 2 ** -11), (mult, rel)
+        if D in (32, 64, 128):
+            o2, lse = _ops.flash_fwd(q, k, v, False, D ** -0.5)
+            assert torch.equal(o2, o)
+            err = float((lse.double() - torch.logsumexp(s, -1) / math.log(2)).abs().max())
+            assert err <= 1e-5 * mult * mult, (mult, err)

@@ -302,7 +302,8 @@ constexpr int64_t kFwdDecodeQueries = 32;
 // (two work-groups per head) 13-17 % slower; with 128 a tie.
 constexpr int64_t kFwdShortQueries = 64;
 
-int fwd_pack(const fa::Variant& var, int64_t group, int64_t N);  // below
+bool fwd_decodes(const fa::Variant& var, int causal, int64_t group, int64_t N);  // below
+int fwd_pack(const fa::Variant& var, int causal, int64_t group, int64_t N);     // below
 
 int64_t visible_keys(int64_t N, int64_t Nkv, int causal);  // below
 
@@ -337,7 +338,7 @@ const fa::Variant* select_fwd(int di, int causal, int64_t N, int64_t Nkv, int64_
   };
   if (N <= kFwdDecodeQueries || (!causal && N <= kFwdShortQueries)) {
     const fa::Variant* half = pick(kFwd16HalfVariant);
-    if (half != var && N <= half->rows / fwd_pack(*half, group, N)) return half;
+    if (half != var && N <= half->rows / fwd_pack(*half, causal, group, N)) return half;
   }
   const int64_t L = visible_keys(N, Nkv, causal);
   if (di == fa::head_dim_index(128)) return pick(fwd_variant_d128(causal, N, L, BH));
@@ -619,6 +620,21 @@ constexpr int64_t kFwdSplitTargetWorkgroups = 768;
 // faster (16.2 vs 21.4 us at B8 Hq32 Hkv8 against 8192 keys).
 constexpr int64_t kFwdSplitTargetFew = 256;
 constexpr int64_t kFwdMinSplitKeys = 1024;
+// The decoding kernel (fa_fwd_decode.hip) runs a range of keys on four waves, so
+// it needs ranges later and shorter: past 2048 keys, for fewer than 128 work-groups
+// (key/value heads), as many as fit the chip's CUs at once (one work-group per CU at
+// D = 128, two below: 48 heads of 20000 keys, D64, 39.9 us on the general tiling, 46.5
+// with 288 work-groups) with at least 512 keys each. MI355X, the whole call from
+// Python, ranges / one pass / the general tiling, us: B2 Hq32 Hkv8 3001 keys D128
+// 15.4 / 18.2 / 23.8, B1 4096 keys 15.1 / 22.0 / 18.2, B8 8192 keys 44.2 / 48.3 / 44.4
+// (D64 24.1 / 26.2 / 24.9, D32 15.6 / 20.2 / 16.7); not taken: B2 1500 keys 14.7 /
+// 11.5 / 21.0, B1 2000 keys 14.7 / 13.6 / 26.4, 128 work-groups (B8 Hkv16) 16 queries
+// 2048 keys 25.7 / 21.4 / 25.0, 8 queries 8192 keys D64 44.5 / 39.1 / 41.1.
+constexpr int64_t kDecodeSplitBelow = 128;
+constexpr int64_t kDecodeSplitTarget = 512;
+constexpr int64_t kDecodeSplitTarget128 = 256;
+constexpr int64_t kDecodeOnePassKeys = 2048;
+constexpr int64_t kDecodeMinSplitKeys = 512;
 constexpr int kMaxFwdSplit = fa::kMaxFwdSplitKv;
 
 struct FwdSplit {
@@ -626,10 +642,18 @@ struct FwdSplit {
   int split_keys;
 };
 
+// Without the mask, a launch of tiling 11 whose query rows per key/value head fit one
+// 16-row block runs the decoding kernel (fa_fwd_decode.hip), which packs all of
+// the group's heads and splits the keys over the work-group's waves.
+bool fwd_decodes(const fa::Variant& var, int causal, int64_t group, int64_t N) {
+  return (var.flags & fa::kFewSplits) && !causal && group * N <= fa::kDecodeRows;
+}
+
 // Query heads per forward work-group: GQA launches of at most 32 queries
 // (decoding) pack gcd(group, waves) heads, which then share each K/V tile the
 // work-group streams; otherwise 1.
-int fwd_pack(const fa::Variant& var, int64_t group, int64_t N) {
+int fwd_pack(const fa::Variant& var, int causal, int64_t group, int64_t N) {
+  if (fwd_decodes(var, causal, group, N)) return (int)group;
   if (N > 32 || group < 2 || (var.flags & fa::kKeyGroups)) return 1;
   return (int)std::gcd<int64_t>(group, var.waves);
 }
@@ -648,19 +672,25 @@ int64_t visible_keys(int64_t N, int64_t Nkv, int causal) {
 // keys, D128, causal: 24 ranges, of which 23 were empty). A launch that does
 // not split keeps the whole key range.
 FwdSplit key_split(int64_t wgs, int64_t Nkv, int64_t visible, int64_t below,
-                   int64_t target = kFwdSplitTargetWorkgroups) {
+                   int64_t target = kFwdSplitTargetWorkgroups,
+                   int64_t min_keys = kFwdMinSplitKeys) {
   const int whole = (int)((Nkv + 127) / 128 * 128);
   if (wgs >= below) return {1, whole};
   int64_t s = (target + wgs - 1) / wgs;
-  s = std::min<int64_t>(s, std::max<int64_t>(1, visible / kFwdMinSplitKeys));
+  s = std::min<int64_t>(s, std::max<int64_t>(1, visible / min_keys));
   s = std::min<int64_t>(s, kMaxFwdSplit);
   if (s <= 1) return {1, whole};
   const int64_t keys = ((visible + s - 1) / s + 127) / 128 * 128;
   return {(int)((visible + keys - 1) / keys), (int)keys};
 }
 
-FwdSplit fwd_split(const fa::Variant& var, int64_t B, int64_t Hq, int64_t N, int64_t Nkv,
-                   int64_t D, int pack, int causal) {
+FwdSplit fwd_split(const fa::Variant& var, int64_t B, int64_t Hq, int64_t Hkv, int64_t N,
+                   int64_t Nkv, int64_t D, int pack, int causal) {
+  if (fwd_decodes(var, causal, Hq / Hkv, N)) {
+    const int64_t wgs = B * Hkv, most = D == 128 ? kDecodeSplitTarget128 : kDecodeSplitTarget;
+    return key_split(wgs, Nkv, Nkv, Nkv > kDecodeOnePassKeys ? kDecodeSplitBelow : 0,
+                     most / wgs * wgs, kDecodeMinSplitKeys);
+  }
   const int64_t rows = var.rows / pack;  // query rows per head and work-group
   const int64_t target = (var.flags & fa::kFewSplits) && D >= 64 ? kFwdSplitTargetFew
                                                                 : kFwdSplitTargetWorkgroups;
@@ -897,7 +927,7 @@ static int fwd_check(int dt, const char* name, const Inputs& in, fa_half_t* o, f
   if ((rc = check_scale(scale))) return rc;
   *var = select_fwd(fa::head_dim_index(D), causal, N, Nkv, B * Hq, Hq / Hkv, dt);
   if (!*var) return fail(FA_ERR_BAD_TILING, "%s: no kernel for the selected tiling", name);
-  const FwdSplit sp = fwd_split(**var, B, Hq, N, Nkv, D, fwd_pack(**var, Hq / Hkv, N), causal);
+  const FwdSplit sp = fwd_split(**var, B, Hq, Hkv, N, Nkv, D, fwd_pack(**var, causal, Hq / Hkv, N), causal);
   *need = fwd_workspace_bytes(sp, B, Hq, N, D);
   return FA_OK;
 }
@@ -927,10 +957,15 @@ static int fwd_launch_impl(int dt, const char* name, const Inputs& in, fa_half_t
   a.BH = (int)(B * Hq);
   a.num_tiles = 0;
   a.c = scale * fa::kLog2e;
-  auto fn = reinterpret_cast<fa::fwd_launch_fn>(var->fn[dt][fa::head_dim_index(D)][causal ? 1 : 0]);
+  const auto tiling =
+      reinterpret_cast<fa::fwd_launch_fn>(var->fn[dt][fa::head_dim_index(D)][causal ? 1 : 0]);
+  const bool decodes = fwd_decodes(*var, causal, Hq / Hkv, N);
+  const auto fn = [&](const fa::FwdArgs& args, hipStream_t st) {
+    return decodes ? fa::launch_fwd_decode(args, (int)D, dt, st) : tiling(args, st);
+  };
   hipStream_t s = static_cast<hipStream_t>(stream);
-  a.pack = fwd_pack(*var, Hq / Hkv, N);
-  const FwdSplit sp = fwd_split(*var, B, Hq, N, Nkv, D, a.pack, causal);
+  a.pack = fwd_pack(*var, causal, Hq / Hkv, N);
+  const FwdSplit sp = fwd_split(*var, B, Hq, Hkv, N, Nkv, D, a.pack, causal);
   a.nsplit = 1;
   a.split_keys = (int)((Nkv + 127) / 128 * 128);
   a.part = nullptr;
@@ -988,7 +1023,7 @@ int64_t fa_fwd_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t N_q, 
   for (int dt : {fa::kF16, fa::kBF16}) {
     const fa::Variant* var = select_fwd(fa::head_dim_index(D), causal, N_q, N_kv, B * Hq, Hq / Hkv, dt);
     if (!var) return fail(FA_ERR_BAD_TILING, "fa_fwd_workspace_bytes: no kernel for the selected tiling");
-    const FwdSplit sp = fwd_split(*var, B, Hq, N_q, N_kv, D, fwd_pack(*var, Hq / Hkv, N_q), causal);
+    const FwdSplit sp = fwd_split(*var, B, Hq, Hkv, N_q, N_kv, D, fwd_pack(*var, causal, Hq / Hkv, N_q), causal);
     bytes = std::max(bytes, fwd_workspace_bytes(sp, B, Hq, N_q, D));
   }
   return bytes;
@@ -1002,8 +1037,8 @@ int fa_fwd_plan_info(int64_t B, int64_t Hq, int64_t Hkv, int64_t N_q, int64_t N_
   if ((rc = check_kv_length(N_kv, D))) return rc;
   const fa::Variant* var = select_fwd(fa::head_dim_index(D), causal, N_q, N_kv, B * Hq, Hq / Hkv, fa::kF16);
   if (!var) return fail(FA_ERR_BAD_TILING, "fa_fwd_plan_info: no kernel for the selected tiling");
-  const int pack = fwd_pack(*var, Hq / Hkv, N_q);
-  const FwdSplit sp = fwd_split(*var, B, Hq, N_q, N_kv, D, pack, causal);
+  const int pack = fwd_pack(*var, causal, Hq / Hkv, N_q);
+  const FwdSplit sp = fwd_split(*var, B, Hq, Hkv, N_q, N_kv, D, pack, causal);
   const int64_t grid_wgs = (N_q + var->rows / pack - 1) / (var->rows / pack) * (B * Hq / pack);
   const auto plan = fwd_launch_plan(*var, causal, pack, sp.nsplit, B * Hq, N_q, N_kv,
                                     compute_units);

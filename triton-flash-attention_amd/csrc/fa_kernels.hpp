@@ -224,6 +224,11 @@ hipError_t launch_preprocess(const half_t* o, const half_t* dO, const Layout& do
 hipError_t launch_split_sum(const float* part, half_t* out, int64_t rows, int D, int cols,
                             int nsplit, int dtype, hipStream_t stream);
 
+// The forward for launches whose query rows per key/value head (group x N) are at
+// most kDecodeRows, without the mask (fa_fwd_decode.hip); pack is unused.
+constexpr int kDecodeRows = 16;
+hipError_t launch_fwd_decode(const FwdArgs& a, int D, int dtype, hipStream_t stream);
+
 // Merge of the forward's nsplit partials (FwdArgs::part) into O (16-bit) and
 // base-2 LSE, rows = B * Hq * N: O = sum_s w_s O_s / sum_s w_s with
 // w_s = exp2(lse_s - max_s lse_s), LSE = max + log2(sum_s w_s).

@@ -23,7 +23,7 @@ INCLUDE_DIR = PACKAGE_DIR.parent.parent / "include"
 LIB_NAME = "libfa_gfx950.so"
 LIB_PATH = PACKAGE_DIR / LIB_NAME
 
-SOURCES = ("fa_fwd.hip", "fa_bwd.hip", "fa_bwd_pair.hip", "fa_capi.hip")
+SOURCES = ("fa_fwd.hip", "fa_fwd_decode.hip", "fa_bwd.hip", "fa_bwd_pair.hip", "fa_capi.hip")
 HEADERS = ("fa_common.hpp", "fa_kernels.hpp", "fa_bwd_pipe.hpp")
 
 # -packed-fp32-ops: no v_pk_{add,mul,fma}_f32 in generated code.

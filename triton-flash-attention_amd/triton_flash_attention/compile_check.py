@@ -76,7 +76,8 @@ def _defaults() -> tuple[str, ...]:
         names.append(f"fa::fwd_pipe16_kernel<32, true, {e}, 2>")
         names += [f"fa::fwd_pipe16_kernel<{d}, {c}, {e}, 1>"
                   for d in (32, 64, 128) for c in ("false", "true")]
-        names += [f"fa::preprocess_kernel<{d}, {e}>" for d in (32, 64, 128)]
+        names += [f"fa::{k}_kernel<{d}, {e}>" for k in ("fwd_decode", "preprocess")
+                  for d in (32, 64, 128)]
         names.append(f"fa::split_reduce_kernel<{e}>")
     names += [f"fa::{k}_kernel<128, false, 4, 32, {e}>" for k in ("dq", "dkdv")
               for e in ("fa::F16", "fa::BF16")]
