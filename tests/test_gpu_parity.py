@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import math
 import sys
+import warnings
 
 import numpy as np
 import pytest
@@ -2395,3 +2396,66 @@ def test_decoding_kernel_matches_float64(case, dtype):
             assert torch.equal(o2, o)
             err = float((lse.double() - torch.logsumexp(s, -1) / math.log(2)).abs().max())
             assert err <= 1e-5 * mult * mult, (mult, err)
+
+
+def test_plain_call_check_agrees_with_the_rules(monkeypatch):
+    """The native check of a plain call says yes only where the rules do, at their
+    scale, and a call that it passes on gives what it gives without the check:
+    the same output, or the same error."""
+    from triton_flash_attention import _native
+    from triton_flash_attention.attention import _dispatch, _kernel_scale, _validate_inputs
+
+    base = dict(q=(2, 4, 5, 64), k=(2, 2, 7, 64), v=None, dt=(torch.float16,) * 3, dev=(DEV,) * 3,
+                is_causal=False, scale=None, enable_gqa=True, backend="auto")
+    yes = [{}, {"dt": (torch.bfloat16,) * 3}, {"is_causal": True}, {"scale": 0.25}, {"backend": "triton"},
+           {"k": (2, 4, 7, 64), "enable_gqa": False}, {"q": (2, 4, 1, 8), "k": (2, 2, 1, 8)},
+           {"q": (1, 3, 9, 96), "k": (1, 1, 9, 96)}]
+    no = [{"enable_gqa": False}, {"enable_gqa": 1}, {"is_causal": 0}, {"is_causal": None}, {"scale": 1},
+          {"scale": -0.5}, {"scale": 0.0}, {"scale": float("nan")}, {"scale": float("inf")}, {"scale": 1e38},
+          {"scale": 1e300}, {"scale": 1e-45}, {"scale": "1"}, {"scale": True}, {"scale": np.float64(0.5)},
+          {"scale": torch.tensor(0.5)}, {"backend": "torch"}, {"backend": "cuda"}, {"backend": None},
+          {"q": (2, 4, 5, 60), "k": (2, 2, 7, 60)}, {"q": (2, 4, 5, 136), "k": (2, 2, 7, 136)},
+          {"q": (2, 4, 5, 0), "k": (2, 2, 7, 0)}, {"q": (2, 4, 0, 64)}, {"k": (2, 2, 0, 64)},
+          {"q": (2, 5, 5, 64)}, {"q": (3, 4, 5, 64)}, {"k": (2, 2, 7, 32)}, {"v": (2, 2, 7, 32)},
+          {"v": (2, 2, 6, 64)}, {"v": (2, 1, 7, 64)}, {"q": (4, 5, 64)}, {"k": (2, 7, 64)},
+          {"v": (2, 2, 1, 7, 64)}, {"dt": (torch.float32,) * 3}, {"dt": (torch.float16, torch.bfloat16, torch.float16)},
+          {"dt": (torch.float16, torch.float16, torch.float32)}, {"dev": ("cpu",) * 3},
+          {"dev": (DEV, DEV, "cpu")}, {"dev": (DEV, "cpu", "cpu")}, {"dev": ("meta",) * 3}]
+
+    def call(c, q, k, v):
+        try:
+            with torch.no_grad(), warnings.catch_warnings():
+                warnings.simplefilter("ignore")
+                return scaled_dot_product_attention(q, k, v, is_causal=c["is_causal"], scale=c["scale"],
+                                                    enable_gqa=c["enable_gqa"], backend=c["backend"])
+        except Exception as exc:  # noqa: BLE001 - compared below
+            return type(exc), str(exc)
+
+    assert _native.available()
+    for change in yes + no:
+        c = {**base, **change}
+        _note(f"plain call {change}")
+        shapes = (c["q"], c["k"], c["v"] or c["k"])
+        q, k, v = (torch.randn(s, generator=torch.Generator().manual_seed(i)).to(t).to(d)
+                   for i, (s, t, d) in enumerate(zip(shapes, c["dt"], c["dev"])))
+        plain = _native.plain_scale(q, k, v, c["is_causal"], c["scale"], c["enable_gqa"])
+        if change in yes:
+            assert plain == (c["scale"] or q.shape[-1] ** -0.5), change
+        if plain:
+            _validate_inputs(q, k, v, enable_gqa=c["enable_gqa"])
+            assert _dispatch(q, k, v).backend == "triton" and _kernel_scale(plain) == (plain, "plain")
+        else:
+            assert change in no, change
+        got = call(c, q, k, v)
+        with monkeypatch.context() as m:
+            m.setattr(_native, "plain_scale", lambda *a: 0.0)
+            want = call(c, q, k, v)
+        if isinstance(want, torch.Tensor):
+            assert got.device == want.device and got.shape == want.shape, change
+            if want.device.type != "meta":  # NaN where the scaled scores overflow
+                torch.testing.assert_close(got, want, rtol=0, atol=0, equal_nan=True)
+        else:
+            assert got == want, change
+    sub = torch.randn(2, 4, 5, 64, device=DEV, dtype=torch.float16).as_subclass(type("Sub", (torch.Tensor,), {}))
+    assert _native.plain_scale(sub, sub, sub, False, None, False) == 0.0
+    assert _native.plain_scale(None, [], 3, False, None, False) == 0.0

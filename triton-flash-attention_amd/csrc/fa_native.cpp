@@ -29,6 +29,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <stdexcept>
 #include <string>
@@ -243,6 +244,41 @@ at::Tensor forward_only(const at::Tensor& query, const at::Tensor& key, const at
   return run_forward(query, key, value, causal, scale).o;
 }
 
+// The softmax scale of a public call that passes every check of attention.py
+// (arguments, _validate_inputs, _decide_rules but the device's architecture,
+// _kernel_scale) well inside its bounds, at one head size that is a multiple of 8;
+// 0.0 for any other call, which attention.py then checks itself, one rule at a time, to
+// word its error or choose its path. In Python the checks of a small call took as
+// long as its forward launch (11-12 us for the two, 4.7 for the launch).
+double plain_scale(py::handle query, py::handle key, py::handle value, py::handle is_causal,
+                   py::handle scale, py::handle enable_gqa) {
+  if (!THPVariable_CheckExact(query.ptr()) || !THPVariable_CheckExact(key.ptr()) ||
+      !THPVariable_CheckExact(value.ptr()) || !PyBool_Check(is_causal.ptr()) ||
+      !PyBool_Check(enable_gqa.ptr()))
+    return 0.0;
+  const at::Tensor& q = THPVariable_Unpack(query.ptr());
+  const at::Tensor& k = THPVariable_Unpack(key.ptr());
+  const at::Tensor& v = THPVariable_Unpack(value.ptr());
+  const at::ScalarType dtype = q.scalar_type();
+  if ((dtype != at::kHalf && dtype != at::kBFloat16) || k.scalar_type() != dtype ||
+      v.scalar_type() != dtype || !q.is_cuda() || k.device() != q.device() ||
+      v.device() != q.device() || q.dim() != 4 || k.dim() != 4 || v.sizes() != k.sizes())
+    return 0.0;
+  const int64_t B = q.size(0), Hq = q.size(1), N = q.size(2), D = q.size(3);
+  const int64_t Hkv = k.size(1), Nkv = k.size(2);
+  constexpr int64_t kMany = int64_t{1} << 20;
+  const auto within = [](int64_t n, int64_t most) { return n >= 1 && n <= most; };
+  if (!within(B, kMany) || !within(Hq, kMany) || !within(Hkv, kMany) || !within(B * Hq, kMany) ||
+      !within(N, kMany) || !within(Nkv, kMany) || !within(D, 128) || D % 8 != 0 ||
+      k.size(0) != B || k.size(3) != D || Hq % Hkv != 0 ||
+      (Hq != Hkv && enable_gqa.ptr() != Py_True))
+    return 0.0;
+  double s = 0.0;
+  if (scale.is_none()) s = std::pow(static_cast<double>(D), -0.5);
+  else if (PyFloat_CheckExact(scale.ptr())) s = PyFloat_AS_DOUBLE(scale.ptr());
+  return s >= 1e-30 && s <= 1e30 ? s : 0.0;
+}
+
 // Takes the entry points' addresses: fa_fwd_view, fa_fwd_view_bf16, fa_bwd_view,
 // fa_bwd_view_bf16, fa_fwd_workspace_bytes, fa_bwd_workspace_bytes, fa_last_error.
 void init(int64_t fwd, int64_t fwd_bf16, int64_t bwd, int64_t bwd_bf16, int64_t fwd_ws_bytes,
@@ -268,4 +304,5 @@ PYBIND11_MODULE(_fa_native, m) {
   m.def("ready", &ready);
   m.def("attention", &attention);
   m.def("forward", &forward_only);
+  m.def("plain_scale", &plain_scale);
 }

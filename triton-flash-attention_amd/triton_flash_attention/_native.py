@@ -67,6 +67,15 @@ def status() -> tuple[bool, str]:
     return available(), _error or ""
 
 
+def plain_scale(query, key, value, is_causal, scale, enable_gqa) -> float:
+    """The softmax scale of a call whose arguments pass every check of the public API,
+    or 0.0 where Python has to look (csrc/fa_native.cpp), which it does for a
+    process's first calls, until one has loaded the binding."""
+    if _module is None:
+        return 0.0
+    return _module.plain_scale(query, key, value, is_causal, scale, enable_gqa)
+
+
 def forward(query, key, value, causal: bool, scale: float):
     """O = attention(query, key, value) without autograd, through the binding
     (same served case as :func:`attention`)."""

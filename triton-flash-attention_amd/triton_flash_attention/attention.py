@@ -339,8 +339,21 @@ def _native_narrow(query: torch.Tensor, value: torch.Tensor, softmax_scale: floa
 
 
 def _native_scale(softmax_scale: float) -> bool:
-    return (not _forward_ad_active() and _kernel_scale(softmax_scale)[1] == "plain"
+    return (not _forward_ad_active()
+            and (1e-30 <= softmax_scale <= 1e30 or _kernel_scale(softmax_scale)[1] == "plain")
             and _native.available())
+
+
+def _differentiable(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor) -> bool:
+    return (torch.is_grad_enabled() and (query.requires_grad or key.requires_grad
+                                         or value.requires_grad)) or _forward_ad_active()
+
+
+def _native_run(query, key, value, is_causal: bool, softmax_scale: float) -> torch.Tensor:
+    """TritonAttention's launches (or only the forward's) from C++: less host time,
+    and strided inputs are read as they stand."""
+    run = _native.attention if _differentiable(query, key, value) else _native.forward
+    return run(query, key, value, is_causal, softmax_scale)
 
 
 def _forward_ad_active() -> bool:
@@ -453,6 +466,13 @@ def scaled_dot_product_attention(
     ``backend="triton"`` requires the custom kernel and raises RuntimeError
     otherwise; ``backend="torch"`` always uses PyTorch SDPA.
     """
+    if backend == "auto" or backend == "triton":
+        # A plain call: one native check in place of the ones below, which word the
+        # errors and choose among the other paths.
+        plain = _native.plain_scale(query, key, value, is_causal, scale, enable_gqa)
+        if (plain and _device_arch(query.device).startswith(_SUPPORTED_ARCH)
+                and (_native_serves(query, value, plain) or _native_narrow(query, value, plain))):
+            return _native_run(query, key, value, is_causal, plain)
     if backend not in ("auto", "triton", "torch"):
         raise ValueError("backend must be one of: 'auto', 'triton', 'torch'")
     if not isinstance(is_causal, bool):
@@ -484,16 +504,11 @@ def scaled_dot_product_attention(
             query, key, value, is_causal=is_causal, scale=scale, enable_gqa=enable_gqa
         )
 
-    differentiable = (torch.is_grad_enabled() and (
-        query.requires_grad or key.requires_grad or value.requires_grad)) or _forward_ad_active()
     if (_native_serves(query, value, softmax_scale)
             or _native_narrow(query, value, softmax_scale)):
-        # TritonAttention's launches (or only the forward's) from C++: less host
-        # time, and strided inputs are read as they stand.
-        run = _native.attention if differentiable else _native.forward
-        return run(query, key, value, is_causal, softmax_scale)
+        return _native_run(query, key, value, is_causal, softmax_scale)
     query, key, value = query.contiguous(), key.contiguous(), value.contiguous()
-    if differentiable:
+    if _differentiable(query, key, value):
         return TritonAttention.apply(query, key, value, is_causal, softmax_scale)
     # No gradient can flow (inference, or under torch.no_grad()): the same
     # forward launch without the autograd Function's bookkeeping.
