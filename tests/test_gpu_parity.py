@@ -2459,3 +2459,27 @@ def test_plain_call_check_agrees_with_the_rules(monkeypatch):
     sub = torch.randn(2, 4, 5, 64, device=DEV, dtype=torch.float16).as_subclass(type("Sub", (torch.Tensor,), {}))
     assert _native.plain_scale(sub, sub, sub, False, None, False) == 0.0
     assert _native.plain_scale(None, [], 3, False, None, False) == 0.0
+
+
+@pytest.mark.parametrize("n_kv", [100, 1500, 3001])  # one unit per wave, one pass, key ranges
+@pytest.mark.parametrize("d", [32, 80, 128])
+def test_decoding_weighs_keys_that_score_minus_infinity_with_zero(d, n_kv):
+    """Infinite key elements score -inf: such keys weigh 0 wherever they lie (the first
+    32-key units of the waves, a whole key range), and a row that scores nothing else
+    is NaN, as softmax has it. Tolerance: rounding to fp16, as the other decoding
+    tests."""
+    _note(f"decode -inf keys d={d} n_kv={n_kv}")
+    q, k, v, _ = make_inputs(2, 8, 2, 1, d, seed=77 + d, n_kv=n_kv)
+    q[..., 0] = q[..., 0].abs() + 0.5
+    k[0, :, :min(n_kv - 20, 1100), 0] = -math.inf
+    k[1, 0, 40:70, 0] = -math.inf
+    k[1, 1, :, 0] = -math.inf
+    with torch.no_grad():
+        o = scaled_dot_product_attention(q.to(DEV), k.to(DEV), v.to(DEV), enable_gqa=True,
+                                         backend="triton").cpu().double()
+    kd, vd = (t.double().repeat_interleave(4, dim=1) for t in (k, v))
+    s = (q.double() * d ** -0.5) @ kd.transpose(2, 3)
+    ref = torch.softmax(s, dim=-1) @ vd
+    assert bool(o[1, 4:].isnan().all()) and bool(ref[1, 4:].isnan().all())
+    assert_close("decode -inf keys", o[0].numpy(), ref[0].numpy())
+    assert_close("decode -inf keys", o[1, :4].numpy(), ref[1, :4].numpy())

@@ -167,33 +167,36 @@ __global__ __launch_bounds__(256) void fwd_decode_kernel(FwdArgs a) {
           if (ka + 16 * kb + 4 * gq + j >= kv_hi) s[kb][j] = -INFINITY;
     }
     half8 pa;
-    auto probs = [&]() {
+    auto probs = [&](float ref) {
       float sum = 0.f;
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const float p = exp2_fast(fmaf(s[kb][j], c, -m));
+          const float p = exp2_fast(fmaf(s[kb][j], c, -ref));
           sum += p;
           pa[4 * kb + j] = to_elem<E>(p);
         }
       return sum;
     };
-    float l_u = probs();
+    float l_u = probs(m);
     if (__builtin_amdgcn_ballot_w64(!(l_u <= kDecodeSumLimit)) != 0) {
       float mt = s[0][0];
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int j = 0; j < 4; ++j) mt = __builtin_fmaxf(mt, s[kb][j]);
-      mt = quarters_max(mt) * c;  // finite: a unit of the loop holds at least one key
+      mt = quarters_max(mt) * c;
       const float m_new = __builtin_fmaxf(m, mt);
-      const float alpha = exp2_fast(m - m_new);
+      // While every key of the wave has scored -inf (infinite inputs) m stays there
+      // and the probabilities are zeros.
+      const float ref = m_new == -INFINITY ? 0.f : m_new;
+      const float alpha = exp2_fast(m - ref);
       l *= alpha;
 #pragma unroll
       for (int dd = 0; dd < DD; ++dd) o[dd] *= alpha;
       m = m_new;
-      l_u = probs();
+      l_u = probs(ref);
     }
     l += l_u;
 #pragma unroll
@@ -225,8 +228,10 @@ __global__ __launch_bounds__(256) void fwd_decode_kernel(FwdArgs a) {
     wt[w] = mw == -INFINITY ? 0.f : exp2_fast(mw - mt);  // a wave that saw no key weighs 0
     lt += wt[w] * xm[(T::NW + w) * T::ROWS + c16];
   }
-  const float inv = lt > 0.f ? 1.0f / lt : 0.f;
+  // A range in which every score is -inf is a partial of weight 0; a row of them is
+  // 0 / 0, as in the combine.
   const bool split_mode = a.nsplit > 1;
+  const float inv = lt > 0.f || !split_mode ? 1.0f / lt : 0.f;
   const int64_t row = (int64_t)(kvh * P + h) * a.N + n;  // of [B * Hq, N]
   const int64_t prow = (int64_t)split * a.BH * a.N + row;
 #pragma unroll
