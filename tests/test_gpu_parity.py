@@ -2483,3 +2483,22 @@ def test_decoding_weighs_keys_that_score_minus_infinity_with_zero(d, n_kv):
     assert bool(o[1, 4:].isnan().all()) and bool(ref[1, 4:].isnan().all())
     assert_close("decode -inf keys", o[0].numpy(), ref[0].numpy())
     assert_close("decode -inf keys", o[1, :4].numpy(), ref[1, :4].numpy())
+
+
+def test_cache_written_between_forward_and_backward():
+    """Part of a cache that takes no gradient may be written again before the backward,
+    which still sees the keys and values of its forward: the gradient of q is the one of
+    contiguous copies, bit for bit."""
+    q, k, v, do = (t.to(DEV) for t in make_inputs(1, 4, 2, 64, 64, seed=91, n_kv=512))
+    grads = []
+    for cached in (False, True):
+        leaf = q.clone().requires_grad_()
+        kk, vv = k.clone(), v.clone()
+        kp, vp = kk[:, :, :300], vv[:, :, :300]
+        if not cached:
+            kp, vp = kp.contiguous(), vp.contiguous()
+        out = scaled_dot_product_attention(leaf, kp, vp, enable_gqa=True, backend="triton")
+        if cached:
+            kk.zero_(), vv.zero_()
+        grads.append(torch.autograd.grad(out, leaf, do)[0])
+    assert torch.equal(*grads)

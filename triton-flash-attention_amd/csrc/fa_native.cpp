@@ -189,7 +189,10 @@ class FlashAttention : public torch::autograd::Function<FlashAttention> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& query,
                             const at::Tensor& key, const at::Tensor& value, bool causal,
                             double scale) {
-    Forward f = run_forward(query, key, value, causal, scale);
+    // A strided tensor without a gradient may be a buffer (part of a key/value cache)
+    // that the program writes again before the backward: its copy is kept.
+    const auto kept = [](const at::Tensor& t) { return t.requires_grad() ? t : t.contiguous(); };
+    Forward f = run_forward(kept(query), kept(key), kept(value), causal, scale);
     ctx->save_for_backward({f.q, f.k, f.v, f.o, f.lse});
     ctx->saved_data["causal"] = causal;
     ctx->saved_data["scale"] = scale;
