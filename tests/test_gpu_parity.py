@@ -2502,3 +2502,32 @@ def test_cache_written_between_forward_and_backward():
             kk.zero_(), vv.zero_()
         grads.append(torch.autograd.grad(out, leaf, do)[0])
     assert torch.equal(*grads)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [72, 96])  # between the kernels' widths, and the last size of the branch
+@pytest.mark.parametrize("n, n_kv", [(1, 40), (97, 97), (300, 1000), (1025, 1025), (64, 5000)])
+def test_head_sizes_up_to_96_leave_the_last_columns_out(n, n_kv, d, causal):
+    """The pipelined kernels of width 128 leave columns 96-127 out for head sizes up to
+    96: those hold zeros, so every tiling's results equal those on zero-padded tensors
+    of 128 columns bit for bit (remainders of tiles, split keys, unequal lengths)."""
+    q, k, v, do = (t.to(DEV) for t in make_inputs(1, 4, 2, n, d, seed=n + d, n_kv=n_kv))
+    wide = [torch.nn.functional.pad(t, (0, 128 - d)) for t in (q, k, v, do)]
+    scale = d ** -0.5
+    for fwd, dkdv, dq in [(6, 4, 4), (7, 4, 4), (8, 4, 4), (-1, -1, -1)]:
+        _note(f"used96 n={n} n_kv={n_kv} d={d} causal={causal} tilings {fwd} {dkdv} {dq}")
+        tilings = ((_lib.KERNEL_FWD, fwd), (_lib.KERNEL_DKDV, dkdv), (_lib.KERNEL_DQ, dq))
+        try:
+            for kernel, variant in tilings:
+                _lib.set_tiling(kernel, 128, causal, variant)
+            leaves = [t.clone().requires_grad_() for t in (q, k, v)]
+            out = scaled_dot_product_attention(*leaves, is_causal=causal, enable_gqa=True,
+                                               backend="triton")
+            got = (out.detach(), *torch.autograd.grad(out, leaves, do))
+            o, lse = _ops.flash_fwd(*wide[:3], causal, scale)
+            want = (o, *_ops.flash_bwd(*wide[:3], o, lse, wide[3], causal, scale))
+        finally:
+            for kernel, _ in tilings:
+                _lib.set_tiling(kernel, 128, causal, -1)
+        for name, a, b in zip(("o", "dq", "dk", "dv"), got, want):
+            assert torch.equal(a, b[..., :d]), (name, fwd)

@@ -489,6 +489,15 @@ void dkdv_pipe_kernel(BwdArgs a) {
   dkdv_pipe_body<D, CAUSAL, NW, E>(a, blockIdx.x, lds);
 }
 
+// The same at D = 128 for head sizes up to kUsed96.
+template <bool CAUSAL, int NW, class E>
+__global__ __launch_bounds__(64 * NW)
+__attribute__((amdgpu_waves_per_eu(DkdvPipeTile<128, NW>::WGS_PER_CU)))
+void dkdv_pipe_used96_kernel(BwdArgs a) {
+  __shared__ __attribute__((aligned(16))) half_t lds[DkdvPipeTile<128, NW>::LDS_HALVES];
+  dkdv_pipe_body<128, CAUSAL, NW, E, kUsed96>(a, blockIdx.x, lds);
+}
+
 template <int D, bool CAUSAL, int NW, class E = F16>
 hipError_t dkdv_pipe_launch(const BwdArgs& a, hipStream_t stream) {
   using T = DkdvPipeTile<D, NW>;
@@ -497,8 +506,10 @@ hipError_t dkdv_pipe_launch(const BwdArgs& a, hipStream_t stream) {
   if (b.nsplit < 1 || (b.nsplit > 1 && b.part == nullptr)) return hipErrorInvalidValue;
   const int64_t blocks = (int64_t)b.num_tiles * a.BHkv * b.nsplit;
   if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((dkdv_pipe_kernel<D, CAUSAL, NW, E>), dim3((unsigned)blocks), dim3(T::NT), 0,
-                     stream, b);
+  auto kernel = &dkdv_pipe_kernel<D, CAUSAL, NW, E>;
+  if constexpr (D == 128)
+    if (a.d <= kUsed96) kernel = &dkdv_pipe_used96_kernel<CAUSAL, NW, E>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(T::NT), 0, stream, b);
   return hipGetLastError();
 }
 
@@ -732,6 +743,16 @@ void dq_pipe_kernel(BwdArgs a) {
   dq_pipe_body<D, CAUSAL, NW, E, TAIL>(a, blockIdx.x, lds);
 }
 
+// The same at D = 128 for head sizes up to kUsed96.
+template <bool CAUSAL, int NW, class E, bool TAIL>
+__global__ __launch_bounds__(64 * NW)
+__attribute__((amdgpu_waves_per_eu(DqPipeTile<128, NW>::WGS_PER_CU)))
+void dq_pipe_used96_kernel(BwdArgs a) {
+  using T = DqPipeTile<128, NW>;
+  __shared__ __attribute__((aligned(16))) half_t lds[T::NSTAGE * T::STAGE];
+  dq_pipe_body<128, CAUSAL, NW, E, TAIL, kUsed96>(a, blockIdx.x, lds);
+}
+
 template <int D, bool CAUSAL, int NW, class E = F16>
 hipError_t dq_pipe_launch(const BwdArgs& a, hipStream_t stream) {
   using T = DqPipeTile<D, NW>;
@@ -742,12 +763,13 @@ hipError_t dq_pipe_launch(const BwdArgs& a, hipStream_t stream) {
     return hipErrorInvalidValue;
   const int64_t blocks = (int64_t)b.num_tiles * a.BH * b.nsplit;
   if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
-  if (dq_tail_free(b, CAUSAL))
-    hipLaunchKernelGGL((dq_pipe_kernel<D, CAUSAL, NW, E, false>), dim3((unsigned)blocks),
-                       dim3(T::NT), 0, stream, b);
-  else
-    hipLaunchKernelGGL((dq_pipe_kernel<D, CAUSAL, NW, E, true>), dim3((unsigned)blocks),
-                       dim3(T::NT), 0, stream, b);
+  const bool tail = !dq_tail_free(b, CAUSAL);
+  auto kernel = tail ? &dq_pipe_kernel<D, CAUSAL, NW, E, true> : &dq_pipe_kernel<D, CAUSAL, NW, E, false>;
+  if constexpr (D == 128)
+    if (a.d <= kUsed96)
+      kernel = tail ? &dq_pipe_used96_kernel<CAUSAL, NW, E, true>
+                    : &dq_pipe_used96_kernel<CAUSAL, NW, E, false>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(T::NT), 0, stream, b);
   return hipGetLastError();
 }
 

@@ -26,17 +26,17 @@ __device__ __forceinline__ void static_for(F&& f) {
 // dQ epilogue: lane (query qrow, half g) holds d = 32*db + 8*(j/4) + 4*g + j%4
 // of dQ / mul: 16-bit through rdq, or in split mode the fp32 partial of split
 // `split` (part[split][B*Hq][N][D]).
-template <int D, class E>
+template <int D, class E, int DU = D>
 __device__ __forceinline__ void store_dq(const BwdArgs& a, const rsrc_t& rdq, int split, int head,
-                                         int qrow, const float16v (&dq)[D / 32], float mul) {
+                                         int qrow, const float16v (&dq)[DU / 32], float mul) {
   const bool split_mode = a.nsplit > 1;
   // The lane's half, recomputed (mbcnt needs no live register).
   const int g = (int)(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) >> 5);
   const int64_t prow = ((int64_t)split * a.BH + head) * a.N + qrow;
   float* po = split_mode ? a.part + prow * D : nullptr;  // part is null in one-pass mode
-  with_cols<D>(a.d, [&](auto cols) {
+  with_cols<DU>(a.d, [&](auto cols) {
 #pragma unroll
-    for (int db = 0; db < D / 32; ++db)
+    for (int db = 0; db < DU / 32; ++db)
 #pragma unroll
       for (int jq = 0; jq < 4; ++jq) {
         float4v v;
@@ -161,7 +161,7 @@ constexpr int dkdv_task_q(int i) {
   return NQ - 2 + (p - 2 - 2 * (NQ - 2));
 }
 
-template <int D, bool CAUSAL, int NW, class E>
+template <int D, bool CAUSAL, int NW, class E, int DU = D>
 __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned block,
                                         half_t* __restrict__ lds) {
   using T = DkdvPipeTile<D, NW>;
@@ -256,10 +256,10 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
   // c K in fp32 rounded to fp16. With the S accumulator started from LSE',
   // the MFMA yields LSE' - s and P = exp2(-acc) needs no multiply-add.
   const float c = a.c;
-  half8 kf[D / 16], vn[D / 16];
-  with_cols<D>(a.d, [&](auto cols) {
+  half8 kf[DU / 16], vn[DU / 16];
+  with_cols<DU>(a.d, [&](auto cols) {
 #pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) {
+    for (int kk = 0; kk < DU / 16; ++kk) {
       const uint32_t off = elem_off(krow, a.kl.row, 16 * kk + 8 * g, cols);
       kf[kk] = __builtin_bit_cast(half8, buf_load_b128(rk, off));
       vn[kk] = neg8(__builtin_bit_cast(half8, buf_load_b128(rv, off)));
@@ -267,12 +267,12 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
   });
   wait_all_vm();
 #pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk)
+  for (int kk = 0; kk < DU / 16; ++kk)
 #pragma unroll
     for (int e = 0; e < 8; ++e) kf[kk][e] = to_elem<E>(-c * elem_to_f32<E>(kf[kk][e]));
   // Opaque from here on, so that the operands are not recomputed inside the loop.
 #pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk) asm volatile("" : "+v"(kf[kk]), "+v"(vn[kk]));
+  for (int kk = 0; kk < DU / 16; ++kk) asm volatile("" : "+v"(kf[kk]), "+v"(vn[kk]));
 
 #pragma unroll
   for (int u = 3; u < T::AHEAD; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
@@ -288,14 +288,14 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
   // Units 0, 1, 2 landed (3, 4 in flight), zeros and table written.
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(2 * IPU) : "memory");
 
-  int r_off[D / 16];  // row reads: row row_perm(ql), chunk 2*kk + g
+  int r_off[DU / 16];  // row reads: row row_perm(ql), chunk 2*kk + g
 #pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk) r_off[kk] = swz_offset<D>(row_perm(ql), 2 * kk + g);
-  int t_off[D / 32][2];  // transposed reads (see read_tr)
+  for (int kk = 0; kk < DU / 16; ++kk) r_off[kk] = swz_offset<D>(row_perm(ql), 2 * kk + g);
+  int t_off[DU / 32][2];  // transposed reads (see read_tr)
   {
     const int grp = lane >> 4, i = lane & 15, r = i >> 2, qq = i & 3;
 #pragma unroll
-    for (int db = 0; db < D / 32; ++db) {
+    for (int db = 0; db < DU / 32; ++db) {
       const int col = 32 * db + 16 * (grp & 1) + 4 * qq;
 #pragma unroll
       for (int h2 = 0; h2 < 2; ++h2) {
@@ -335,9 +335,9 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
     return r;
   };
 
-  float16v dk[D / 32], dv[D / 32];
+  float16v dk[DU / 32], dv[DU / 32];
 #pragma unroll
-  for (int db = 0; db < D / 32; ++db)
+  for (int db = 0; db < DU / 32; ++db)
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       dk[db][j] = 0.f;
@@ -360,7 +360,7 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
     dp_cur = table16(reinterpret_cast<const float*>(first + 2 * T::TILE) + 64 + 8 * g);
     s_cur = table16(fl + lse_table(s0, c_row));
 #pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) {
+    for (int kk = 0; kk < DU / 16; ++kk) {
       s_cur = mma<E>(*reinterpret_cast<const half8*>(first + r_off[kk]), kf[kk], s_cur);
       dp_cur = mma<E>(*reinterpret_cast<const half8*>(first + T::TILE + r_off[kk]), vn[kk], dp_cur);
     }
@@ -384,7 +384,7 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int db = 0; db < D / 32; ++db) {
+      for (int db = 0; db < DU / 32; ++db) {
         acc_mfma(dv[db], tr8(slot + T::TILE + 16 * h * D, db), pa_prev[h]);
         acc_mfma(dk[db], tr8(slot + 16 * h * D, db), sa_prev[h]);
       }
@@ -424,7 +424,7 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
     // adjacent tasks share an accumulator. Group i issues the LDS reads of
     // task i + kLead, runs task i and part of unit u's vector work; fences
     // keep the compiler from regrouping.
-    constexpr int NQ = D / 16;  // tasks of each kind
+    constexpr int NQ = DU / 16;  // tasks of each kind
     constexpr int NTASK = 4 * NQ;
     constexpr int kLead = FA_DKDV_LEAD;
     // Operand of task t of the body whose previous unit's rows are at p and
@@ -432,7 +432,7 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
     auto load_op_at = [&](auto t_c, const half_t* p, const half_t* n) -> half8 {
       constexpr int t = decltype(t_c)::value;
       constexpr int kind = dkdv_task_kind<NQ>(t), q = dkdv_task_q<NQ>(t);
-      constexpr int h = q / (D / 32), db = q % (D / 32);
+      constexpr int h = q / (DU / 32), db = q % (DU / 32);
       if constexpr (kind == 0) return tr8(p + T::TILE + 16 * h * D, db);
       else if constexpr (kind == 1) return tr8(p + 16 * h * D, db);
       else if constexpr (kind == 2) return *reinterpret_cast<const half8*>(n + r_off[q]);
@@ -445,7 +445,7 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
     auto run_task = [&](auto t_c, const half8& op) {
       constexpr int t = decltype(t_c)::value;
       constexpr int kind = dkdv_task_kind<NQ>(t), q = dkdv_task_q<NQ>(t);
-      constexpr int h = q / (D / 32), db = q % (D / 32);
+      constexpr int h = q / (DU / 32), db = q % (DU / 32);
       if constexpr (kind == 0) acc_mfma(dv[db], op, pa_prev[h]);
       else if constexpr (kind == 1) acc_mfma(dk[db], op, sa_prev[h]);
       else if constexpr (kind == 2) s_nx = mma<E>(op, kf[q], s_nx);
@@ -573,7 +573,7 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
     float* pv = pk + plane;
     if (krow < Nkv) {
 #pragma unroll
-      for (int db = 0; db < D / 32; ++db)
+      for (int db = 0; db < DU / 32; ++db)
 #pragma unroll
         for (int jq = 0; jq < 4; ++jq) {
           const int64_t e0 = (int64_t)krow * D + 32 * db + 8 * jq + 4 * g;
@@ -591,9 +591,9 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
   }
   const rsrc_t rdk = make_rsrc(a.dk + (int64_t)kvh * Nkv * a.d, (uint32_t)(Nkv * a.d) * 2u);
   const rsrc_t rdv = make_rsrc(a.dv + (int64_t)kvh * Nkv * a.d, (uint32_t)(Nkv * a.d) * 2u);
-  with_cols<D>(a.d, [&](auto cols) {
+  with_cols<DU>(a.d, [&](auto cols) {
 #pragma unroll
-    for (int db = 0; db < D / 32; ++db)
+    for (int db = 0; db < DU / 32; ++db)
 #pragma unroll
       for (int jq = 0; jq < 4; ++jq) {
         const uint32_t off = elem_off(krow, cols, 32 * db + 8 * jq + 4 * g, cols);
@@ -669,7 +669,7 @@ inline bool dq_tail_free(const BwdArgs& a, bool causal) {
 
 // TAIL: the launch may have units with keys past its range (see the body);
 // dq_tail_free() says when it cannot.
-template <int D, bool CAUSAL, int NW, class E, bool TAIL = true>
+template <int D, bool CAUSAL, int NW, class E, bool TAIL = true, int DU = D>
 __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned block,
                                         half_t* __restrict__ lds) {
   using T = DqPipeTile<D, NW>;
@@ -737,10 +737,10 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
   for (int u = 0; u < 3; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
   // -fp16(c Q) and -dO as B operands (column = query ql, d = 16*kk + 8*g .. +7).
   const float c = a.c;
-  half8 qf[D / 16], don[D / 16];
-  with_cols<D>(a.d, [&](auto cols) {
+  half8 qf[DU / 16], don[DU / 16];
+  with_cols<DU>(a.d, [&](auto cols) {
 #pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) {
+    for (int kk = 0; kk < DU / 16; ++kk) {
       const uint32_t off = elem_off(qrow, a.ql.row, 16 * kk + 8 * g, cols);
       qf[kk] = __builtin_bit_cast(half8, buf_load_b128(rq, off));
       don[kk] = neg8(__builtin_bit_cast(half8, buf_load_b128(rdo, off)));
@@ -753,9 +753,9 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
     // the two 8-wide halves of every 16-wide chunk of the row).
     const rsrc_t ro = make_rsrc(a.o + (int64_t)head * N * a.d, (uint32_t)(N * a.d) * 2u);
     float part = 0.f;
-    with_cols<D>(a.d, [&](auto cols) {
+    with_cols<DU>(a.d, [&](auto cols) {
 #pragma unroll
-      for (int kk = 0; kk < D / 16; ++kk) {
+      for (int kk = 0; kk < DU / 16; ++kk) {
         const half8 ov = __builtin_bit_cast(
             half8, buf_load_b128(ro, elem_off(qrow, cols, 16 * kk + 8 * g, cols)));
 #pragma unroll
@@ -770,11 +770,11 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
   }
   wait_all_vm();
 #pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk)
+  for (int kk = 0; kk < DU / 16; ++kk)
 #pragma unroll
     for (int e = 0; e < 8; ++e) qf[kk][e] = to_elem<E>(-c * elem_to_f32<E>(qf[kk][e]));
 #pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk) asm volatile("" : "+v"(qf[kk]), "+v"(don[kk]));
+  for (int kk = 0; kk < DU / 16; ++kk) asm volatile("" : "+v"(qf[kk]), "+v"(don[kk]));
 
 #pragma unroll
   for (int u = 3; u < T::AHEAD; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
@@ -812,14 +812,14 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
     return;
   }
 
-  int r_off[D / 16];  // row reads: row row_perm(ql), chunk 2*kk + g
+  int r_off[DU / 16];  // row reads: row row_perm(ql), chunk 2*kk + g
 #pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk) r_off[kk] = swz_offset<D>(row_perm(ql), 2 * kk + g);
-  int t_off[D / 32][2];  // transposed reads (see read_tr)
+  for (int kk = 0; kk < DU / 16; ++kk) r_off[kk] = swz_offset<D>(row_perm(ql), 2 * kk + g);
+  int t_off[DU / 32][2];  // transposed reads (see read_tr)
   {
     const int grp = lane >> 4, i = lane & 15, r = i >> 2, qq = i & 3;
 #pragma unroll
-    for (int db = 0; db < D / 32; ++db) {
+    for (int db = 0; db < DU / 32; ++db) {
       const int col = 32 * db + 16 * (grp & 1) + 4 * qq;
 #pragma unroll
       for (int h2 = 0; h2 < 2; ++h2) {
@@ -842,9 +842,9 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
     return v;
   };
 
-  float16v dq[D / 32];
+  float16v dq[DU / 32];
 #pragma unroll
-  for (int db = 0; db < D / 32; ++db)
+  for (int db = 0; db < DU / 32; ++db)
 #pragma unroll
     for (int j = 0; j < 16; ++j) dq[db][j] = 0.f;
 
@@ -859,7 +859,7 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
   // Pipeline registers: Sl^T, dPd^T of the current unit; dS'^T of the previous one.
   float16v s_cur = lse16, dp_cur = delta16;
 #pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk) {
+  for (int kk = 0; kk < DU / 16; ++kk) {
     s_cur = mma<E>(*reinterpret_cast<const half8*>(lds + s0 * T::STAGE + r_off[kk]), qf[kk], s_cur);
     dp_cur = mma<E>(*reinterpret_cast<const half8*>(lds + s0 * T::STAGE + T::TILE + r_off[kk]),
                     don[kk], dp_cur);
@@ -880,7 +880,7 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int db = 0; db < D / 32; ++db) acc_mfma(dq[db], tr8(slot + 16 * h * D, db), sa_prev[h]);
+      for (int db = 0; db < DU / 32; ++db) acc_mfma(dq[db], tr8(slot + 16 * h * D, db), sa_prev[h]);
   };
 
   int c_key = kv_lo;  // first key of the unit the body works on
@@ -933,7 +933,7 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
     // Hand-ordered body: 3 * D/16 MFMA tasks in the order dQ (unit u-1),
     // S^T, dPd^T (unit u+1), repeated; group i issues the LDS reads of task
     // i + kLead, runs task i and part of unit u's vector work.
-    constexpr int NQ = D / 16;
+    constexpr int NQ = DU / 16;
     constexpr int NTASK = 3 * NQ;
     constexpr int kLead = FA_DQ_LEAD;
     // Operand of task t of the body whose previous unit's rows are at p and
@@ -941,7 +941,7 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
     auto load_op_at = [&](auto t_c, const half_t* p, const half_t* n) -> half8 {
       constexpr int t = decltype(t_c)::value;
       constexpr int kind = t % 3, q = t / 3;
-      constexpr int h = q / (D / 32), db = q % (D / 32);
+      constexpr int h = q / (DU / 32), db = q % (DU / 32);
       if constexpr (kind == 0) return tr8(p + 16 * h * D, db);
       else if constexpr (kind == 1) return *reinterpret_cast<const half8*>(n + r_off[q]);
       else return *reinterpret_cast<const half8*>(n + T::TILE + r_off[q]);
@@ -951,7 +951,7 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
     auto run_task = [&](auto t_c, const half8& op) {
       constexpr int t = decltype(t_c)::value;
       constexpr int kind = t % 3, q = t / 3;
-      constexpr int h = q / (D / 32), db = q % (D / 32);
+      constexpr int h = q / (DU / 32), db = q % (DU / 32);
       if constexpr (kind == 0) acc_mfma(dq[db], op, sa_prev[h]);
       else if constexpr (kind == 1) s_nx = mma<E>(op, qf[q], s_nx);
       else dp_nx = mma<E>(op, don[q], dp_nx);
@@ -1031,7 +1031,7 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   const rsrc_t rdq = make_rsrc(a.dq + (int64_t)head * N * a.d, (uint32_t)(N * a.d) * 2u);
-  store_dq<D, E>(a, rdq, split, head, qrow, dq, -a.scale);  // accumulated -dS
+  store_dq<D, E, DU>(a, rdq, split, head, qrow, dq, -a.scale);  // accumulated -dS
 }
 
 }  // namespace fa

@@ -64,10 +64,10 @@ using ic = std::integral_constant<int, V>;
 //   split:   the fp32 partial O / lt and LSE of split `split` (a query that
 //            saw no key of the split, lt == 0, writes O = 0 and LSE = -inf,
 //            which the combine weighs with 0).
-template <int D, class E, bool SPLITS = true>
+template <int D, class E, bool SPLITS = true, int DU = D>
 __device__ __forceinline__ void store_fwd_output(const FwdArgs& a, const rsrc_t& ro, int split,
                                                  int head, int qrow, int g,
-                                                 const float16v (&o)[D / 32], float m, float lt) {
+                                                 const float16v (&o)[DU / 32], float m, float lt) {
   const bool split_mode = SPLITS && a.nsplit > 1;
   const bool seen = lt > 0.f;
   const float inv = seen ? 1.0f / lt : 0.f;
@@ -77,9 +77,9 @@ __device__ __forceinline__ void store_fwd_output(const FwdArgs& a, const rsrc_t&
   const int64_t prow = ((int64_t)split * a.BH + head) * a.N + qrow;
   float* po = split_mode ? a.part + prow * D : nullptr;  // part is null in one-pass mode
   const bool row_ok = qrow < a.N;
-  with_cols<D>(a.d, [&](auto cols) {
+  with_cols<DU>(a.d, [&](auto cols) {
 #pragma unroll
-    for (int db = 0; db < D / 32; ++db)
+    for (int db = 0; db < DU / 32; ++db)
 #pragma unroll
       for (int jq = 0; jq < 4; ++jq) {
         float4v v;
@@ -462,7 +462,8 @@ __device__ __forceinline__ void static_for_fwd_issue(F&& f) {
 // One job of the pipelined forward: query tile `qtile` of head block
 // `head_blk` (the work-group's P = a.pack query heads), keys of split `split`.
 // lds_all: the work-group's KG * NSTAGE * STAGE halves of LDS.
-template <int D, bool CAUSAL, int NW, int UPS, class E, int KG>
+// DU: the columns it works on, a multiple of 32 that holds the head size (kUsed96).
+template <int D, bool CAUSAL, int NW, int UPS, class E, int KG, int DU = D>
 __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int qtile,
                                               int head_blk, half_t* lds_all) {
   using T = FwdPipeTile<D, NW, UPS, KG>;
@@ -532,10 +533,10 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
   // in flight over the first barrier follow the wait.
 #pragma unroll
   for (int u = 0; u < T::AHEAD - T::IN_FLIGHT; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
-  half8 qf[D / 16];
-  with_cols<D>(a.d, [&](auto cols) {
+  half8 qf[DU / 16];
+  with_cols<DU>(a.d, [&](auto cols) {
 #pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk)
+    for (int kk = 0; kk < DU / 16; ++kk)
       qf[kk] = __builtin_bit_cast(
           half8, buf_load_b128(rq, elem_off(qrow, a.ql.row, 16 * kk + 8 * g, cols)));
   });
@@ -558,14 +559,14 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
   // All but the last IN_FLIGHT units landed, zeros written.
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(T::IN_FLIGHT * IPU) : "memory");
 
-  int k_off[D / 16];  // row reads of K: row row_perm(ql), chunk 2*kk + g
+  int k_off[DU / 16];  // row reads of K: row row_perm(ql), chunk 2*kk + g
 #pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk) k_off[kk] = swz_offset<D>(row_perm(ql), 2 * kk + g);
-  int v_off[D / 32][2];  // transposed reads of V (see read_tr)
+  for (int kk = 0; kk < DU / 16; ++kk) k_off[kk] = swz_offset<D>(row_perm(ql), 2 * kk + g);
+  int v_off[DU / 32][2];  // transposed reads of V (see read_tr)
   {
     const int grp = lane >> 4, i = lane & 15, r = i >> 2, qq = i & 3;
 #pragma unroll
-    for (int db = 0; db < D / 32; ++db) {
+    for (int db = 0; db < DU / 32; ++db) {
       const int col = 32 * db + 16 * (grp & 1) + 4 * qq;
 #pragma unroll
       for (int h2 = 0; h2 < 2; ++h2) {
@@ -588,9 +589,9 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
     return v;
   };
 
-  float16v o[D / 32];
+  float16v o[DU / 32];
 #pragma unroll
-  for (int db = 0; db < D / 32; ++db)
+  for (int db = 0; db < DU / 32; ++db)
 #pragma unroll
     for (int j = 0; j < 16; ++j) o[db][j] = 0.f;
   float m = -INFINITY;  // reference max (scaled, log2 units); may lag the true max by <= 8
@@ -603,7 +604,7 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
 #pragma unroll
   for (int j = 0; j < 16; ++j) s_cur[j] = 0.f;
 #pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk)
+  for (int kk = 0; kk < DU / 16; ++kk)
     s_cur = mma<E>(*reinterpret_cast<const half8*>(lds + s0 * T::STAGE + k_off[kk]), qf[kk], s_cur);
   half8 pa_prev[2];
 #pragma unroll
@@ -615,7 +616,7 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int db = 0; db < D / 32; ++db)
+      for (int db = 0; db < DU / 32; ++db)
         o[db] = mma<E>(tr8(slot + T::TILE + 16 * h * D, db), pa_prev[h], o[db]);
   };
 
@@ -643,13 +644,13 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
     // Hand-ordered body: D/16 S tasks (unit u+1) and D/16 O tasks (unit
     // u-1), alternating; group i issues the LDS reads of task i + kLead,
     // runs task i and part of unit u's vector work; fences keep the order.
-    constexpr int NQ = D / 16;
+    constexpr int NQ = DU / 16;
     constexpr int NTASK = 2 * NQ;
     constexpr int kLead = FA_FWD_LEAD;
     auto load_op = [&](auto t_c) -> half8 {
       constexpr int t = decltype(t_c)::value;
       constexpr int q = t / 2;
-      constexpr int h = q / (D / 32), db = q % (D / 32);
+      constexpr int h = q / (DU / 32), db = q % (DU / 32);
       if constexpr (t % 2 == 0) return *reinterpret_cast<const half8*>(nxt + k_off[q]);
       else return tr8(prv + T::TILE + 16 * h * D, db);
     };
@@ -659,7 +660,7 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
     auto run_task = [&](auto t_c, const half8& op) {
       constexpr int t = decltype(t_c)::value;
       constexpr int q = t / 2;
-      constexpr int h = q / (D / 32), db = q % (D / 32);
+      constexpr int h = q / (DU / 32), db = q % (DU / 32);
       if constexpr (t % 2 == 0) s_nx = mma<E>(op, qf[q], s_nx);
       else o[db] = mma<E>(op, pa_prev[h], o[db]);
     };
@@ -743,7 +744,7 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
       const float alpha = exp2_fast(m - m_new);
       l *= alpha;
 #pragma unroll
-      for (int db = 0; db < D / 32; ++db) o[db] *= alpha;
+      for (int db = 0; db < DU / 32; ++db) o[db] *= alpha;
       m = m_new;
       l_u = 0.f;
 #pragma unroll
@@ -788,12 +789,12 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
   if constexpr (KG == 2) {
     // Group 1 hands its O, m and l (per lane) to the group-0 wave serving the
     // same queries through LDS (the rings are drained), [wave][value][lane].
-    constexpr int F = D / 32 * 16 + 2;
+    constexpr int F = DU / 32 * 16 + 2;
     __syncthreads();
     float* const xs = reinterpret_cast<float*>(lds_all) + wave * F * 64 + lane;
     if (gk == 1) {
 #pragma unroll
-      for (int db = 0; db < D / 32; ++db)
+      for (int db = 0; db < DU / 32; ++db)
 #pragma unroll
         for (int j = 0; j < 16; ++j) xs[(16 * db + j) * 64] = o[db][j];
       xs[(F - 2) * 64] = m;
@@ -809,7 +810,7 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
     const float w0 = m == -inf ? 0.f : exp2_fast(m - mt);
     const float w1 = m1 == -inf ? 0.f : exp2_fast(m1 - mt);
 #pragma unroll
-    for (int db = 0; db < D / 32; ++db)
+    for (int db = 0; db < DU / 32; ++db)
 #pragma unroll
       for (int j = 0; j < 16; ++j) o[db][j] = o[db][j] * w0 + xs[(16 * db + j) * 64] * w1;
     l = l * w0 + l1 * w1;
@@ -818,7 +819,7 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
 
   // Epilogue: lane (query qrow, half g) holds d = 32*db + 8*(j/4) + 4*g + j%4.
   const float lt = halves_sum(l);
-  store_fwd_output<D, E>(a, ro, split, head, qrow, g, o, m, lt);
+  store_fwd_output<D, E, true, DU>(a, ro, split, head, qrow, g, o, m, lt);
 }
 
 // --------------------------------------------------------------------------
@@ -1238,18 +1239,33 @@ __device__ __forceinline__ void fwd_pipe16_body(const FwdArgs& a, int split, int
 
 // The grid form: one job per work-group, tile-major / head-minor (heaviest
 // causal tiles first), the split index slowest.
+template <int D, bool CAUSAL, int NW, int UPS, class E, int KG, int DU = D>
+__device__ __forceinline__ void fwd_pipe_grid(const FwdArgs& a, half_t* lds_all) {
+  const int row_wgs = a.BH / a.pack;  // work-groups per tile row
+  const int split = blockIdx.x / (a.num_tiles * row_wgs);
+  const TileHead th = decode_block_grouped(blockIdx.x - split * a.num_tiles * row_wgs, row_wgs,
+                                           a.group / a.pack);
+  const int qtile = CAUSAL ? (a.num_tiles - 1 - th.tile_rank) : th.tile_rank;
+  fwd_pipe_body<D, CAUSAL, NW, UPS, E, KG, DU>(a, split, qtile, th.head, lds_all);
+}
+
 template <int D, bool CAUSAL, int NW, int UPS, class E = F16, int KG = 1>
 __global__ __launch_bounds__(64 * NW)
 __attribute__((amdgpu_waves_per_eu(FwdPipeTile<D, NW, UPS, KG>::WAVES_PER_SIMD)))
 void fwd_pipe_kernel(FwdArgs a) {
   using T = FwdPipeTile<D, NW, UPS, KG>;
   __shared__ __attribute__((aligned(16))) half_t lds_all[KG * T::NSTAGE * T::STAGE];
-  const int row_wgs = a.BH / a.pack;  // work-groups per tile row
-  const int split = blockIdx.x / (a.num_tiles * row_wgs);
-  const TileHead th = decode_block_grouped(blockIdx.x - split * a.num_tiles * row_wgs, row_wgs,
-                                           a.group / a.pack);
-  const int qtile = CAUSAL ? (a.num_tiles - 1 - th.tile_rank) : th.tile_rank;
-  fwd_pipe_body<D, CAUSAL, NW, UPS, E, KG>(a, split, qtile, th.head, lds_all);
+  fwd_pipe_grid<D, CAUSAL, NW, UPS, E, KG>(a, lds_all);
+}
+
+// The same at D = 128 for head sizes up to kUsed96.
+template <bool CAUSAL, int NW, class E, int KG>
+__global__ __launch_bounds__(64 * NW)
+__attribute__((amdgpu_waves_per_eu(FwdPipeTile<128, NW, 1, KG>::WAVES_PER_SIMD)))
+void fwd_pipe_used96_kernel(FwdArgs a) {
+  using T = FwdPipeTile<128, NW, 1, KG>;
+  __shared__ __attribute__((aligned(16))) half_t lds_all[KG * T::NSTAGE * T::STAGE];
+  fwd_pipe_grid<128, CAUSAL, NW, 1, E, KG, kUsed96>(a, lds_all);
 }
 
 // The persistent form (causal, one pass, one head per work-group): one
@@ -1332,8 +1348,10 @@ hipError_t fwd_pipe_launch(const FwdArgs& a, hipStream_t stream) {
     return hipErrorInvalidValue;
   const int64_t blocks = (int64_t)b.num_tiles * (a.BH / b.pack) * b.nsplit;
   if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((fwd_pipe_kernel<D, CAUSAL, NW, UPS, E, KG>), dim3((unsigned)blocks),
-                     dim3(T::NT), 0, stream, b);
+  auto kernel = &fwd_pipe_kernel<D, CAUSAL, NW, UPS, E, KG>;
+  if constexpr (D == 128)
+    if (a.d <= kUsed96) kernel = &fwd_pipe_used96_kernel<CAUSAL, NW, E, KG>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(T::NT), 0, stream, b);
   return hipGetLastError();
 }
 

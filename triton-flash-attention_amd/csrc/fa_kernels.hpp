@@ -229,6 +229,14 @@ hipError_t launch_split_sum(const float* part, half_t* out, int64_t rows, int D,
 constexpr int kDecodeRows = 16;
 hipError_t launch_fwd_decode(const FwdArgs& a, int D, int dtype, hipStream_t stream);
 
+// Columns that the pipelined bodies of width 128 work on where the head size is at
+// most that: the last 32, which hold zeros, take no MFMAs, LDS reads or accumulators
+// (a quarter of each; the LDS layout and the DMA stay those of 128). The results are
+// the same bit for bit. MI355X, B4 H16 N1025 D80 bf16 bidirectional, a training step:
+// 234.9 -> 201.5 us. Between 97 and 128 all four 32-column blocks hold columns; a
+// 64-wide call has no whole block to leave out between 33 and 64.
+constexpr int kUsed96 = 96;
+
 // Merge of the forward's nsplit partials (FwdArgs::part) into O (16-bit) and
 // base-2 LSE, rows = B * Hq * N: O = sum_s w_s O_s / sum_s w_s with
 // w_s = exp2(lse_s - max_s lse_s), LSE = max + log2(sum_s w_s).

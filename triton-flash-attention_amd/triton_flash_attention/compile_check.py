@@ -53,6 +53,12 @@ def _defaults() -> tuple[str, ...]:
                       f"fa::fwd_pipe_kernel<128, {c}, 8, 1, {e}, 1>", f"fa::fwd_kernel<128, {c}, 4, 32, {e}>",
                       f"fa::fwd_pipe_kernel<128, {c}, 4, 1, {e}, 1>",
                       f"fa::fwd_pipe_kernel<128, {c}, 8, 1, {e}, 2>",
+                      f"fa::fwd_pipe_used96_kernel<{c}, 4, {e}, 1>",
+                      f"fa::fwd_pipe_used96_kernel<{c}, 8, {e}, 1>",
+                      f"fa::fwd_pipe_used96_kernel<{c}, 8, {e}, 2>",
+                      f"fa::dkdv_pipe_used96_kernel<{c}, 4, {e}>",
+                      f"fa::dq_pipe_used96_kernel<{c}, 4, {e}, true>",
+                      f"fa::dq_pipe_used96_kernel<{c}, 4, {e}, false>",
                       f"fa::dkdv_pipe_kernel<32, {c}, 4, {e}>", f"fa::dkdv_pipe_kernel<64, {c}, 4, {e}>",
                       f"fa::dkdv_pipe_kernel<128, {c}, 4, {e}>", f"fa::dkdv_pipe16_kernel<64, {c}, 4, {e}>",
                       f"fa::dkdv_pipe16_kernel<32, false, 4, {e}>",
