@@ -62,7 +62,7 @@ import torch
 
 from . import _lib, _native, _ops
 
-_SUPPORTED_HEAD_DIMS = (32, 64, 128)  # the kernels' widths; smaller sizes are zero-padded
+_SUPPORTED_HEAD_DIMS = (32, 64, 128)  # the kernels' widths; other sizes run at the next
 _SUPPORTED_DTYPES = (torch.float16, torch.bfloat16)
 _SUPPORTED_ARCH = "gfx950"
 Backend = Literal["auto", "triton", "torch"]
@@ -461,7 +461,9 @@ def scaled_dot_product_attention(
     The custom gfx950 path supports forward/backward, causal and bidirectional
     attention, arbitrary positive sequence lengths, GQA and any finite scale,
     for float16 or bfloat16 self- or cross-attention with head_dim and value
-    head_dim up to 128 (32, 64 and 128 natively, other sizes zero-padded).
+    head_dim up to 128 (32, 64 and 128 natively, other sizes at the next width).
+    Strided inputs are read as they stand where they can be; one that takes a
+    gradient is saved for the backward as it is and must not be written before.
     Other inputs fall back to PyTorch when ``backend="auto"``;
     ``backend="triton"`` requires the custom kernel and raises RuntimeError
     otherwise; ``backend="torch"`` always uses PyTorch SDPA.
