@@ -2485,6 +2485,51 @@ def test_decoding_weighs_keys_that_score_minus_infinity_with_zero(d, n_kv):
     assert_close("decode -inf keys", o[1, :4].numpy(), ref[1, :4].numpy())
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [32, 64, 96, 128])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+def test_forward_weighs_keys_that_score_minus_infinity_with_zero(dtype, d, causal):
+    """The same for every forward tiling, and for the library's own choice: infinite keys
+    in the first unit or tile of the loop, in the first one of a key group's or of a key
+    range's half, over many of them, and scattered. A row whose keys all score -inf is
+    NaN, as softmax has it. Against 64-bit softmax at the rounding of P and O (2^-9 each
+    in bf16, 2^-12 in fp16), for 700 queries in one pass and 64 against split keys."""
+    scale = d ** -0.5
+    for n, n_kv in ((700, 1500), (64, 8192)):
+        q, k, v, _ = make_inputs(1, 4, 2, n, d, seed=78 + d + n, n_kv=n_kv, dtype=dtype)
+        q[..., 0] = q[..., 0].abs() + 0.5
+        half = (n_kv // 2 + 31) // 32 * 32
+        k[0, 0, half - 64:half + 96, 0] = -math.inf
+        k[0, 1, :n_kv - 100, 0] = -math.inf
+        k[0, 1, n_kv - 40, 0] = -math.inf
+        if causal:  # rows that see finite keys only, -inf keys only, and both
+            k[0, 0, 0:40, 0] = -math.inf
+            k[0, 1, :, 0] = 0.25
+            k[0, 1, 32:160, 0] = -math.inf
+        kd, vd = (t.double().repeat_interleave(2, dim=1) for t in (k, v))
+        s = (q.double() @ kd.transpose(2, 3).contiguous()) * scale
+        if causal:
+            s.masked_fill_(torch.ones(n, n_kv, dtype=torch.bool).triu(1), -math.inf)
+        ref = torch.softmax(s, dim=-1) @ vd
+        nan = ref.isnan()
+        assert bool(nan.any()) == causal and not bool(nan.all())
+        wide = d if d in (32, 64, 128) else 128
+        tilings = [t["variant"] for t in _lib.tiling_variants(_lib.KERNEL_FWD, wide, causal)]
+        for variant in (-1, *tilings):
+            _note(f"-inf keys {dtype} n={n} d={d} causal={causal} tiling {variant}")
+            _lib.set_tiling(_lib.KERNEL_FWD, wide, causal, variant)
+            try:
+                with torch.no_grad():
+                    o = scaled_dot_product_attention(q.to(DEV), k.to(DEV), v.to(DEV),
+                                                     is_causal=causal, enable_gqa=True,
+                                                     backend="triton").cpu().double()
+            finally:
+                _lib.set_tiling(_lib.KERNEL_FWD, wide, causal, -1)
+            assert torch.equal(o.isnan(), nan), variant
+            rel = float((o - ref)[~nan].norm() / ref[~nan].norm())
+            assert rel <= (2 ** -8 if dtype == torch.bfloat16 else 2 ** -11), (variant, rel)
+
+
 def test_cache_written_between_forward_and_backward():
     """Part of a cache that takes no gradient may be written again before the backward,
     which still sees the keys and values of its forward: the gradient of q is the one of

@@ -196,6 +196,10 @@ __device__ __forceinline__ int quad16(int G) {
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// What a row's exponentials are taken against for the reference max m: m, or 0 while
+// no finite score was seen (-inf - -inf is NaN; against 0 those scores give 0).
+__device__ __forceinline__ float exp_reference(float m) { return m == -INFINITY ? 0.f : m; }
 __device__ __forceinline__ float log2_fast(float x) { return __builtin_amdgcn_logf(x); }
 
 // Value of the same register in lane (l ^ 32).

@@ -51,7 +51,9 @@ struct FwdTile {
 // (exact in fp16 and fp32) and nothing else is done. Otherwise (and on the
 // first tile, where m = -inf gives inf / NaN sums) a rare branch computes the
 // tile max, moves m to it, rescales O and l, and recomputes P. The max is
-// thus only reduced when it is needed.
+// thus only reduced when it is needed. While every key of a row has scored -inf
+// (infinite inputs) m stays there and P is taken against 0 (exp_reference), so
+// such keys weigh 0 wherever they lie.
 constexpr float kSumLimit = 256.0f;
 
 template <int V>
@@ -60,7 +62,7 @@ using ic = std::integral_constant<int, V>;
 // Epilogue, lane (query qrow, half g) holding d = 32*db + 8*(j/4) + 4*g + j%4
 // of O (unnormalised), the reference max m and the row sum lt:
 //   unsplit: O / lt as 16-bit through the range-checked resource ro, and the
-//            base-2 LSE m + log2(lt);
+//            base-2 LSE m + log2(lt) (a row whose scores are all -inf: 0 / 0);
 //   split:   the fp32 partial O / lt and LSE of split `split` (a query that
 //            saw no key of the split, lt == 0, writes O = 0 and LSE = -inf,
 //            which the combine weighs with 0).
@@ -70,7 +72,7 @@ __device__ __forceinline__ void store_fwd_output(const FwdArgs& a, const rsrc_t&
                                                  const float16v (&o)[DU / 32], float m, float lt) {
   const bool split_mode = SPLITS && a.nsplit > 1;
   const bool seen = lt > 0.f;
-  const float inv = seen ? 1.0f / lt : 0.f;
+  const float inv = seen || !split_mode ? 1.0f / lt : 0.f;
   // The lane's half is recomputed here (mbcnt needs no live register), so
   // no lane value has to stay live, and spill, across the main loop.
   g = (int)(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) >> 5);
@@ -281,21 +283,20 @@ __global__ __launch_bounds__(64 * NW) void fwd_kernel(FwdArgs a) {
           }
       }
       half8 pk[KB][2];
-      // P against the current reference max, and this lane's row sum.
-      auto probs = [&](const float16v* s) {
-        const float nm = -m;
+      // P against the reference max `ref`, and this lane's row sum.
+      auto probs = [&](const float16v* s, float ref) {
         float ls4[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
           for (int j = 0; j < 16; ++j) {
-            const float p = exp2_fast(fmaf(s[kb][j], c, nm));
+            const float p = exp2_fast(fmaf(s[kb][j], c, -ref));
             ls4[j & 3] += p;
             pk[kb][j >> 3][j & 7] = to_elem<E>(p);
           }
         return (ls4[0] + ls4[1]) + (ls4[2] + ls4[3]);
       };
-      float lt = probs(sc);
+      float lt = probs(sc, m);
       if (__builtin_amdgcn_ballot_w64(!(lt <= kSumLimit)) != 0) {
         // Rare: the scores are rebuilt from the K tile (still in this slot)
         // rather than kept alive across the common path.
@@ -321,12 +322,13 @@ __global__ __launch_bounds__(64 * NW) void fwd_kernel(FwdArgs a) {
           }
         mx = halves_max(mx) * c;
         const float m_new = fmaxf(m, mx);
-        const float alpha = exp2_fast(m - m_new);
+        const float ref = exp_reference(m_new);
+        const float alpha = exp2_fast(m - ref);
         l *= alpha;
 #pragma unroll
         for (int db = 0; db < D / 32; ++db) o[db] *= alpha;
         m = m_new;
-        lt = probs(s2);
+        lt = probs(s2, ref);
       }
       l += lt;
       // O^T += V^T P^T
@@ -741,7 +743,8 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
       for (int j = 1; j < 16; ++j) mt = __builtin_fmaxf(mt, s_cur[j]);
       mt = halves_max(mt) * c;
       const float m_new = __builtin_fmaxf(m, mt);
-      const float alpha = exp2_fast(m - m_new);
+      const float ref = exp_reference(m_new);
+      const float alpha = exp2_fast(m - ref);
       l *= alpha;
 #pragma unroll
       for (int db = 0; db < DU / 32; ++db) o[db] *= alpha;
@@ -749,7 +752,7 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
       l_u = 0.f;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        const float p = exp2_fast(fmaf(s_cur[j], c, -m));
+        const float p = exp2_fast(fmaf(s_cur[j], c, -ref));
         l_u += p;
         pa[j >> 3][j & 7] = to_elem<E>(p);
       }
@@ -1152,7 +1155,8 @@ __device__ __forceinline__ void fwd_pipe16_body(const FwdArgs& a, int split, int
           for (int j = 0; j < 4; ++j) mt = __builtin_fmaxf(mt, s_cur[kb][qb][j]);
         mt = quarters_max(mt) * c;
         const float m_new = __builtin_fmaxf(m[qb], mt);
-        const float alpha = exp2_fast(m[qb] - m_new);
+        const float ref = exp_reference(m_new);
+        const float alpha = exp2_fast(m[qb] - ref);
         l[qb] *= alpha;
 #pragma unroll
         for (int dd = 0; dd < DD; ++dd) o[dd][qb] *= alpha;
@@ -1162,7 +1166,7 @@ __device__ __forceinline__ void fwd_pipe16_body(const FwdArgs& a, int split, int
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const float p = exp2_fast(fmaf(s_cur[kb][qb][j], c, -m[qb]));
+            const float p = exp2_fast(fmaf(s_cur[kb][qb][j], c, -ref));
             l_u[qb] += p;
             pa[qb][4 * kb + j] = to_elem<E>(p);
           }
@@ -1210,7 +1214,7 @@ __device__ __forceinline__ void fwd_pipe16_body(const FwdArgs& a, int split, int
   for (int qb = 0; qb < QB; ++qb) {
     const float lt = quarters_sum(l[qb]);
     const bool seen = lt > 0.f;
-    const float inv = seen ? 1.0f / lt : 0.f;
+    const float inv = seen || !split_mode ? 1.0f / lt : 0.f;
     const int qrow = qrow0 + 16 * qb;
     const bool row_ok = qrow < N;
     const int64_t prow = ((int64_t)split * a.BH + head) * N + qrow;

@@ -188,9 +188,7 @@ __global__ __launch_bounds__(256) void fwd_decode_kernel(FwdArgs a) {
         for (int j = 0; j < 4; ++j) mt = __builtin_fmaxf(mt, s[kb][j]);
       mt = quarters_max(mt) * c;
       const float m_new = __builtin_fmaxf(m, mt);
-      // While every key of the wave has scored -inf (infinite inputs) m stays there
-      // and the probabilities are zeros.
-      const float ref = m_new == -INFINITY ? 0.f : m_new;
+      const float ref = exp_reference(m_new);
       const float alpha = exp2_fast(m - ref);
       l *= alpha;
 #pragma unroll
