@@ -147,6 +147,22 @@ def test_validation_order_and_messages() -> None:
         explain_dispatch(q, torch.randn(1, 3, 6, 32), torch.randn(1, 3, 6, 32), enable_gqa=True)
 
 
+def test_fallback_compiles_as_one_graph_with_the_binding_loaded() -> None:
+    """A call that falls back to torch can be traced whole by torch.compile, also once
+    the native binding (which torch.compile cannot trace) has been loaded."""
+    from triton_flash_attention import _native
+
+    if not _native.available():
+        pytest.skip(_native.status()[1])
+    q = torch.randn(1, 2, 8, 64)
+
+    def f(x):
+        return 2.0 * scaled_dot_product_attention(x, x, x, is_causal=True)
+
+    torch._dynamo.reset()
+    torch.testing.assert_close(torch.compile(f, fullgraph=True, backend="eager")(q), f(q))
+
+
 def test_exports_match_reference_surface() -> None:
     import triton_flash_attention as pkg
 

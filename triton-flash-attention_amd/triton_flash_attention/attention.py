@@ -468,9 +468,10 @@ def scaled_dot_product_attention(
     ``backend="triton"`` requires the custom kernel and raises RuntimeError
     otherwise; ``backend="torch"`` always uses PyTorch SDPA.
     """
-    if backend == "auto" or backend == "triton":
+    if (backend == "auto" or backend == "triton") and not torch.compiler.is_dynamo_compiling():
         # A plain call: one native check in place of the ones below, which word the
-        # errors and choose among the other paths.
+        # errors and choose among the other paths. (torch.compile cannot trace into it,
+        # and traces the Python checks of a call that falls back to torch.)
         plain = _native.plain_scale(query, key, value, is_causal, scale, enable_gqa)
         if (plain and _device_arch(query.device).startswith(_SUPPORTED_ARCH)
                 and (_native_serves(query, value, plain) or _native_narrow(query, value, plain))):
