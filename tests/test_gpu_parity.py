@@ -2549,6 +2549,68 @@ def test_cache_written_between_forward_and_backward():
     assert torch.equal(*grads)
 
 
+@pytest.mark.parametrize("layout, d", [("tokens", 64), ("fused", 128), ("cache", 32), ("wide", 64),
+                                       ("columns", 64), ("shifted", 64), ("heads", 80),
+                                       ("tokens", 80), ("cache", 8)])
+@pytest.mark.parametrize("through", ["in place", "data"])
+def test_inputs_written_between_forward_and_backward(layout, d, through):
+    """Strided inputs and head sizes below a kernel's width may be written before the
+    backward also where they take gradients, in place or through .data: the gradients
+    are those of the values the forward saw, bit for bit. (A contiguous input at a
+    kernel's width is saved as it stands, and autograd raises for a write in place.)"""
+    q, k, v, do = (t.to(DEV) for t in make_inputs(2, 4, 2, 65, d, seed=92 + d, n_kv=130))
+    grads = []
+    for written in (False, True):
+        leaves = [_laid_out(t, layout).requires_grad_() for t in (q, k, v)]
+        out = scaled_dot_product_attention(*leaves, is_causal=True, enable_gqa=True,
+                                           backend="triton")
+        if written:
+            with torch.no_grad():
+                for t in leaves:
+                    (t if through == "in place" else t.data).fill_(7.0)
+        grads.append(torch.autograd.grad(out, leaves, _laid_out(do, layout)))
+    for a, b in zip(*grads):
+        assert torch.equal(a, b)
+
+
+def test_strided_inputs_are_copied_once_at_most():
+    """Allocations of a call: without gradients strided inputs are read as they stand (O
+    and LSE only); with gradients each is copied once, in its own order, so that a dO
+    laid out as the projections is read as it stands in the backward (Delta, dQ, dK, dV,
+    workspace only), slices of a fused projection included."""
+    def allocations(f):
+        torch.cuda.synchronize()
+        count = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]
+        before, result = count(), f()
+        return count() - before, result
+
+    B, H, N, D = 2, 4, 256, 64   # one-pass forward, split or combined backward
+    base = [t.to(DEV) for t in make_inputs(B, H, H, N, D, seed=17)]
+    for layout in ("tokens", "fused", "cache"):
+        q, k, v = (_laid_out(t, layout) for t in base[:3])
+        do = _laid_out(base[3], "cache" if layout == "cache" else "tokens")
+        run = lambda *t: scaled_dot_product_attention(*t, backend="triton")
+        with torch.no_grad():
+            run(q, k, v)
+            assert allocations(lambda: run(q, k, v))[0] == 2, layout
+        leaves = [t.detach().requires_grad_() for t in (q, k, v)]
+        made, out = allocations(lambda: run(*leaves))
+        assert made == 5, layout
+        workspace = int(_lib.load().fa_bwd_workspace_bytes(B, H, H, N, N, D, 0) > 0)
+        copies = int(layout == "cache")  # a part of a cache: q is dense, its dO is not
+        made, _ = allocations(lambda: torch.autograd.grad(out, leaves, do))
+        assert made == 4 + workspace + copies, layout
+
+
+def test_contiguous_input_written_before_the_backward_raises():
+    leaf = torch.randn(1, 2, 64, 64, device=DEV, dtype=torch.float16, requires_grad=True)
+    out = scaled_dot_product_attention(leaf, leaf, leaf, backend="triton")
+    with torch.no_grad():
+        leaf.zero_()
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.sum().backward()
+
+
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("d", [72, 96])  # between the kernels' widths, and the last size of the branch
 @pytest.mark.parametrize("n, n_kv", [(1, 40), (97, 97), (300, 1000), (1025, 1025), (64, 5000)])

@@ -15,11 +15,14 @@
 // scales, other head sizes, forward-mode AD).
 //
 // The kernels read strided q, k, v and dO and head sizes below their width as
-// they stand. A model's transposed projections, slices of a fused projection
-// and the filled part of a key/value cache are thus passed on without a copy
-// (B1 Hq32 Hkv8 N3001 D128: the three copies took 34 us beside an 82 us forward;
+// they stand. Without gradients a model's transposed projections, slices of a fused
+// projection and the filled part of a key/value cache are thus passed on without a
+// copy (B1 Hq32 Hkv8 N3001 D128: the three copies took 34 us beside an 82 us forward;
 // one query against a 3001-token part of a cache, 16 beside 23). operand() says
-// which tensors qualify; the others are copied.
+// which tensors qualify; the others are copied, as are k and v where their layouts
+// differ (pair_up). With gradients q, k and v are copied once unless they are
+// contiguous at a kernel's width (kept()), and dO is read as it stands where its
+// layout is that of the q kept.
 //
 // The library's entry points come from the copy Python has already loaded
 // (init() takes their addresses), so one libfa_gfx950.so serves both paths.
@@ -128,6 +131,20 @@ void pair_up(Operand& a, Operand& b) {
   b = as_operand(aligned(b.t));
 }
 
+// An input of a call with gradients, as it is saved for the backward: a contiguous one
+// at a kernel width as it stands (a write before the backward then raises autograd's
+// version error), any other one copied, so that the program may write its buffer (a
+// fused projection, part of a key/value cache) before the backward. The copy is dense
+// and keeps the order of the strides, so that q's copy pairs up with a dO of the same
+// layout (a training step of B2 Hq32 Hkv8 N2048 D128 bf16 on projection views: 425 us;
+// with the views themselves saved 401, with contiguous copies of all four 456).
+at::Tensor kept(const at::Tensor& t) {
+  const int64_t d = t.size(-1);
+  if (t.is_contiguous() && (d == 32 || d == 64 || d == 128)) return t;
+  return t.stride(-1) == 1 ? t.clone(at::MemoryFormat::Preserve)
+                          : t.clone(at::MemoryFormat::Contiguous);
+}
+
 void* stream_of(const at::Tensor& t) {
   return static_cast<void*>(c10::hip::getCurrentHIPStream(t.device().index()).stream());
 }
@@ -189,9 +206,6 @@ class FlashAttention : public torch::autograd::Function<FlashAttention> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& query,
                             const at::Tensor& key, const at::Tensor& value, bool causal,
                             double scale) {
-    // A strided tensor without a gradient may be a buffer (part of a key/value cache)
-    // that the program writes again before the backward: its copy is kept.
-    const auto kept = [](const at::Tensor& t) { return t.requires_grad() ? t : t.contiguous(); };
     Forward f = run_forward(kept(query), kept(key), kept(value), causal, scale);
     ctx->save_for_backward({f.q, f.k, f.v, f.o, f.lse});
     ctx->saved_data["causal"] = causal;

@@ -3,8 +3,8 @@
 The binding runs the public API's training path (forward + backward through
 the autograd engine) in C++ with the same kernel launches as the Python
 ``TritonAttention`` Function, so its results are identical bit for bit; it
-saves host time, and the copies the Python Function makes of strided inputs and
-of head sizes between the kernels' widths. It is built in-tree next to libfa_gfx950.so
+saves host time, the copies the Python Function makes of strided inputs in calls
+without gradients, and its zero-padding of head sizes between the kernels' widths. It is built in-tree next to libfa_gfx950.so
 (``_build.build_native``) and takes the entry points of the copy of the
 library that ``_lib`` has loaded. If it is missing or fails to load, the
 public API uses the Python Function (the same kernels); ``status()`` says why.

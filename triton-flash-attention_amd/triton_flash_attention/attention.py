@@ -462,8 +462,9 @@ def scaled_dot_product_attention(
     attention, arbitrary positive sequence lengths, GQA and any finite scale,
     for float16 or bfloat16 self- or cross-attention with head_dim and value
     head_dim up to 128 (32, 64 and 128 natively, other sizes at the next width).
-    Strided inputs are read as they stand where they can be; one that takes a
-    gradient is saved for the backward as it is and must not be written before.
+    Strided inputs are read as they stand where they can be. A call with gradients
+    keeps copies of them for its backward, so they may be written before it;
+    contiguous inputs of a native head_dim are kept as they are.
     Other inputs fall back to PyTorch when ``backend="auto"``;
     ``backend="triton"`` requires the custom kernel and raises RuntimeError
     otherwise; ``backend="torch"`` always uses PyTorch SDPA.
