@@ -34,22 +34,20 @@ __device__ __forceinline__ void store_dq(const BwdArgs& a, const rsrc_t& rdq, in
   const int g = (int)(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) >> 5);
   const int64_t prow = ((int64_t)split * a.BH + head) * a.N + qrow;
   float* po = split_mode ? a.part + prow * D : nullptr;  // part is null in one-pass mode
-  with_cols<DU>(a.d, [&](auto cols) {
 #pragma unroll
-    for (int db = 0; db < DU / 32; ++db)
+  for (int db = 0; db < DU / 32; ++db)
 #pragma unroll
-      for (int jq = 0; jq < 4; ++jq) {
-        float4v v;
+    for (int jq = 0; jq < 4; ++jq) {
+      float4v v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = dq[db][4 * jq + e] * mul;
-        const int col = 32 * db + 8 * jq + 4 * g;
-        if (split_mode) {
-          if (qrow < a.N) *reinterpret_cast<float4v*>(po + col) = v;
-        } else {
-          buf_store_b64(rdq, elem_off(qrow, cols, col, cols), pack4<E>(v[0], v[1], v[2], v[3]));
-        }
+      for (int e = 0; e < 4; ++e) v[e] = dq[db][4 * jq + e] * mul;
+      const int col = 32 * db + 8 * jq + 4 * g;
+      if (split_mode) {
+        if (qrow < a.N) *reinterpret_cast<float4v*>(po + col) = v;
+      } else {
+        buf_store_b64(rdq, elem_off(qrow, a.d, col, a.d), pack4<E>(v[0], v[1], v[2], v[3]));
       }
-  });
+    }
 }
 
 template <int I, int N, typename F>
@@ -195,6 +193,19 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
   const int k0w = k0 + 32 * wave;
   const int krow = k0w + ql;
 
+  // K and V, the register operands (column = key ql, d = 16*kk + 8*g .. +7). They are
+  // asked for before the units' arithmetic and DMA and awaited with the first units, so
+  // that the three run at once: behind them, with their latency after 270 scalar
+  // instructions, work-groups of two units paid for it (B2 H16, 64 queries against
+  // 16384 keys, D = 64: 71.8 us; here 68.7).
+  half8 kf[DU / 16], vn[DU / 16];
+#pragma unroll
+  for (int kk = 0; kk < DU / 16; ++kk) {
+    const uint32_t off = elem_off(krow, a.kl.row, 16 * kk + 8 * g, a.d);
+    kf[kk] = __builtin_bit_cast(half8, buf_load_b128(rk, off));
+    vn[kk] = __builtin_bit_cast(half8, buf_load_b128(rv, off));
+  }
+
   const int q_begin = CAUSAL ? k0 : 0;  // k0 is a multiple of 32
   // Under the causal mask a key tile past the last query (N < Nkv) sees no
   // query: it takes no unit (every chunk gets none, as the chunks past the
@@ -246,30 +257,22 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
       set_head();
     }
   };
-  // The units the first step needs, then the register operands, so that both
-  // latencies run at once; the units in flight over the first barrier follow the
-  // wait.
+  // The units the first step needs; the units in flight over the first barrier follow
+  // the wait.
 #pragma unroll
   for (int u = 0; u < 3; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
-  // -fp16(c K) and -V as B operands (column = key ql, d = 16*kk + 8*g .. +7).
-  // The scaled key operand is the reference's k_scaled (attention.py:435):
-  // c K in fp32 rounded to fp16. With the S accumulator started from LSE',
-  // the MFMA yields LSE' - s and P = exp2(-acc) needs no multiply-add.
-  const float c = a.c;
-  half8 kf[DU / 16], vn[DU / 16];
-  with_cols<DU>(a.d, [&](auto cols) {
-#pragma unroll
-    for (int kk = 0; kk < DU / 16; ++kk) {
-      const uint32_t off = elem_off(krow, a.kl.row, 16 * kk + 8 * g, cols);
-      kf[kk] = __builtin_bit_cast(half8, buf_load_b128(rk, off));
-      vn[kk] = neg8(__builtin_bit_cast(half8, buf_load_b128(rv, off)));
-    }
-  });
   wait_all_vm();
+  // -fp16(c K) and -V as B operands. The scaled key operand is the reference's
+  // k_scaled (attention.py:435): c K in fp32 rounded to fp16. With the S accumulator
+  // started from LSE', the MFMA yields LSE' - s and P = exp2(-acc) needs no
+  // multiply-add.
+  const float c = a.c;
 #pragma unroll
-  for (int kk = 0; kk < DU / 16; ++kk)
+  for (int kk = 0; kk < DU / 16; ++kk) {
+    vn[kk] = neg8(vn[kk]);
 #pragma unroll
     for (int e = 0; e < 8; ++e) kf[kk][e] = to_elem<E>(-c * elem_to_f32<E>(kf[kk][e]));
+  }
   // Opaque from here on, so that the operands are not recomputed inside the loop.
 #pragma unroll
   for (int kk = 0; kk < DU / 16; ++kk) asm volatile("" : "+v"(kf[kk]), "+v"(vn[kk]));
@@ -591,20 +594,18 @@ __device__ __forceinline__ void dkdv_pipe_body(const BwdArgs& a, const unsigned 
   }
   const rsrc_t rdk = make_rsrc(a.dk + (int64_t)kvh * Nkv * a.d, (uint32_t)(Nkv * a.d) * 2u);
   const rsrc_t rdv = make_rsrc(a.dv + (int64_t)kvh * Nkv * a.d, (uint32_t)(Nkv * a.d) * 2u);
-  with_cols<DU>(a.d, [&](auto cols) {
 #pragma unroll
-    for (int db = 0; db < DU / 32; ++db)
+  for (int db = 0; db < DU / 32; ++db)
 #pragma unroll
-      for (int jq = 0; jq < 4; ++jq) {
-        const uint32_t off = elem_off(krow, cols, 32 * db + 8 * jq + 4 * g, cols);
-        buf_store_b64(rdk, off,
-                      pack4<E>(dk[db][4 * jq] * nscale, dk[db][4 * jq + 1] * nscale,
-                               dk[db][4 * jq + 2] * nscale, dk[db][4 * jq + 3] * nscale));
-        buf_store_b64(rdv, off,
-                      pack4<E>(dv[db][4 * jq], dv[db][4 * jq + 1], dv[db][4 * jq + 2],
-                               dv[db][4 * jq + 3]));
-      }
-  });
+    for (int jq = 0; jq < 4; ++jq) {
+      const uint32_t off = elem_off(krow, a.d, 32 * db + 8 * jq + 4 * g, a.d);
+      buf_store_b64(rdk, off,
+                    pack4<E>(dk[db][4 * jq] * nscale, dk[db][4 * jq + 1] * nscale,
+                             dk[db][4 * jq + 2] * nscale, dk[db][4 * jq + 3] * nscale));
+      buf_store_b64(rdv, off,
+                    pack4<E>(dv[db][4 * jq], dv[db][4 * jq + 1], dv[db][4 * jq + 2],
+                             dv[db][4 * jq + 3]));
+    }
 }
 
 // --------------------------------------------------------------------------
@@ -707,6 +708,27 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
   const int q0w = q0 + 32 * wave;
   const int qrow = q0w + ql;
 
+  // The register operands Q, dO (column = query ql, d = 16*kk + 8*g .. +7), LSE and
+  // Delta or O: asked for before the units' arithmetic and DMA (see dkdv_pipe_body).
+  half8 qf[DU / 16], don[DU / 16], of[DU / 16];
+#pragma unroll
+  for (int kk = 0; kk < DU / 16; ++kk) {
+    const uint32_t off = elem_off(qrow, a.ql.row, 16 * kk + 8 * g, a.d);
+    qf[kk] = __builtin_bit_cast(half8, buf_load_b128(rq, off));
+    don[kk] = __builtin_bit_cast(half8, buf_load_b128(rdo, off));
+  }
+  const float lse = buf_load_f32(rl, (uint32_t)qrow * 4u);
+  float delta = 0.f;
+  if (a.o != nullptr) {
+    const rsrc_t ro = make_rsrc(a.o + (int64_t)head * N * a.d, (uint32_t)(N * a.d) * 2u);
+#pragma unroll
+    for (int kk = 0; kk < DU / 16; ++kk)
+      of[kk] = __builtin_bit_cast(
+          half8, buf_load_b128(ro, elem_off(qrow, a.d, 16 * kk + 8 * g, a.d)));
+  } else {
+    delta = buf_load_f32(rd, (uint32_t)qrow * 4u);
+  }
+
   const int kv_end = CAUSAL ? min(Nkv, q0 + T::BQ) : Nkv;
   // This work-group's keys [kv_lo, kv_hi): all of [0, kv_end) unless split.
   const int kv_lo = split * a.split_keys;
@@ -730,49 +752,31 @@ __device__ __forceinline__ void dq_pipe_body(const BwdArgs& a, const unsigned bl
         lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
     i_row += T::KT;
   };
-  // The units the first step needs, then the register operands, so that both
-  // latencies run at once; the units in flight over the first barrier follow the
-  // wait.
+  // The units the first step needs; the units in flight over the first barrier follow
+  // the wait.
 #pragma unroll
   for (int u = 0; u < 3; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
-  // -fp16(c Q) and -dO as B operands (column = query ql, d = 16*kk + 8*g .. +7).
-  const float c = a.c;
-  half8 qf[DU / 16], don[DU / 16];
-  with_cols<DU>(a.d, [&](auto cols) {
-#pragma unroll
-    for (int kk = 0; kk < DU / 16; ++kk) {
-      const uint32_t off = elem_off(qrow, a.ql.row, 16 * kk + 8 * g, cols);
-      qf[kk] = __builtin_bit_cast(half8, buf_load_b128(rq, off));
-      don[kk] = neg8(__builtin_bit_cast(half8, buf_load_b128(rdo, off)));
-    }
-  });
-  const float lse = buf_load_f32(rl, (uint32_t)qrow * 4u);
-  float delta;
   if (a.o != nullptr) {
     // Delta = rowsum(O * dO) of this lane's query (the halves g = 0, 1 hold
     // the two 8-wide halves of every 16-wide chunk of the row).
-    const rsrc_t ro = make_rsrc(a.o + (int64_t)head * N * a.d, (uint32_t)(N * a.d) * 2u);
     float part = 0.f;
-    with_cols<DU>(a.d, [&](auto cols) {
 #pragma unroll
-      for (int kk = 0; kk < DU / 16; ++kk) {
-        const half8 ov = __builtin_bit_cast(
-            half8, buf_load_b128(ro, elem_off(qrow, cols, 16 * kk + 8 * g, cols)));
+    for (int kk = 0; kk < DU / 16; ++kk)
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          part = fmaf(elem_to_f32<E>(ov[e]), -elem_to_f32<E>(don[kk][e]), part);
-      }
-    });
+      for (int e = 0; e < 8; ++e)
+        part = fmaf(elem_to_f32<E>(of[kk][e]), elem_to_f32<E>(don[kk][e]), part);
     delta = halves_sum(part);
     if (g == 0 && qrow < N && split == 0) a.delta_out[(int64_t)head * N + qrow] = delta;
-  } else {
-    delta = buf_load_f32(rd, (uint32_t)qrow * 4u);
   }
   wait_all_vm();
+  // -fp16(c Q) and -dO as B operands.
+  const float c = a.c;
 #pragma unroll
-  for (int kk = 0; kk < DU / 16; ++kk)
+  for (int kk = 0; kk < DU / 16; ++kk) {
+    don[kk] = neg8(don[kk]);
 #pragma unroll
     for (int e = 0; e < 8; ++e) qf[kk][e] = to_elem<E>(-c * elem_to_f32<E>(qf[kk][e]));
+  }
 #pragma unroll
   for (int kk = 0; kk < DU / 16; ++kk) asm volatile("" : "+v"(qf[kk]), "+v"(don[kk]));
 

@@ -75,6 +75,34 @@ __device__ __forceinline__ void dq_pipe16_body(const BwdArgs& a, const unsigned 
   const int q0w = q0 + 32 * wave;
   const int qrow0 = q0w + c16;  // query of block qb: qrow0 + 16 qb
 
+  // The register operands Q, dO (column = query 16 qb + c16, d = 32 kd + 8 sg .. +7),
+  // LSE and Delta or O: asked for before the units' arithmetic and DMA, awaited with the
+  // first units (see dkdv_pipe_body). Rows past N read as zeros (buffer range check).
+  half8 qf[2][KD], don[2][KD], of[2][KD];
+#pragma unroll
+  for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+    for (int kd = 0; kd < KD; ++kd) {
+      const uint32_t off = elem_off(qrow0 + 16 * qb, a.ql.row, 32 * kd + 8 * sg, a.d);
+      qf[qb][kd] = __builtin_bit_cast(half8, buf_load_b128(rq, off));
+      don[qb][kd] = __builtin_bit_cast(half8, buf_load_b128(rdo, off));
+    }
+  float lse[2], delta[2];
+#pragma unroll
+  for (int qb = 0; qb < 2; ++qb) lse[qb] = buf_load_f32(rl, (uint32_t)(qrow0 + 16 * qb) * 4u);
+  if (a.o != nullptr) {
+    const rsrc_t ro = make_rsrc(a.o + (int64_t)head * N * a.d, (uint32_t)(N * a.d) * 2u);
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+      for (int kd = 0; kd < KD; ++kd)
+        of[qb][kd] = __builtin_bit_cast(
+            half8, buf_load_b128(ro, elem_off(qrow0 + 16 * qb, a.d, 32 * kd + 8 * sg, a.d)));
+  } else {
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) delta[qb] = buf_load_f32(rd, (uint32_t)(qrow0 + 16 * qb) * 4u);
+  }
+
   const int kv_end = CAUSAL ? min(Nkv, q0 + T::BQ) : Nkv;
   // This work-group's keys [kv_lo, kv_hi): all of [0, kv_end) unless split.
   const int kv_lo = split * a.split_keys;
@@ -96,60 +124,37 @@ __device__ __forceinline__ void dq_pipe16_body(const BwdArgs& a, const unsigned 
         lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
     i_row += T::KT;
   };
-  // The units the first step needs, then the register operands, so that both
-  // latencies run at once; the units in flight over the first barrier follow the
-  // wait.
+  // The units the first step needs; the units in flight over the first barrier follow
+  // the wait.
 #pragma unroll
   for (int u = 0; u < 3; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
-  // -fp16(c Q) and -dO as B operands: column = query 16 qb + c16,
-  // d = 32 kd + 8 sg .. +7. Rows past N read as zeros (buffer range check).
-  const float c = a.c;
-  half8 qf[2][KD], don[2][KD];
-  with_cols<D>(a.d, [&](auto cols) {
-#pragma unroll
-    for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-      for (int kd = 0; kd < KD; ++kd) {
-        const uint32_t off = elem_off(qrow0 + 16 * qb, a.ql.row, 32 * kd + 8 * sg, cols);
-        qf[qb][kd] = __builtin_bit_cast(half8, buf_load_b128(rq, off));
-        don[qb][kd] = neg8(__builtin_bit_cast(half8, buf_load_b128(rdo, off)));
-      }
-  });
-  float lse[2], delta[2];
-#pragma unroll
-  for (int qb = 0; qb < 2; ++qb) lse[qb] = buf_load_f32(rl, (uint32_t)(qrow0 + 16 * qb) * 4u);
   if (a.o != nullptr) {
     // Delta = rowsum(O * dO) of each of the lane's two queries; the lanes
     // l, l^16, l^32, l^48 hold the four quarters of every 32-wide chunk.
-    const rsrc_t ro = make_rsrc(a.o + (int64_t)head * N * a.d, (uint32_t)(N * a.d) * 2u);
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
       float part = 0.f;
-      with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-        for (int kd = 0; kd < KD; ++kd) {
-          const half8 ov = __builtin_bit_cast(
-              half8, buf_load_b128(ro, elem_off(qrow0 + 16 * qb, cols, 32 * kd + 8 * sg, cols)));
+      for (int kd = 0; kd < KD; ++kd)
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
-            part = fmaf(elem_to_f32<E>(ov[e]), -elem_to_f32<E>(don[qb][kd][e]), part);
-        }
-      });
+        for (int e = 0; e < 8; ++e)
+          part = fmaf(elem_to_f32<E>(of[qb][kd][e]), elem_to_f32<E>(don[qb][kd][e]), part);
       delta[qb] = quarters_sum(part);
       const int qr = qrow0 + 16 * qb;
       if (G == 0 && qr < N && split == 0) a.delta_out[(int64_t)head * N + qr] = delta[qb];
     }
-  } else {
-#pragma unroll
-    for (int qb = 0; qb < 2; ++qb) delta[qb] = buf_load_f32(rd, (uint32_t)(qrow0 + 16 * qb) * 4u);
   }
   wait_all_vm();
+  // -fp16(c Q) and -dO as B operands.
+  const float c = a.c;
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
-    for (int kd = 0; kd < KD; ++kd)
+    for (int kd = 0; kd < KD; ++kd) {
+      don[qb][kd] = neg8(don[qb][kd]);
 #pragma unroll
       for (int e = 0; e < 8; ++e) qf[qb][kd][e] = to_elem<E>(-c * elem_to_f32<E>(qf[qb][kd][e]));
+    }
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
@@ -456,20 +461,18 @@ __device__ __forceinline__ void dq_pipe16_body(const BwdArgs& a, const unsigned 
     const int qr = qrow0 + 16 * qb;
     const int64_t prow = ((int64_t)split * a.BH + head) * a.N + qr;
     float* po = split_mode ? a.part + prow * D : nullptr;  // part is null in one-pass mode
-    with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-      for (int dd = 0; dd < DD; ++dd) {
-        float4v v;
+    for (int dd = 0; dd < DD; ++dd) {
+      float4v v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = dq[dd][qb][e] * mul;
-        const int col = 16 * dd + 4 * G;
-        if (split_mode) {
-          if (qr < a.N) *reinterpret_cast<float4v*>(po + col) = v;
-        } else {
-          buf_store_b64(rdq, elem_off(qr, cols, col, cols), pack4<E>(v[0], v[1], v[2], v[3]));
-        }
+      for (int e = 0; e < 4; ++e) v[e] = dq[dd][qb][e] * mul;
+      const int col = 16 * dd + 4 * G;
+      if (split_mode) {
+        if (qr < a.N) *reinterpret_cast<float4v*>(po + col) = v;
+      } else {
+        buf_store_b64(rdq, elem_off(qr, a.d, col, a.d), pack4<E>(v[0], v[1], v[2], v[3]));
       }
-    });
+    }
   }
 }
 
@@ -529,6 +532,19 @@ __device__ __forceinline__ void dkdv_pipe16_body(const BwdArgs& a, const unsigne
   const int k0w = k0 + 32 * wave;
   const int krow0 = k0w + c16;  // key of block kb: krow0 + 16 kb
 
+  // K and V, the register operands (column = key 16 kb + c16, d = 32 kd + 8 sg .. +7):
+  // asked for before the units' arithmetic and DMA, awaited with the first units (see
+  // dkdv_pipe_body). Rows past N_kv read as zeros.
+  half8 kf[2][KD], vn[2][KD];
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+    for (int kd = 0; kd < KD; ++kd) {
+      const uint32_t off = elem_off(krow0 + 16 * kb, a.kl.row, 32 * kd + 8 * sg, a.d);
+      kf[kb][kd] = __builtin_bit_cast(half8, buf_load_b128(rk, off));
+      vn[kb][kd] = __builtin_bit_cast(half8, buf_load_b128(rv, off));
+    }
+
   const int q_begin = CAUSAL ? k0 : 0;  // k0 is a multiple of 32
   const int ntq = max(1, (N - q_begin + T::QT - 1) / T::QT);
   const int total_units = CAUSAL && q_begin >= N ? 0 : QG * ntq;  // as in dkdv_pipe_body
@@ -572,33 +588,22 @@ __device__ __forceinline__ void dkdv_pipe16_body(const BwdArgs& a, const unsigne
       set_head();
     }
   };
-  // The units the first step needs, then the register operands, so that both
-  // latencies run at once; the units in flight over the first barrier follow the
-  // wait.
+  // The units the first step needs; the units in flight over the first barrier follow
+  // the wait.
 #pragma unroll
   for (int u = 0; u < 3; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
-  // -fp16(c K) and -V as B operands (column = key 16 kb + c16, d = 32 kd +
-  // 8 sg .. +7); the scaled key operand is the reference's k_scaled
-  // (attention.py:435). Rows past N_kv read as zeros.
-  const float c = a.c;
-  half8 kf[2][KD], vn[2][KD];
-  with_cols<D>(a.d, [&](auto cols) {
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int kd = 0; kd < KD; ++kd) {
-        const uint32_t off = elem_off(krow0 + 16 * kb, a.kl.row, 32 * kd + 8 * sg, cols);
-        kf[kb][kd] = __builtin_bit_cast(half8, buf_load_b128(rk, off));
-        vn[kb][kd] = neg8(__builtin_bit_cast(half8, buf_load_b128(rv, off)));
-      }
-  });
   wait_all_vm();
+  // -fp16(c K) and -V as B operands; the scaled key operand is the reference's
+  // k_scaled (attention.py:435).
+  const float c = a.c;
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-    for (int kd = 0; kd < KD; ++kd)
+    for (int kd = 0; kd < KD; ++kd) {
+      vn[kb][kd] = neg8(vn[kb][kd]);
 #pragma unroll
       for (int e = 0; e < 8; ++e) kf[kb][kd][e] = to_elem<E>(-c * elem_to_f32<E>(kf[kb][kd][e]));
+    }
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -924,19 +929,17 @@ __device__ __forceinline__ void dkdv_pipe16_body(const BwdArgs& a, const unsigne
   }
   const rsrc_t rdk = make_rsrc(a.dk + (int64_t)kvh * Nkv * a.d, (uint32_t)(Nkv * a.d) * 2u);
   const rsrc_t rdv = make_rsrc(a.dv + (int64_t)kvh * Nkv * a.d, (uint32_t)(Nkv * a.d) * 2u);
-  with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+  for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int dd = 0; dd < DD; ++dd) {
-        const uint32_t off = elem_off(krow0 + 16 * kb, cols, 16 * dd + 4 * G, cols);
-        buf_store_b64(rdk, off,
-                      pack4<E>(dk[dd][kb][0] * nscale, dk[dd][kb][1] * nscale,
-                               dk[dd][kb][2] * nscale, dk[dd][kb][3] * nscale));
-        buf_store_b64(rdv, off,
-                      pack4<E>(dv[dd][kb][0], dv[dd][kb][1], dv[dd][kb][2], dv[dd][kb][3]));
-      }
-  });
+    for (int dd = 0; dd < DD; ++dd) {
+      const uint32_t off = elem_off(krow0 + 16 * kb, a.d, 16 * dd + 4 * G, a.d);
+      buf_store_b64(rdk, off,
+                    pack4<E>(dk[dd][kb][0] * nscale, dk[dd][kb][1] * nscale,
+                             dk[dd][kb][2] * nscale, dk[dd][kb][3] * nscale));
+      buf_store_b64(rdv, off,
+                    pack4<E>(dv[dd][kb][0], dv[dd][kb][1], dv[dd][kb][2], dv[dd][kb][3]));
+    }
 }
 
 }  // namespace fa

@@ -9,8 +9,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <type_traits>
-
 namespace fa {
 
 typedef _Float16 half_t;
@@ -43,15 +41,6 @@ constexpr uint32_t kOutOfRange = 0x80000000u;
 // range (reads zero, stores nothing) for the columns from `cols` on.
 __device__ __forceinline__ uint32_t elem_off(int row, int stride, int col, int cols) {
   return col < cols ? (uint32_t)(row * stride + col) * 2u : kOutOfRange;
-}
-
-// f(cols) with the columns that exist of the kernel width D: an integral constant
-// where that is all of them, so that elem_off's test folds away and a row's chunks
-// differ by immediate offsets.
-template <int D, class F>
-__device__ __forceinline__ void with_cols(int d, F&& f) {
-  if (d == D) f(std::integral_constant<int, D>{});
-  else f(d);
 }
 
 __device__ __forceinline__ u32x4 buf_load_b128(rsrc_t r, uint32_t byte_off) {

@@ -79,22 +79,20 @@ __device__ __forceinline__ void store_fwd_output(const FwdArgs& a, const rsrc_t&
   const int64_t prow = ((int64_t)split * a.BH + head) * a.N + qrow;
   float* po = split_mode ? a.part + prow * D : nullptr;  // part is null in one-pass mode
   const bool row_ok = qrow < a.N;
-  with_cols<DU>(a.d, [&](auto cols) {
 #pragma unroll
-    for (int db = 0; db < DU / 32; ++db)
+  for (int db = 0; db < DU / 32; ++db)
 #pragma unroll
-      for (int jq = 0; jq < 4; ++jq) {
-        float4v v;
+    for (int jq = 0; jq < 4; ++jq) {
+      float4v v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = o[db][4 * jq + e] * inv;
-        const int col = 32 * db + 8 * jq + 4 * g;
-        if (split_mode) {
-          if (row_ok) *reinterpret_cast<float4v*>(po + col) = v;
-        } else {
-          buf_store_b64(ro, elem_off(qrow, cols, col, cols), pack4<E>(v[0], v[1], v[2], v[3]));
-        }
+      for (int e = 0; e < 4; ++e) v[e] = o[db][4 * jq + e] * inv;
+      const int col = 32 * db + 8 * jq + 4 * g;
+      if (split_mode) {
+        if (row_ok) *reinterpret_cast<float4v*>(po + col) = v;
+      } else {
+        buf_store_b64(ro, elem_off(qrow, a.d, col, a.d), pack4<E>(v[0], v[1], v[2], v[3]));
       }
-  });
+    }
   if (g == 0 && row_ok) {
     const float lse = seen ? m + log2_fast(lt) : -INFINITY;
     if (split_mode) a.part[(int64_t)a.nsplit * a.BH * a.N * D + prow] = lse;
@@ -157,12 +155,10 @@ __global__ __launch_bounds__(64 * NW) void fwd_kernel(FwdArgs a) {
   // Q^T operand fragments: lane (query ql, k-half g), d = 16*kk + 8*g .. +7.
   // Completed before the first DMA so no later wait on them drains the ring.
   half8 qf[D / 16];
-  with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk)
-      qf[kk] = __builtin_bit_cast(
-          half8, buf_load_b128(rq, elem_off(qrow, a.ql.row, 16 * kk + 8 * g, cols)));
-  });
+  for (int kk = 0; kk < D / 16; ++kk)
+    qf[kk] = __builtin_bit_cast(
+        half8, buf_load_b128(rq, elem_off(qrow, a.ql.row, 16 * kk + 8 * g, a.d)));
   wait_all_vm();
 
   // DMA prologue: tiles 0 .. AHEAD-1 into ring slots 0 .. AHEAD-1. Every
@@ -501,6 +497,15 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
   const int q0w = q0 + 32 * (wave / P);
   const int qrow = q0w + ql;
 
+  // Q^T, the register operand (lane: query ql, k-half g, d = 16*kk + 8*g .. +7): asked
+  // for before the units' arithmetic and DMA and awaited with the first units, so that
+  // the three run at once.
+  half8 qf[DU / 16];
+#pragma unroll
+  for (int kk = 0; kk < DU / 16; ++kk)
+    qf[kk] = __builtin_bit_cast(
+        half8, buf_load_b128(rq, elem_off(qrow, a.ql.row, 16 * kk + 8 * g, a.d)));
+
   const int kv_end = CAUSAL ? min(Nkv, q0 + bm) : Nkv;
   // This work-group's keys: all of [0, kv_end) unless split; with two key
   // groups, the first ceil(units / 2) units go to group 0, the rest to group
@@ -530,18 +535,10 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
         lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
     i_row += T::KT;
   };
-  // The units the first step needs, then the Q^T operand fragments (lane: query ql,
-  // k-half g, d = 16*kk + 8*g .. +7), so that both latencies run at once; the units
-  // in flight over the first barrier follow the wait.
+  // The units the first step needs; the units in flight over the first barrier follow
+  // the wait.
 #pragma unroll
   for (int u = 0; u < T::AHEAD - T::IN_FLIGHT; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
-  half8 qf[DU / 16];
-  with_cols<DU>(a.d, [&](auto cols) {
-#pragma unroll
-    for (int kk = 0; kk < DU / 16; ++kk)
-      qf[kk] = __builtin_bit_cast(
-          half8, buf_load_b128(rq, elem_off(qrow, a.ql.row, 16 * kk + 8 * g, cols)));
-  });
   wait_all_vm();
 #pragma unroll
   for (int u = T::AHEAD - T::IN_FLIGHT; u < T::AHEAD; ++u)
@@ -892,6 +889,16 @@ __device__ __forceinline__ void fwd_pipe16_body(const FwdArgs& a, int split, int
   const int q0w = q0 + 16 * QB * (wave / P);
   const int qrow0 = q0w + c16;  // query of block qb: qrow0 + 16 qb
 
+  // Q^T, the register operand (column = query 16 qb + c16, d = 32 kd + 8 sg .. +7), asked
+  // for first as in fwd_pipe_body.
+  half8 qf[QB][KD];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+    for (int kd = 0; kd < KD; ++kd)
+      qf[qb][kd] = __builtin_bit_cast(
+          half8, buf_load_b128(rq, elem_off(qrow0 + 16 * qb, a.ql.row, 32 * kd + 8 * sg, a.d)));
+
   const int kv_end = CAUSAL ? min(Nkv, q0 + bm) : Nkv;
   const int kv_lo = split * a.split_keys;
   const int kv_hi = min(kv_end, kv_lo + a.split_keys);
@@ -912,19 +919,9 @@ __device__ __forceinline__ void fwd_pipe16_body(const FwdArgs& a, int split, int
         lds0 + (uint32_t)slot * (T::STAGE * 2u) + (uint32_t)dma.piece0 * 1024u);
     i_row += T::KT;
   };
-  // The first units, the Q^T operand fragments (column = query 16 qb + c16, d =
-  // 32 kd + 8 sg .. +7), the other units (as in fwd_pipe_body).
+  // The first units; the others after the wait (as in fwd_pipe_body).
 #pragma unroll
   for (int u = 0; u < T::AHEAD - T::IN_FLIGHT; ++u) issue(s0 + u < NS ? s0 + u : s0 + u - NS);
-  half8 qf[QB][KD];
-  with_cols<D>(a.d, [&](auto cols) {
-#pragma unroll
-    for (int qb = 0; qb < QB; ++qb)
-#pragma unroll
-      for (int kd = 0; kd < KD; ++kd)
-        qf[qb][kd] = __builtin_bit_cast(
-            half8, buf_load_b128(rq, elem_off(qrow0 + 16 * qb, a.ql.row, 32 * kd + 8 * sg, cols)));
-  });
   wait_all_vm();
 #pragma unroll
   for (int u = T::AHEAD - T::IN_FLIGHT; u < T::AHEAD; ++u)
@@ -1219,20 +1216,18 @@ __device__ __forceinline__ void fwd_pipe16_body(const FwdArgs& a, int split, int
     const bool row_ok = qrow < N;
     const int64_t prow = ((int64_t)split * a.BH + head) * N + qrow;
     float* po = split_mode ? a.part + prow * D : nullptr;  // part is null in one-pass mode
-    with_cols<D>(a.d, [&](auto cols) {
 #pragma unroll
-      for (int dd = 0; dd < DD; ++dd) {
-        float4v v;
+    for (int dd = 0; dd < DD; ++dd) {
+      float4v v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = o[dd][qb][e] * inv;
-        const int col = 16 * dd + 4 * G;
-        if (split_mode) {
-          if (row_ok) *reinterpret_cast<float4v*>(po + col) = v;
-        } else {
-          buf_store_b64(ro, elem_off(qrow, cols, col, cols), pack4<E>(v[0], v[1], v[2], v[3]));
-        }
+      for (int e = 0; e < 4; ++e) v[e] = o[dd][qb][e] * inv;
+      const int col = 16 * dd + 4 * G;
+      if (split_mode) {
+        if (row_ok) *reinterpret_cast<float4v*>(po + col) = v;
+      } else {
+        buf_store_b64(ro, elem_off(qrow, a.d, col, a.d), pack4<E>(v[0], v[1], v[2], v[3]));
       }
-    });
+    }
     if (G == 0 && row_ok) {
       const float lse = seen ? m[qb] + log2_fast(lt) : -INFINITY;
       if (split_mode) a.part[(int64_t)a.nsplit * a.BH * N * D + prow] = lse;

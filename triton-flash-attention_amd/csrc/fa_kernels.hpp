@@ -3,6 +3,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 namespace fa {
@@ -57,22 +58,29 @@ struct Layout {
 // attention.py:690-718). The kernel of width D serves any head size d <= D that
 // is a multiple of 8: columns past it read as zeros (their 16-byte chunks take
 // an out-of-range offset) and are not stored.
+// The fields are ordered so that the first ones a kernel reads (num_tiles, BH, pack)
+// touch both 64-byte lines of the arguments at once: read one after the other, each
+// line is a miss of the scalar cache in the prologue of a new launch.
 struct FwdArgs {
-  const half_t* q;
-  const half_t* k;
-  const half_t* v;
-  Layout ql;       // of q
-  Layout kl;       // of k and v
-  half_t* o;       // contiguous [B, Hq, N, d]
-  float* lse;
+  int num_tiles;   // filled in by the launcher
   int N;           // query sequence length
   int Nkv;         // key/value sequence length (== N for self-attention)
   int Hq, Hkv;     // query heads, key/value heads
   int group;       // Hq / Hkv
-  int BH;          // B * Hq
   int d;           // columns of q, k, v and o
-  int num_tiles;   // filled in by the launcher
   float c;         // scale * log2(e)
+  const half_t* q;
+  const half_t* k;
+  const half_t* v;
+  float* lse;
+  // --- second line ---
+  int BH;          // B * Hq
+  // Query heads per work-group. 1: a work-group serves 32 * NW query rows of
+  // one head. pack > 1 (GQA, pack dividing both the group and NW): it serves
+  // 32 * NW / pack rows of `pack` consecutive query heads of one key/value
+  // head, wave w taking head w % pack and rows 32 * (w / pack) onward, so the
+  // heads share each K/V tile the work-group streams.
+  int pack;
   // Split-KV mode (nsplit > 1): work-group split s covers keys
   // [s * split_keys, (s + 1) * split_keys) and writes its fp32 partial O
   // ([nsplit, BH, N, D], normalised by its own row sums) and base-2 LSE
@@ -82,57 +90,60 @@ struct FwdArgs {
   // nsplit = 1: split_keys >= Nkv, part unused.
   int nsplit;
   int split_keys;  // a multiple of 128
+  Layout ql;       // of q
+  Layout kl;       // of k and v
+  half_t* o;       // contiguous [B, Hq, N, d]
   float* part;
-  // Query heads per work-group. 1: a work-group serves 32 * NW query rows of
-  // one head. pack > 1 (GQA, pack dividing both the group and NW): it serves
-  // 32 * NW / pack rows of `pack` consecutive query heads of one key/value
-  // head, wave w taking head w % pack and rows 32 * (w / pack) onward, so the
-  // heads share each K/V tile the work-group streams.
-  int pack;
   // Host-side plan of the persistent forward variant (kJobs); its launcher
   // passes *jobs to the kernel by value. Unused by the other variants.
   const FwdJobs* jobs = nullptr;
 };
+static_assert(offsetof(FwdArgs, BH) == 64 && offsetof(FwdArgs, jobs) == 128, "two lines");
 
 // Arguments of the backward launches (attention.py:736-770).
+// Ordered as FwdArgs: num_tiles and BH or BHkv touch the first two lines; the third is
+// for the epilogues and the fused Delta.
 struct BwdArgs {
-  const half_t* q;
-  const half_t* k;
-  const half_t* v;
-  const half_t* dO;
-  Layout ql;       // of q and dO
-  Layout kl;       // of k and v
-  const float* lse;
-  const float* delta;
-  half_t* dq;      // contiguous [B, Hq, N, d]
-  half_t* dk;      // contiguous [B, Hkv, Nkv, d]
-  half_t* dv;      // contiguous [B, Hkv, Nkv, d]
-  int d;           // columns of every tensor (see FwdArgs)
+  int num_tiles;   // filled in by the launcher
   int N;           // query sequence length
   int Nkv;         // key/value sequence length (== N for self-attention)
   int Hq, Hkv, group;
-  int BH;          // B * Hq
-  int BHkv;        // B * Hkv
-  int num_tiles;   // filled in by the launcher
-  float c;         // scale * log2(e)
-  float scale;
+  int d;           // columns of every tensor (see FwdArgs)
   // dK/dV split mode (nsplit > 1): work-group (tile, head, split) covers one
   // contiguous chunk of its key tile's (query head, query tile) steps and
   // writes fp32 partials part[split][B*Hkv][N][D] (dK then dV planes).
   int nsplit;
-  float* part;
+  const half_t* q;
+  const half_t* k;
+  const half_t* v;
+  const half_t* dO;
+  // --- second line ---
+  int BH;          // B * Hq
+  int BHkv;        // B * Hkv
   // dQ split mode (nsplit > 1 in a dQ launch): work-group split s covers keys
   // [s * split_keys, (s + 1) * split_keys) and writes its fp32 partial dQ
   // (scaled) to part[split][B*Hq][N][D]; launch_split_sum adds them. The
   // ranges cover visible_kv keys; with nsplit = 1, split_keys >= Nkv. Unused
   // by the dK/dV launches.
   int split_keys;
+  float c;         // scale * log2(e)
+  Layout ql;       // of q and dO
+  Layout kl;       // of k and v
+  const float* lse;
+  const float* delta;
+  // --- third line ---
   // Fused Delta (dQ kernels whose variant has kFusesDelta): when o is set the
   // kernel computes Delta = rowsum(O * dO) itself and writes it to delta_out
   // instead of reading delta. o is contiguous [B, Hq, N, d].
   const half_t* o;
   float* delta_out;
+  half_t* dq;      // contiguous [B, Hq, N, d]
+  half_t* dk;      // contiguous [B, Hkv, Nkv, d]
+  half_t* dv;      // contiguous [B, Hkv, Nkv, d]
+  float* part;
+  float scale;
 };
+static_assert(offsetof(BwdArgs, BH) == 64 && offsetof(BwdArgs, o) == 128, "lines");
 
 // Keys some query can see, which a split launch's key ranges must cover: all
 // Nkv, or under the top-left causal mask the first min(N, Nkv) (query i sees
