@@ -453,6 +453,56 @@ def test_native_binding_loads_and_takes_the_library_entry_points(lib):
         _native._module.attention(q[0], q[0], q[0], True, 0.125)
 
 
+# (B, Hq, Hkv, N_q, N_kv, D, causal, query rows per work-group, key ranges) of the forward
+# the library chooses, on both sides of its lines by launch size
+FWD_PLANS = [
+    # D = 128: tiling 7 has 256 rows, 11 has 64, the others 128
+    (1, 32, 8, 3001, 3001, 128, True, 128, 1), (1, 32, 8, 3900, 3900, 128, True, 256, 1),
+    (1, 32, 8, 1500, 1500, 128, True, 64, 1), (1, 32, 8, 1700, 1700, 128, True, 128, 1),
+    (4, 32, 8, 200, 200, 128, True, 64, 1), (4, 32, 8, 300, 300, 128, True, 128, 1),
+    (4, 16, 16, 1025, 1025, 128, False, 128, 1), (3, 32, 8, 4096, 4096, 128, False, 256, 1),
+    (3, 32, 8, 2000, 2000, 128, False, 128, 1), (1, 16, 16, 8192, 8192, 128, False, 256, 1),
+    (1, 16, 16, 8192, 8191, 128, False, 128, 1), (5, 8, 8, 1024, 1024, 128, False, 256, 1),
+    (5, 8, 8, 1024, 511, 128, False, 128, 1), (5, 8, 8, 1024, 2048, 128, False, 128, 1),
+    (1, 8, 8, 1000, 1000, 128, False, 64, 1), (1, 8, 8, 1000, 5000, 128, False, 128, 4),
+    # long loops just above 128, 256 and 384 work-groups
+    (1, 2, 2, 8320, 16384, 128, False, 128, 1), (1, 2, 2, 17000, 7000, 128, False, 128, 3),
+    (1, 2, 2, 17000, 6999, 128, False, 128, 1), (1, 2, 2, 21632, 16384, 128, False, 128, 1),
+    (1, 2, 2, 8320, 5499, 64, False, 128, 1), (1, 2, 2, 8320, 5500, 64, False, 128, 5),
+    (1, 2, 2, 10240, 5500, 64, False, 128, 1), (1, 2, 2, 12288, 11000, 64, False, 128, 4),
+    (1, 2, 2, 12416, 11000, 64, False, 128, 1), (1, 2, 2, 17000, 4000, 64, False, 128, 3),
+    (1, 2, 2, 17000, 3999, 64, False, 128, 1), (1, 2, 2, 24576, 6000, 64, False, 128, 2),
+    (1, 2, 2, 24704, 16384, 64, False, 128, 1), (1, 2, 2, 17000, 16384, 64, True, 128, 3),
+    (1, 2, 2, 9216, 4999, 32, False, 128, 1), (1, 2, 2, 9216, 5000, 32, False, 128, 4),
+    (1, 2, 2, 14336, 13999, 32, False, 128, 1), (1, 2, 2, 14336, 14000, 32, False, 128, 4),
+    (1, 2, 2, 20480, 3500, 32, False, 128, 3), (1, 2, 2, 24576, 4999, 32, False, 128, 1),
+    (1, 2, 2, 24576, 5000, 32, False, 128, 2), (1, 2, 2, 24704, 16384, 32, False, 128, 1),
+    # smallest launches
+    (1, 8, 2, 2048, 2048, 64, False, 64, 1), (1, 2, 2, 8192, 8192, 64, False, 128, 6),
+    (1, 16, 4, 1000, 1000, 64, True, 64, 1), (8, 32, 32, 130, 130, 64, False, 128, 1),
+]
+
+
+@pytest.mark.parametrize("case", FWD_PLANS, ids=lambda c: f"B{c[0]}H{c[1]}-{c[2]}Nq{c[3]}"
+                                                          f"Nkv{c[4]}D{c[5]}{'c' if c[6] else 'b'}")
+def test_forward_plan_by_launch_size(lib, case):
+    """The work-groups of the forward's grid say how many query rows the tiling it chooses
+    has (64, 128 or 256) and how many key ranges it splits into."""
+    B, Hq, Hkv, N, Nkv, D, causal, rows, ranges = case
+    grid = _lib.fwd_plan_info(B, Hq, Hkv, N, Nkv, D, causal, 256)["grid_workgroups"]
+    assert grid == -(-N // rows) * B * Hq * ranges
+
+
+def test_forward_partials_of_late_splits_fit_the_noalloc_scratch(lib):
+    """Launches past one work-group per CU that split their keys keep within the scratch of
+    fa_fwd_noalloc, which served them in one pass before they split."""
+    limit = lib.fa_fwd_noalloc_max_workspace_bytes()
+    for D in (32, 64, 128):
+        for work_groups in range(257, 386):
+            need = lib.fa_fwd_workspace_bytes(1, 1, 1, 128 * work_groups, 16384, D, 0)
+            assert 0 <= need <= limit, (D, work_groups)
+
+
 def test_strided_entries_check_strides_and_head_size(lib):
     """fa_fwd_view / fa_bwd_view take a head size that is a multiple of 8 up to
     128 and strides the kernels can address, and reject the rest before any HIP

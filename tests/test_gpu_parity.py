@@ -905,6 +905,27 @@ def test_forward_size_rule(case, dtype):
     assert float((rule[1] - classic[1]).abs().max()) <= 1e-5
 
 
+# Short and uneven launches: the classic tiling and 6 past one round of tiling 11, short
+# loops that tiling 8's merge would not pay for, one round of tiling 7, long loops on key
+# ranges just above 128 and 256 work-groups
+UNEVEN_FWD_SIZE_RULE_CASES = [
+    (4, 32, 8, 200, 200, 128, True, 11), (4, 32, 8, 300, 300, 128, True, 2),
+    (4, 32, 8, 384, 384, 128, True, 6), (5, 16, 16, 135, 135, 128, False, 6),
+    (4, 16, 16, 300, 300, 64, False, 6), (8, 16, 16, 130, 130, 32, False, 6),
+    (5, 8, 8, 1024, 1024, 128, False, 7), (1, 2, 2, 8320, 5600, 64, False, 6),
+    (1, 2, 2, 17000, 5001, 64, False, 6), (1, 2, 2, 17000, 3501, 32, False, 6),
+    (1, 1, 1, 33000, 7010, 128, False, 6), (1, 4, 1, 12288, 6000, 64, False, 6),
+]
+
+
+@pytest.mark.parametrize("case", UNEVEN_FWD_SIZE_RULE_CASES,
+                         ids=lambda c: f"B{c[0]}H{c[1]}-{c[2]}Nq{c[3]}Nkv{c[4]}D{c[5]}"
+                                       f"{'c' if c[6] else 'b'}")
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+def test_forward_size_rule_for_uneven_launches(case, dtype):
+    test_forward_size_rule(case, dtype)
+
+
 def test_decoding_forward_rule_runs_the_64_query_tiling():
     """Launches of at most 32 queries (decoding, any head size) whose queries fit
     one 64-query work-group of packed heads (N_q <= 64 / P, P = gcd(Hq / Hkv,

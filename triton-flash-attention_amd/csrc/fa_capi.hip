@@ -206,8 +206,10 @@ const fa::Variant* select_dq(int di, int causal, int64_t N, int64_t BH, int dt) 
 //     N 1500 87.2 / 76.3, B2 Hq32 Hkv8 N 4500 605 / 587, B8 Hq32 Hkv8 N 1100 188 / 167.
 //   * 7 where its rounds are whole and its loops long, as it stages K and V half
 //     as often: without the mask from three rounds of 256 work-groups exactly and
-//     L >= 4096 (B2 H32 N 8192 1902 / 1947, B1 H32 N 8192 892 / 907, B4 H16 N 4096
-//     495.6 / 499.6; with shorter loops B16 Hq32 Hkv8 N 1024 302 / 294); under the
+//     L >= 4096, from two at L >= 8192 (B2 H32 N 8192 1902 / 1947, B1 H32 N 8192 892 /
+//     907, B4 H16 N 4096 495.6 / 499.6, W 1024 with L 8192 501 / 519; with shorter loops
+//     B16 Hq32 Hkv8 N 1024 302 / 294); for 256 < W <= 384 and 512 <= L < 2048, one round
+//     of at most 192 (W 264-384, L 1024 30.0-35.1 / 31.5-35.6); under the
 //     mask at exactly two work-groups per CU, where the heaviest-first order pairs
 //     tile t with tile T - 1 - t (B1 Hq32 N 4096 133.4 / 136.8, B1 H16 N 8192 257.4 /
 //     265.2, B1 H8 N 16384 493 / 513; with more, B2 H32 N 4096 280 / 271).
@@ -218,12 +220,16 @@ const fa::Variant* select_dq(int di, int causal, int64_t N, int64_t BH, int dt) 
 //     6) beats it: B1 H4 N 8192 89.6 / 98.5, B1 H2 N 16384 152.7 / 186.8.
 //   * Without the mask 8 takes 128 < W <= 256 (one work-group per CU; launches of
 //     one query tile keep 6 and its key ranges, B8 Hq32 Hkv8 N_q 128 against 8192 keys
-//     154.5 / 169.2): B1 H16 N 2048
-//     38.9 against 39.2 (6) and 43.6 (11), B1 H4 N 8192 131.7 / 137.3 / 155.6; past
-//     W = 256 it needs a second round (B1 H12 N 3000 90.9 / 75.1).
+//     154.5 / 169.2) from L = 1536: B1 H16 N 2048
+//     38.9 against 39.2 (6) and 43.6 (11), B1 H4 N 8192 131.7 / 137.3 / 155.6; with
+//     shorter loops its merge costs more (8 / 6: W 160, L 256 12.4 / 10.8, L 800 18.6 /
+//     17.8), past W = 256 it needs a second round (B1 H12 N 3000 90.9 / 75.1).
 //   * 11 for the smallest: causal L < 2048 up to W = 384 (6 / 11: B1 Hq32 Hkv8 N 512
 //     14.3 / 11.2, N 1024 21.9 / 19.7, B2 H16 N 1300 29.0 / 24.6; at W = 512 B4 H16
-//     N 1024 29.6 / 31.5), and W <= 128 with L < 4096 (B1 H8 N 1024 without the mask
+//     N 1024 29.6 / 31.5), below L = 640 while its work-groups are one round of two per
+//     CU; past that the classic tiling 2 up to 320 queries and W = 600 (11 / 6 / 2: 128
+//     heads of 300 16.9 / 15.2 / 15.0, 192 of 129 13.3 / 12.4 / 11.7, 256 of 160 14.2 / 14.0
+//     / 13.2) and 6 above (128 heads of 384 19.7 / 17.4 / 18.6, 384 of 160 - / 21.3 / 23.9); and W <= 128 with L < 4096 (B1 H8 N 1024 without the mask
 //     19.5 / 16.6, B1 H4 N 3000 causal 35.1 / 32.1); with longer loops 6 and its key
 //     ranges (B1 H2 N 8192 causal 63.5 / 95.8, B1 H8 N_q 1024 against 4096 33.6 / 36.8).
 constexpr int kFwdWideVariant = 7;
@@ -233,16 +239,29 @@ constexpr int kFwdPipeVariant = 6;
 // Hkv8 N_q 17 against 8192 keys 54.6 / 63.9, N_q 32 63.2 / 82.7).
 constexpr int kFwdNarrowVariant = 2;
 constexpr int64_t kFwdNarrowQueries = 96;
+constexpr int64_t kFwdNarrowCausalQueries = 320;
 constexpr int64_t kFwdComputeUnits = 256;
-// Without the mask at D <= 64, from two query tiles, 128 < W <= 256 (up to 512 at D = 32, where two of
-// its work-groups fit a CU) takes the two-key-group tiling 8 in one pass; tiling
-// 6 with its keys split, as such launches ran before, / 8: D = 64 B1 H16 N 2048
-// 34.6 / 23.1, B1 H8 N 4096 53.6 / 41.4, B1 H4 N 8192 86.8 / 78.5, B1 H10 N 2500
-// 33.1 / 25.4, B1 H16 N 1500 (not split) 19.3 / 17.8; D = 32 25.5 / 18.3, 39.4 /
-// 31.8, 65.1 / 58.6, B1 H16 N 4096 58.4 / 54.6. Smaller launches of short loops
-// (W <= 128, L < 4096; causal 512 <= N < 2048 below W = 256) take tiling 11: D = 64 B1 H16
-// N 1024 14.3 / 12.1 (causal 15.8 / 12.4), B1 H8 N 2048 22.7 / 20.5; with longer
-// loops tiling 6 splits its keys (B1 H2 N 8192 52.9 / 70.2).
+// Without the mask, from two query tiles, the two-key-group tiling 8 takes 128 < W <=
+// 256 in one pass where its loops pay for its merge (from L = 640 at D = 32, 1024 at 64,
+// 1536 at 128), and at D = 32, where two of its work-groups fit a CU, up to W = 512 from
+// L = 2048. Tiling 6 with its keys split, as such launches ran before, / 8, us: D = 64 B1
+// H16 N 2048 34.6 / 23.1, B1 H8 N 4096 53.6 / 41.4, B1 H4 N 8192 86.8 / 78.5, B1 H10
+// N 2500 33.1 / 25.4; D = 32 25.5 / 18.3, 39.4 / 31.8, 65.1 / 58.6, B1 H16 N 4096 58.4 /
+// 54.6; shorter, 6 / 8: D = 64 W 192, L 512 10.6 / 11.0, D = 32 W 512, L 256 8.3 / 10.1.
+// It leaves 256 - W CUs idle, so long loops keep 6 and its key ranges while W is small: 6 /
+// 8 at D = 64 W 130, L 6000 47.6 / 51.5, L 16384 106 / 129, W 160 128 / 134, W 192, L 12000
+// 101 / 104; D = 32 W 144, L 6000 37.6 / 43.7, W 224, L 16384 113 / 117. Smaller launches
+// of short loops (W <= 128, L < 4096; causal 512 <= N < 2048 below W = 256) take tiling 11:
+// D = 64 B1 H16 N 1024 14.3 / 12.1 (causal 15.8 / 12.4), B1 H8 N 2048 22.7 / 20.5; with
+// longer loops tiling 6 splits its keys (B1 H2 N 8192 52.9 / 70.2).
+bool fwd_groups_keys(int di, int64_t W, int64_t L) {
+  if (W <= 128) return false;
+  if (di == fa::head_dim_index(128)) return W <= 256 && L >= 1536;
+  if (di == fa::head_dim_index(64))
+    return W <= 256 && L >= 1024 && !(W <= 144 && L >= 5500) && !(W <= 192 && L >= 11000);
+  if (W <= 256) return L >= 640 && !(W <= 192 && L >= 5000) && !(W <= 224 && L >= 14000);
+  return W <= 512 && L >= 2048 && !(W <= 320 && L >= 3500) && !(W <= 384 && L >= 5000);
+}
 
 // At D = 32 a causal launch over few heads (B*H * (query tiles + 1) < 1536)
 // takes the two-key-group forward: 8 waves per work-group as two groups that
@@ -314,15 +333,19 @@ int fwd_variant_d128(int causal, int64_t N, int64_t L, int64_t BH) {
   const int64_t wide = (N + 255) / 256 * BH;  // tiling 7's work-groups
   if (W <= 128) return L < 4096 ? kFwd16HalfVariant : kFwdPipeVariant;
   if (causal) {
+    if (L < 640 && (N + 63) / 64 * BH > 2 * kFwdComputeUnits)
+      return N <= kFwdNarrowCausalQueries && W <= 600 ? kFwdNarrowVariant : kFwdPipeVariant;
     if (L < 2048) return W <= 384 ? kFwd16HalfVariant : kFwdPipeVariant;
     if (W <= 256 && L > 4096) return kFwdPipeVariant;
     if (W <= 512) return kFwdKeyGroupVariant;
     return wide == 2 * kFwdComputeUnits && L > 3584 ? kFwdWideVariant : kFwdPipeVariant;
   }
-  if (W <= 256 && N > 128) return kFwdKeyGroupVariant;
-  return wide % kFwdComputeUnits == 0 && wide >= 3 * kFwdComputeUnits && L >= 4096
-             ? kFwdWideVariant
-             : kFwdPipeVariant;
+  if (N > 128 && fwd_groups_keys(fa::head_dim_index(128), W, L)) return kFwdKeyGroupVariant;
+  const bool whole = wide % kFwdComputeUnits == 0 &&
+                     (wide >= 3 * kFwdComputeUnits ? L >= 4096
+                                                   : wide == 2 * kFwdComputeUnits && L >= 8192);
+  const bool one_round = W > 256 && W <= 384 && wide <= 192 && L >= 512 && L < 2048;
+  return whole || one_round ? kFwdWideVariant : kFwdPipeVariant;
 }
 
 const fa::Variant* select_fwd(int di, int causal, int64_t N, int64_t Nkv, int64_t BH,
@@ -345,8 +368,7 @@ const fa::Variant* select_fwd(int di, int causal, int64_t N, int64_t Nkv, int64_
   const int64_t W = (N + 127) / 128 * BH;
   if (!causal && N > 128) {
     if (W <= 128 && L < 4096) return pick(kFwd16HalfVariant);
-    if (W > 128 && W <= (di == fa::head_dim_index(32) ? 512 : 256))
-      return pick(kFwdKeyGroupVariant);
+    if (fwd_groups_keys(di, W, L)) return pick(kFwdKeyGroupVariant);
   }
   if (causal) {
     if (N >= 2048 && W <= 512 && (W >= 384 || (W >= 256 && N <= 4096)))
@@ -607,6 +629,19 @@ constexpr int64_t kFwdSplitBelowWorkgroups = 512;
 // splits its keys inside the work-group, does not split there at all (D = 128
 // causal B1 H16 N 2048 46.3 / 31.5, B1 H12 N 4096 88.5 / 61.1).
 constexpr int64_t kFwdLateSplitBelow = 257;
+// Without the mask, long loops of 257 to 384 work-groups do split: one pass leaves up to
+// half of the second round of CUs idle for their whole length, three key ranges (two above
+// 341 work-groups) fill four rounds (three). Split / one pass, us: D = 64 W 264, L 6000 85 /
+// 94, L 16384 208 / 250, W 320, L 4096 68.0 / 68.8, W 384, L 8192 133 / 142, but W 264,
+// L 3000 53.5 / 49.9, W 416, L 16384 303 / 288; D = 32 (one pass on tiling 8) W 320, L 4096 49.0 / 51.1, W 384, L 8192
+// 93 / 100; D = 128 W 264, L 8192 186 / 201, W 320, L 16384 363 / 405, but L 6000 160 / 160,
+// W 384, L 8192 233 / 226.
+// (336 work-groups at D = 128: their partials are the most that fa_fwd_noalloc holds.)
+bool fwd_splits_late(int64_t D, int64_t wgs, int64_t L) {
+  if (wgs < kFwdLateSplitBelow || wgs > (D == 128 ? 336 : 384)) return false;
+  if (D == 32) return L >= (wgs <= 320 ? 3500 : 5000);
+  return L >= (D == 128 ? 7000 : wgs <= 320 ? 4000 : 6000);
+}
 constexpr int64_t kFwdSplitTargetWorkgroups = 768;
 // The 64-query forward (kFewSplits) decodes at D >= 64 faster with one
 // work-group per CU than with three: its key ranges run quicker, so partials
@@ -694,12 +729,16 @@ FwdSplit fwd_split(const fa::Variant& var, int64_t B, int64_t Hq, int64_t Hkv, i
   const int64_t rows = var.rows / pack;  // query rows per head and work-group
   const int64_t target = (var.flags & fa::kFewSplits) && D >= 64 ? kFwdSplitTargetFew
                                                                 : kFwdSplitTargetWorkgroups;
+  const int64_t wgs = (N + rows - 1) / rows * B * Hq / pack;
+  const int64_t visible = visible_keys(N, Nkv, causal);
   int64_t below = var.flags & fa::kSplitsKv ? kFwdSplitBelowWorkgroups : 0;
-  if ((var.flags & fa::kLateSplit) && (D == 128 || !causal) && N > 128)
+  if ((var.flags & fa::kLateSplit) && (D == 128 || !causal) && N > 128) {
+    if (!causal && fwd_splits_late(D, wgs, visible))
+      return key_split(wgs, Nkv, visible, below, 4 * kFwdComputeUnits / wgs * wgs);
     below = std::min(below, kFwdLateSplitBelow);
+  }
   if ((var.flags & fa::kKeyGroups) && (D == 128 || !causal)) below = 0;
-  return key_split((N + rows - 1) / rows * B * Hq / pack, Nkv, visible_keys(N, Nkv, causal), below,
-                   target);
+  return key_split(wgs, Nkv, visible, below, target);
 }
 
 // dQ: the same split of its key loop; the partials (fp32 dQ) are summed.
