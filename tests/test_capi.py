@@ -503,6 +503,20 @@ def test_forward_partials_of_late_splits_fit_the_noalloc_scratch(lib):
             assert 0 <= need <= limit, (D, work_groups)
 
 
+@pytest.mark.parametrize("heads, n_kv, D, ranges", [
+    (8, 2048, 128, 1), (8, 2049, 128, 4), (48, 20000, 64, 5), (56, 20000, 64, 4),
+    (64, 30000, 64, 4), (72, 30000, 64, 7), (96, 8192, 128, 2), (127, 3000, 64, 2),
+    (128, 8192, 64, 1), (128, 8192, 128, 2), (128, 32768, 64, 2), (128, 32768, 32, 2),
+    (136, 8192, 128, 3), (152, 32768, 128, 1), (256, 32768, 128, 1), (264, 2000, 64, 1),
+    (264, 3200, 64, 4), (264, 8192, 32, 4), (320, 8192, 64, 4), (341, 8192, 64, 3),
+    (342, 32768, 64, 1), (512, 32768, 64, 1), (520, 8192, 128, 1)])
+def test_decoding_plan_by_heads_and_keys(lib, heads, n_kv, D, ranges):
+    """Key ranges per key/value head of a decoding launch, on both sides of its lines (one
+    query, groups of four query heads)."""
+    info = _lib.fwd_plan_info(heads, 4, 1, 1, n_kv, D, False, 256)
+    assert info["grid_workgroups"] == heads * ranges
+
+
 def test_strided_entries_check_strides_and_head_size(lib):
     """fa_fwd_view / fa_bwd_view take a head size that is a multiple of 8 up to
     128 and strides the kernels can address, and reject the rest before any HIP

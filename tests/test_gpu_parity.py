@@ -2419,6 +2419,16 @@ def test_decoding_kernel_matches_float64(case, dtype):
             assert err <= 1e-5 * mult * mult, (mult, err)
 
 
+@pytest.mark.parametrize("case", [(264, 2, 1, 3, 3201, 64), (128, 1, 1, 5, 5300, 80),
+                                  (136, 4, 1, 1, 5001, 128)],  # 4, 2 and 3 ranges a head
+                         ids=lambda c: f"B{c[0]}H{c[1]}-{c[2]}Nq{c[3]}Nkv{c[4]}D{c[5]}")
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+def test_decoding_of_many_heads_with_key_ranges_matches_float64(case, dtype):
+    """The same from 128 key/value heads on, where long launches that leave much of a round
+    of CUs idle split their keys."""
+    test_decoding_kernel_matches_float64(case, dtype)
+
+
 def test_plain_call_check_agrees_with_the_rules(monkeypatch):
     """The native check of a plain call says yes only where the rules do, at their
     scale, and a call that it passes on gives what it gives without the check:

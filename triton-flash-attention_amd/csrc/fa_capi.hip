@@ -664,12 +664,21 @@ constexpr int64_t kFwdMinSplitKeys = 1024;
 // 15.4 / 18.2 / 23.8, B1 4096 keys 15.1 / 22.0 / 18.2, B8 8192 keys 44.2 / 48.3 / 44.4
 // (D64 24.1 / 26.2 / 24.9, D32 15.6 / 20.2 / 16.7); not taken: B2 1500 keys 14.7 /
 // 11.5 / 21.0, B1 2000 keys 14.7 / 13.6 / 26.4, 128 work-groups (B8 Hkv16) 16 queries
-// 2048 keys 25.7 / 21.4 / 25.0, 8 queries 8192 keys D64 44.5 / 39.1 / 41.1.
+// 2048 keys 25.7 / 21.4 / 25.0, 8 queries 8192 keys D64 44.5 / 39.1 / 41.1. Where one
+// work-group per CU already fills 7/8 of them, more ranges only add partials (kernels
+// alone, one / two per CU: D64 64 heads of 30000 keys 85.3 / 88.5, of 3000 12.6 / 13.7).
+// From 128 work-groups on one pass leaves up to half of its last round of CUs idle; long
+// ranges fill it, with 2 to 4 per head, once that saves more than the merge costs (kernels
+// alone, ranges / one pass / the general tiling, us): 128 heads of 8192 keys D128 94.9 /
+// 105.9 / 94.7, of 32768 363 / 408 / 368, D64 of 32768 180 / 202 / 182; 264 heads of 8192
+// keys D64 103 / 122 / 112, D32 46.5 / 54.8 / 53.7; 320 heads of 32768 D64 450 / 514 / 492;
+// not taken: 128 heads of 8192 keys D64 43.5 / 39.3 / 43.8, of 4096 D128 44.4 / 41.8 / 44.9,
+// 160 of 8192 D128 118 / 113 / 132, 400 of 32768 D32 281 / 278 / 336.
 constexpr int64_t kDecodeSplitBelow = 128;
-constexpr int64_t kDecodeSplitTarget = 512;
-constexpr int64_t kDecodeSplitTarget128 = 256;
 constexpr int64_t kDecodeOnePassKeys = 2048;
 constexpr int64_t kDecodeMinSplitKeys = 512;
+constexpr int64_t kDecodeLongBytes = int64_t{320} << 20;      // of K and V, up to 256 heads
+constexpr int64_t kDecodeLongBytesMore = int64_t{192} << 20;  // above
 constexpr int kMaxFwdSplit = fa::kMaxFwdSplitKv;
 
 struct FwdSplit {
@@ -719,13 +728,35 @@ FwdSplit key_split(int64_t wgs, int64_t Nkv, int64_t visible, int64_t below,
   return {(int)((visible + keys - 1) / keys), (int)keys};
 }
 
+// Key ranges of the decoding kernel for `heads` key/value heads (see kDecodeSplitBelow).
+FwdSplit decode_split(int64_t heads, int64_t Nkv, int64_t D) {
+  const int64_t cus = kFwdComputeUnits;
+  const FwdSplit one_pass = key_split(heads, Nkv, Nkv, 0);
+  if (heads < kDecodeSplitBelow) {
+    if (Nkv <= kDecodeOnePassKeys) return one_pass;
+    const bool fills = cus / heads * heads * 8 >= cus * 7;
+    const int64_t most = D == 128 || fills ? cus : 2 * cus;
+    return key_split(heads, Nkv, Nkv, kDecodeSplitBelow, most / heads * heads,
+                     kDecodeMinSplitKeys);
+  }
+  // Rounds of CUs that `ranges` per head take, times the work each work-group keeps.
+  const auto rounds = [&](int64_t ranges) {
+    return (double)((heads * ranges + cus - 1) / cus) / (double)ranges;
+  };
+  const double idle = rounds(1) * (double)cus / (double)heads;  // 1: none
+  const int64_t bytes = heads * Nkv * D * 4;
+  if (idle < (heads <= cus ? 1.7 : 1.5) ||
+      bytes < (heads <= cus ? kDecodeLongBytes : kDecodeLongBytesMore))
+    return one_pass;
+  int64_t best = 2;
+  for (int64_t r = 3; r <= 4; ++r)
+    if (rounds(r) < rounds(best)) best = r;
+  return key_split(heads, Nkv, Nkv, heads + 1, best * heads, kDecodeMinSplitKeys);
+}
+
 FwdSplit fwd_split(const fa::Variant& var, int64_t B, int64_t Hq, int64_t Hkv, int64_t N,
                    int64_t Nkv, int64_t D, int pack, int causal) {
-  if (fwd_decodes(var, causal, Hq / Hkv, N)) {
-    const int64_t wgs = B * Hkv, most = D == 128 ? kDecodeSplitTarget128 : kDecodeSplitTarget;
-    return key_split(wgs, Nkv, Nkv, Nkv > kDecodeOnePassKeys ? kDecodeSplitBelow : 0,
-                     most / wgs * wgs, kDecodeMinSplitKeys);
-  }
+  if (fwd_decodes(var, causal, Hq / Hkv, N)) return decode_split(B * Hkv, Nkv, D);
   const int64_t rows = var.rows / pack;  // query rows per head and work-group
   const int64_t target = (var.flags & fa::kFewSplits) && D >= 64 ? kFwdSplitTargetFew
                                                                 : kFwdSplitTargetWorkgroups;
