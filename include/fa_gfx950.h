@@ -377,7 +377,8 @@ int fa_abi_version(void);
 
 /* Tiling table (replaces the Triton autotuner, attention.py:82-90, 353-381).
  * kernel: 0 = fwd, 1 = bwd_dkdv, 2 = bwd_dq.
- * fa_get_tiling writes the entry used for (kernel, D, causal):
+ * fa_get_tiling writes the table's entry for (kernel, D, causal), or the one set,
+ * which the shape rules below refine launch by launch unless one was set:
  *   out[0] = waves per work-group, out[1] = rows per work-group,
  *   out[2] = streamed tile length (keys for fwd/dq, queries for dkdv),
  *   out[3] = variant index.
@@ -396,20 +397,32 @@ int fa_abi_version(void);
  * tiling (variant 1); at D = 128 under the mask, launches of at least 128
  * queries and at most 768 work-groups of 128 queries run the pipelined
  * tiling (variant 4).
- * The forward's shape rules, unless a tiling was set: at D = 128, fewer than
- * 512 queries or fewer than 128 work-groups of 256 queries run the 4-wave
- * tiling (variant 2) instead of the 8-wave one; at D <= 64 under the mask,
- * launches of at least 2048 queries with W = B * Hq * (query tiles of 128)
- * between 384 and 512, or between 256 and 512 with at most 4096 queries, run
- * the pipelined 16x16x32 tiling with 64-query work-groups (variant 11), and
- * so do launches of at most 32 queries (decoding, any head size) whose queries
- * fit one of its work-groups (at most 64 / P queries, P = gcd(Hq / Hkv, 4)
- * query heads packed per work-group), and launches of 33 to 64 queries
- * without the mask, ahead of the D = 128 rule above;
- * otherwise at D = 32 under the mask,
- * launches over few heads (B * Hq * (query tiles of 128 + 1) < 1536) run the
- * two-key-group tiling (variant 8), and the other launches of at least 512
- * queries the pipelined tiling on 16x16x32 MFMAs (variant 10).
+ * The forward's shape rules, unless a tiling was set, first match; W is B * Hq *
+ * (query tiles of 128) and L the keys of the longest loop (all of them, or the
+ * visible ones under the mask):
+ * - Launches without the mask of at most 16 query rows per key/value head (Hq / Hkv *
+ *   N_q) run the decoding kernel, which packs the whole group. Other launches of at
+ *   most 32 queries whose queries fit one of its work-groups (at most 64 / P queries,
+ *   P = gcd(Hq / Hkv, 4) query heads packed per work-group), and launches of 33 to 64
+ *   queries without the mask, run the pipelined 16x16x32 tiling with 64-query
+ *   work-groups (variant 11).
+ * - D = 128 runs the pipelined 4-wave tiling (variant 6) except: the rest of the
+ *   launches of at most 32 queries, 65 to 96 queries without the mask, and up to 320
+ *   queries under it with W <= 600 once variant 11 would take more than 512
+ *   work-groups (variant 2); W <= 128 with L < 4096, and under the mask W <= 384 with L
+ *   < 2048 (below L = 640 up to 512 of its work-groups) (variant 11); without the mask
+ *   128 < W <= 256 with L >= 1536 and more than 128 queries, and under the mask 128 < W
+ *   <= 512 with L >= 2048, unless L > 4096 and W <= 256 (two key groups, variant 8); whole
+ *   rounds of long loops, and one round of at most 192 work-groups of 256 queries
+ *   without the mask for 512 <= L < 2048 (the 8-wave tiling, variant 7).
+ * - D <= 64 without the mask and with more than 128 queries: variant 11 for W <= 128
+ *   with L < 4096; variant 8 for 128 < W <= 256 (512 at D = 32) with loops long enough
+ *   for its merge and not so long that its idle CUs cost more than key ranges.
+ * - D <= 64 under the mask: at least 2048 queries with W between 384 and 512, or between
+ *   256 and 512 with at most 4096 queries, and at D = 64 from 512 to 2047 queries below
+ *   W = 256, run variant 11; otherwise at D = 32 launches over few heads (B * Hq * (query
+ *   tiles of 128 + 1) < 1536, more than 32 queries) run variant 8, and the other launches
+ *   of at least 512 queries the pipelined tiling on 16x16x32 MFMAs (variant 10).
  * fa_set_tiling is safe to call while other threads launch:
  * each (kernel, D, causal) entry is an atomic that a launch reads once, so
  * the launch runs either the previous or the new tiling. */

@@ -643,16 +643,15 @@ bool fwd_splits_late(int64_t D, int64_t wgs, int64_t L) {
   return L >= (D == 128 ? 7000 : wgs <= 320 ? 4000 : 6000);
 }
 constexpr int64_t kFwdSplitTargetWorkgroups = 768;
-// The 64-query forward (kFewSplits) decodes at D >= 64 faster with one
-// work-group per CU than with three: its key ranges run quicker, so partials
-// and the merge weigh more, and at D = 128 one work-group fills a CU (MI355X,
-// interleaved, targets 768 vs 256, us: B32 Hq32 Hkv8 1 query against 2048
-// keys D128 45.4 / 42.3 (no split, no merge), B8 Hq32 Hkv8 16 queries against
-// 8192 keys 51.4 / 49.1, B2 Hq32 Hkv32 1 query against 16384 keys 98.6 / 93.7,
-// B4 Hq16 Hkv16 1 query against 16384 keys D64 47.9 / 43.1; B8 Hq32 Hkv8 1
-// query against 8192 keys D128 45.0 / 46.6; 384 is worse than both: 1.5
-// rounds of work-groups). At D = 32 (half the bytes per key) three stay
-// faster (16.2 vs 21.4 us at B8 Hq32 Hkv8 against 8192 keys).
+// The 64-query forward (kFewSplits) at D >= 64 aims at one work-group per CU, not three:
+// its key ranges run quicker, so partials and the merge weigh more (MI355X, kernels and
+// merge, targets 768 / 512 / 256, us: D64 B8 H16 N_q 64 against 8192 keys 50.1 / 47.7 /
+// 44.1, B2 H16 N_q 32 against 32768 48.2 / 47.0 / 43.7; D128 B8 Hq32 Hkv8 N_q 64 against
+// 2048 34.4 / 34.4 / 30.4). Up to 32 queries of grouped heads the three are within 2 %
+// on average. Against it: 33-64 queries of grouped heads, which do not pack, at D = 64
+// (B8 Hq32 Hkv8 N_q 48 against 8192 keys 52.6 / 54.4 / 71.0). At D = 32 (half the bytes
+// per key) three per CU are faster (33-64 grouped queries 0.77 of the time, ungrouped
+// 0.94).
 constexpr int64_t kFwdSplitTargetFew = 256;
 constexpr int64_t kFwdMinSplitKeys = 1024;
 // The decoding kernel (fa_fwd_decode.hip) runs a range of keys on four waves, so

@@ -388,7 +388,7 @@ __global__ __launch_bounds__(64 * NW) void fwd_kernel(FwdArgs a) {
 // launch ends with less idle. MI355X, one box, 8 waves vs 2 x 4, us: bf16 causal
 // B1 Hq32 Hkv8 N 2048 72.4 / 47.0, N 3001 121.5 / 81.5, N 3800 172.1 / 123.2,
 // N 5000 223.5 / 214.8; B4 H16 N 4096 280.9 / 275.4; bidirectional B4 H16 N 1025
-// 61.8 / 52.3, N 4096 495.6 / 499.6, B2 H32 N 8192 1902 / 1947 (7.8 TFLOP at
+// 61.8 / 52.3, N 4096 495.6 / 499.6, B2 H32 N 8192 1902 / 1947 (2.2 TFLOP at
 // 1.13 PFLOP/s: with whole rounds of long loops the staging it saves decides).
 // KG = key groups: with KG = 2 the NW waves form two groups of NW/2 that
 // serve the same queries, each streaming one half of the work-group's key
@@ -829,8 +829,8 @@ __device__ __forceinline__ void fwd_pipe_body(const FwdArgs& a, int split, int q
 // 32 queries per wave (tiling 10), QB = 1 halves the work-group to 64
 // queries (tiling 11: twice the work-groups and half the work per unit, for
 // launches too small to fill the GPU, whose time is their longest key loop,
-// and for decoding; at D = 128 too, with two DMA pieces per wave and a 96 KiB
-// ring, one work-group per CU).
+// and for decoding; at D = 128 too, with two DMA pieces per wave and tiling 6's
+// 5-slot ring of 80 KiB, two work-groups per CU).
 // Each 32-key unit against a query block is two 16 x 16 score blocks (key
 // block kb); each K row read and each transposed V read from LDS feeds QB
 // MFMAs, so with QB = 2 LDS traffic, vector work and FLOP are tiling 6's.
@@ -1396,7 +1396,7 @@ constexpr void* fwd_pipe16_entry() {
 }
 
 // The same with one 16-row query block per wave (64 queries per work-group);
-// also at D = 128, where a work-group takes a CU alone (a 96 KiB ring).
+// also at D = 128 (a ring of 80 KiB, two work-groups per CU).
 template <int D, bool CAUSAL, int NW, int UPS, class E = F16>
 constexpr void* fwd_pipe16_half_entry() {
   if constexpr (NW == 4 && UPS == 1 && (D == 128 || fwd_pipe_tiling_ok<D, 4, 1>()))
@@ -1568,7 +1568,7 @@ static const Variant kFwdVariants[] = {
     {4, 128, 32, {FA_ENTRIES(fwd_pipe16_entry, F16, 4, 1), FA_ENTRIES(fwd_pipe16_entry, BF16, 4, 1)},
      kSplitsKv},
     // 11: tiling 10 with one 16-row query block per wave, 64 queries per work-group
-    // (all D; at D = 128 one work-group per CU)
+    // (all D; at D = 128 two work-groups per CU)
     {4, 64, 32,
      {FA_ENTRIES(fwd_pipe16_half_entry, F16, 4, 1), FA_ENTRIES(fwd_pipe16_half_entry, BF16, 4, 1)},
      kSplitsKv | kFewSplits},

@@ -234,7 +234,9 @@ def _decide_rules(facts: _DispatchFacts) -> DispatchDecision:
     if (facts.head_dim, facts.value_head_dim) != (width, width):
         sizes = (str(facts.head_dim) if facts.value_head_dim == facts.head_dim
                  else f"{facts.head_dim} / value {facts.value_head_dim}")
-        padded = f" (head_dim {sizes}: zero-padded to {width})"
+        as_read = facts.head_dim == facts.value_head_dim and facts.head_dim % 8 == 0
+        verb = "read as zero-padded" if as_read else "zero-padded"
+        padded = f" (head_dim {sizes}: {verb} to {width})"
     return DispatchDecision(
         "triton",
         f"gfx950 {str(facts.dtype).removeprefix('torch.')} {kind} with a supported "
